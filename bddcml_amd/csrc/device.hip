@@ -2906,8 +2906,13 @@ static void count_pc_applies(Solver &S, int add) {
 // what a captured iteration depends on beyond the solver's fixed buffers
 static std::vector<const void *> pcg_graph_key(Solver &S, const double *rz) {
   std::vector<const void *> key{rz, S.dev->hrr_dev};
-  for (Solver *L = &S; L && L->dev; L = L->lev2.get())
-    key.push_back(L->dev->explicit_inv ? (const void *)L->dev->fpool.p : nullptr);
+  for (Solver *L = &S; L && L->dev; L = L->lev2.get()) {
+    const Device &E = *L->dev;
+    // the factor pool of the level's precision once it holds S'^{-1}
+    key.push_back(!E.explicit_inv ? nullptr
+                  : E.mixed       ? (const void *)E.pool32.p
+                                  : (const void *)E.fpool.p);
+  }
   return key;
 }
 
