@@ -387,7 +387,7 @@ struct Device {
   DBuf<double> sol;
   // vectors
   DBuf<double> vblock;  // the allocation the solve vectors are carved from
-  DBuf<double> yl, zl, rcs, rc, uc, partial, dots;
+  DBuf<double> yl, zl, rcs, zts, rc, uc, partial, dots;
   DBuf<double> pcg;           // PCG scalars per iteration: r.z, p.Ap, r.r
   DBuf<double> recV, recW;    // recycling basis V and W = S V (columns of length nig)
   DBuf<double> recc, recpart; // its projection coefficients and partial sums
@@ -2221,17 +2221,21 @@ void device_setup_finish(Solver &S) {
     DBuf<double> *krylov[] = {&D.u, &D.r, &D.p, &D.z, &D.ap, &D.rs, &D.v, &D.y, &D.s, &D.t, &D.g,
                               &D.xin, &D.xout};
     const size_t nk = sizeof(krylov) / sizeof(krylov[0]);
-    const size_t sizes[] = {(size_t)lv, (size_t)lv, (size_t)std::max(co, 1), (size_t)D.NC,
-                            (size_t)D.NC, (size_t)DOT_BLOCKS * 4, 4, (size_t)D.VT};
-    DBuf<double> *fixed[] = {&D.yl, &D.zl, &D.rcs, &D.rc, &D.uc, &D.partial, &D.dots, &D.vec};
+    const size_t sizes[] = {(size_t)lv, (size_t)lv, (size_t)std::max(co, 1),
+                            (size_t)std::max(co, 1), (size_t)D.NC, (size_t)D.NC,
+                            (size_t)DOT_BLOCKS * 4, 4, (size_t)D.VT};
+    DBuf<double> *fixed[] = {&D.yl,  &D.zl, &D.rcs,     &D.zts, &D.rc,
+                             &D.uc, &D.partial, &D.dots, &D.vec};
+    constexpr size_t nf = sizeof(fixed) / sizeof(fixed[0]);
+    static_assert(nf == sizeof(sizes) / sizeof(sizes[0]), "one size per vector");
     size_t total = 0;
-    for (size_t k = 0; k < 8; k++) total += sizes[k] + 32;
+    for (size_t k = 0; k < nf; k++) total += sizes[k] + 32;
     total += nk * ((size_t)std::max(S.nig, 1) + 32);
     for (DBuf<double> *b : fixed) b->release();
     for (DBuf<double> *b : krylov) b->release();
     D.vblock.alloc(total);
     size_t off = 0;
-    for (size_t k = 0; k < 8; k++) fixed[k]->carve(D.vblock, off, sizes[k]);
+    for (size_t k = 0; k < nf; k++) fixed[k]->carve(D.vblock, off, sizes[k]);
     for (DBuf<double> *b : krylov) b->carve(D.vblock, off, std::max(S.nig, 1));
   }
   D.plan2b.add(D.fixmask, std::vector<char>(S.ig_fixed.begin(), S.ig_fixed.end()));
@@ -2592,10 +2596,10 @@ static void op_schur(Solver &S, const double *x, double *y, bool timed = false) 
   }
   if (D.f32i)
     launch_symv(D.st, (const float *)D.ipool32.p, D.scols.p, D.nscols, D.srows.p, D.nsrows,
-                D.loff.p, D.map.p, nullptr, x, D.spart.p, D.yl.p);
+                D.loff.p, D.map.p, x, D.spart.p, D.yl.p);
   else
     launch_symv(D.st, (const double *)D.pool.p, D.scols.p, D.nscols, D.srows.p, D.nsrows,
-                D.loff.p, D.map.p, nullptr, x, D.spart.p, D.yl.p);
+                D.loff.p, D.map.p, x, D.spart.p, D.yl.p);
   if (timed) {
     HIPCHECK(hipEventRecord(D.ev_apply[1], D.st));
     double tiles = 0;
@@ -2680,7 +2684,9 @@ static void op_pc(Solver &S, const double *r, double *z, bool timed) {
   if (D.inv_auto && !D.explicit_inv) ++D.pc_count;
   // coarse correction uc = Ac^{-1} sum_i R_ci^T Phi_i^T W_i r_i (three
   // levels: the second level's BDDC in place of Ac^{-1})
-  launch_phit(st, D.desc.p, S.nsub, D.Phi.p, D.map.p, D.w.p, r, D.rcs.p, D.maxnc, D.maxNI);
+  // (with the explicit inverse also Z_i^T W_i r_i, for the local part below)
+  launch_phit(st, D.desc.p, S.nsub, D.Phi.p, D.explicit_inv ? D.Z.p : nullptr, D.map.p, D.w.p, r,
+              D.rcs.p, D.zts.p, D.maxnc, D.maxNI);
   launch_coarse_gather(st, S.ndofc, D.cgptr.p, D.cgsrc.p, D.rcs.p, D.rc.p);
   if (S.lev2)
     level2_apply(S, D.rc.p, D.uc.p);
@@ -2691,23 +2697,17 @@ static void op_pc(Solver &S, const double *r, double *z, bool timed) {
     timing_events(D);
     HIPCHECK(hipEventRecord(D.ev_apply[2], st));
   }
-  // explicit inverse: yl = S'^{-1} (w .* r) by the symmetric tile GEMV
-  const double *ysym = nullptr;
-  if (D.explicit_inv) {
-    if (D.mixed)
-      launch_symv(st, (const float *)D.pool32.p, D.pcols.p, D.nscols, D.srows.p, D.nsrows,
-                  D.loff.p, D.map.p, D.w.p, r, D.spart.p, D.yl.p);
+  auto local = [&](const auto *fp) {
+    if (D.explicit_inv)
+      launch_inverse_apply(st, fp, D.pcols.p, D.nscols, D.srows.p, D.nsrows, D.desc.p, D.loff.p,
+                           D.map.p, D.w.p, r, D.spart.p, D.Phi.p, D.cmap.p, D.uc.p, D.zts.p,
+                           D.zl.p, D.maxnc);
     else
-      launch_symv(st, (const double *)D.fpool.p, D.pcols.p, D.nscols, D.srows.p, D.nsrows,
-                  D.loff.p, D.map.p, D.w.p, r, D.spart.p, D.yl.p);
-    ysym = D.yl.p;
-  }
-  if (D.mixed)
-    launch_kapply(st, (const float *)D.pool32.p, D.desc.p, S.nsub, D.map.p, D.w.p, r, D.Phi.p,
-                  D.Z.p, D.cmap.p, D.uc.p, ysym, D.zl.p, D.maxNI, D.maxnc, D.kapply_deep);
-  else
-    launch_kapply(st, (const double *)D.fpool.p, D.desc.p, S.nsub, D.map.p, D.w.p, r, D.Phi.p,
-                  D.Z.p, D.cmap.p, D.uc.p, ysym, D.zl.p, D.maxNI, D.maxnc, D.kapply_deep);
+      launch_kapply(st, fp, D.desc.p, S.nsub, D.map.p, D.w.p, r, D.Phi.p, D.Z.p, D.cmap.p, D.uc.p,
+                    D.zl.p, D.maxNI, D.maxnc, D.kapply_deep);
+  };
+  if (D.mixed) local((const float *)D.pool32.p);
+  else local((const double *)D.fpool.p);
   if (timed) {
     HIPCHECK(hipEventRecord(D.ev_apply[3], st));
     D.kapply_timed = true;

@@ -249,7 +249,7 @@ void launch_tile_gemv(hipStream_t st, const double *pool, const GemvTask *tasks,
 template <typename T>
 void launch_symv(hipStream_t st, const T *pool, const SymvCol *cols, int ncols,
                  const SymvRow *rows, int nrows, const int64_t *loff, const int *map,
-                 const double *wts, const double *xin, double *part, double *yout);
+                 const double *xin, double *part, double *yout);
 // y = A x for a dense nt x nt tile matrix in full storage (tile (I, J) at
 // base + I*nt + J); part holds nt*nt*64 doubles (coarse inverse)
 void launch_dense_gemv(hipStream_t st, const double *pool, int base, int nt, const double *x,
@@ -258,22 +258,29 @@ void launch_dense_gemv(hipStream_t st, const double *pool, int base, int nt, con
 void launch_assemble(hipStream_t st, int n, const int *ptr, const int64_t *src, const double *w,
                      const double *ylocal, double *y);
 // rc_s = Phi_s^T (w .* x_gathered)  -> coarse residual assembled by ptr/src
-void launch_phit(hipStream_t st, const SubDesc *subs, int nsub, const double *Phi,
-                 const int *map, const double *w, const double *x, double *rcs, int maxnc,
-                 int maxNI);
+void launch_phit(hipStream_t st, const SubDesc *subs, int nsub, const double *Phi, const double *Z,
+                 const int *map, const double *w, const double *x, double *rcs, double *zts,
+                 int maxnc, int maxNI);
 void launch_coarse_gather(hipStream_t st, int n, const int *ptr, const int *src,
                           const double *rcs, double *rc);
 // Local part of the BDDC preconditioner on every subdomain, one workgroup
 // each: x = w .* r(map); z = S'^{-1} x through the packed factor of S'
 // (forward and backward tile sweeps); zl = z + Phi (uc(indrowc) - Z^T x).
 // deep: more loads in flight per workgroup at lower occupancy, for few or
-// uneven subdomains (same arithmetic, same results).  ysym (may be null):
-// S'^{-1} x already applied by an explicit inverse; the sweeps are skipped.
+// uneven subdomains (same arithmetic, same results).
 template <typename T>
 void launch_kapply(hipStream_t st, const T *pool, const SubDesc *subs, int nsub, const int *map,
                    const double *w, const double *r, const double *Phi, const double *Z,
-                   const int *cmap, const double *uc, const double *ysym, double *zl, int maxNI,
-                   int maxnc, bool deep);
+                   const int *cmap, const double *uc, double *zl, int maxNI, int maxnc, bool deep);
+// The same local part through the explicit inverse: z = S'^{-1} x by the
+// symmetric tile GEMV over cols (tiles of the factor pool), summed per tile
+// row together with Phi (uc(indrowc) - zts); zts = Z^T x from launch_phit.
+template <typename T>
+void launch_inverse_apply(hipStream_t st, const T *pool, const SymvCol *cols, int ncols,
+                          const SymvRow *rows, int nrows, const SubDesc *subs, const int64_t *loff,
+                          const int *map, const double *wts, const double *xin, double *part,
+                          const double *Phi, const int *cmap, const double *uc, const double *zts,
+                          double *zl, int maxnc);
 
 // deterministic reductions and vector updates on unique vectors
 constexpr int DOT_BLOCKS = 240;

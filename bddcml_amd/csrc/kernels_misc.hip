@@ -727,22 +727,75 @@ __global__ __launch_bounds__(256) void k_symv_reduce(const SymvRow *__restrict__
   yout[loff[R.mat] + R.I * 64 + r] = s;
 }
 
+// The same sums with the coarse-basis part of the local preconditioner
+// added: zl = S'^{-1} x (slots of k_symv over the explicit inverse) + Phi cc,
+// cc = uc(indrowc) - Z^T x (zts).  One workgroup per tile row, its four waves
+// taking every fourth slot and every fourth column of Phi (512-byte column
+// loads), so the read of Phi (HBM-bound) spreads over all tile rows of the
+// chip: as the tail of a one-workgroup-per-subdomain kernel, Z^T x and Phi cc
+// took 386 us for 36 uneven elasticity subdomains of up to 12,000 dofs and
+// 65 us for 512 Poisson subdomains of 16^3.
+__global__ __launch_bounds__(256) void k_symv_reduce_phi(
+    const SymvRow *__restrict__ rows, const SubDesc *__restrict__ subs,
+    const double *__restrict__ part, const double *__restrict__ Phi, const int *__restrict__ cmap,
+    const double *__restrict__ uc, const double *__restrict__ zts, double *__restrict__ zl) {
+  extern __shared__ double cc[];  // nc
+  __shared__ double red[4][64];
+  const SymvRow R = rows[blockIdx.x];
+  const SubDesc d = subs[R.mat];
+  const int w = threadIdx.x >> 6, r = threadIdx.x & 63;
+  for (int c = threadIdx.x; c < d.nc; c += 256) cc[c] = uc[cmap[d.coff + c]] - zts[d.coff + c];
+  double s = 0.0;
+#pragma unroll 4
+  for (int J = w; J <= R.I; J += 4)
+    s += part[(size_t)(R.psub + J * R.nti - J * (J - 1) / 2 + (R.I - J)) * 64 + r];
+  __syncthreads();
+  const double *P = Phi + d.zoff + R.I * 64 + r;
+#pragma unroll 4
+  for (int c = w; c < d.nc; c += 4) s += P[(size_t)c * d.NI] * cc[c];
+  red[w][r] = s;
+  __syncthreads();
+  if (w == 0) zl[d.loff + R.I * 64 + r] = (red[0][r] + red[1][r]) + (red[2][r] + red[3][r]);
+}
+
 template <typename T>
 void launch_symv(hipStream_t st, const T *pool, const SymvCol *cols, int ncols,
                  const SymvRow *rows, int nrows, const int64_t *loff, const int *map,
-                 const double *wts, const double *xin, double *part, double *yout) {
+                 const double *xin, double *part, double *yout) {
   if (ncols <= 0 || nrows <= 0) return;
-  hipLaunchKernelGGL(k_symv<T>, dim3(ncols), dim3(256), 0, st, pool, cols, loff, map, wts, xin,
+  hipLaunchKernelGGL(k_symv<T>, dim3(ncols), dim3(256), 0, st, pool, cols, loff, map, nullptr, xin,
                      part);
   hipLaunchKernelGGL(k_symv_reduce, dim3((nrows + 3) / 4), dim3(256), 0, st, rows, nrows, loff,
                      part, yout);
 }
+template <typename T>
+void launch_inverse_apply(hipStream_t st, const T *pool, const SymvCol *cols, int ncols,
+                          const SymvRow *rows, int nrows, const SubDesc *subs, const int64_t *loff,
+                          const int *map, const double *wts, const double *xin, double *part,
+                          const double *Phi, const int *cmap, const double *uc, const double *zts,
+                          double *zl, int maxnc) {
+  if (ncols <= 0 || nrows <= 0) return;
+  hipLaunchKernelGGL(k_symv<T>, dim3(ncols), dim3(256), 0, st, pool, cols, loff, map, wts, xin,
+                     part);
+  hipLaunchKernelGGL(k_symv_reduce_phi, dim3(nrows), dim3(256), (size_t)maxnc * sizeof(double), st,
+                     rows, subs, part, Phi, cmap, uc, zts, zl);
+}
+template void launch_inverse_apply<double>(hipStream_t, const double *, const SymvCol *, int,
+                                           const SymvRow *, int, const SubDesc *, const int64_t *,
+                                           const int *, const double *, const double *, double *,
+                                           const double *, const int *, const double *,
+                                           const double *, double *, int);
+template void launch_inverse_apply<float>(hipStream_t, const float *, const SymvCol *, int,
+                                          const SymvRow *, int, const SubDesc *, const int64_t *,
+                                          const int *, const double *, const double *, double *,
+                                          const double *, const int *, const double *,
+                                          const double *, double *, int);
 template void launch_symv<double>(hipStream_t, const double *, const SymvCol *, int,
                                   const SymvRow *, int, const int64_t *, const int *,
-                                  const double *, const double *, double *, double *);
+                                  const double *, double *, double *);
 template void launch_symv<float>(hipStream_t, const float *, const SymvCol *, int, const SymvRow *,
-                                 int, const int64_t *, const int *, const double *, const double *,
-                                 double *, double *);
+                                 int, const int64_t *, const int *, const double *, double *,
+                                 double *);
 
 // Block-sparse tile GEMV, one workgroup per output segment of 64:
 // y[yoff..] = (b ? b[boff..] : 0) + sign * sum_p op(T_p) x[xoff_p..], op the
@@ -876,7 +929,9 @@ __device__ __forceinline__ int packed_lower(int n, int I, int J) {
 }
 
 
-// rcs = Phi_i^T (w .* r(map)) per subdomain: the weighted interface vector is
+// rcs = Phi_i^T (w .* r(map)) per subdomain, and with the explicit inverse
+// zts = Z_i^T (w .* r(map)) by the second half of the grid (chunks workgroups
+// per matrix and subdomain): the weighted interface vector is
 // gathered into LDS once per block (STAGE; otherwise, for interfaces too
 // large for LDS, per column from global memory), then each wave reduces
 // PHIT_COLS / 4 of the block's PHIT_COLS columns of Phi_i (contiguous,
@@ -885,14 +940,19 @@ constexpr int PHIT_COLS = 16;
 template <bool STAGE>
 __global__ __launch_bounds__(256) void k_phit(const SubDesc *__restrict__ subs,
                                               const double *__restrict__ Phi,
+                                              const double *__restrict__ Z, int chunks,
                                               const int *__restrict__ map,
                                               const double *__restrict__ w,
                                               const double *__restrict__ x,
-                                              double *__restrict__ rcs) {
+                                              double *__restrict__ rcs,
+                                              double *__restrict__ zts) {
   extern __shared__ double xw[];
   const SubDesc d = subs[blockIdx.y];
-  const int c0 = blockIdx.x * PHIT_COLS;
+  const bool of_z = (int)blockIdx.x >= chunks;
+  const int c0 = ((int)blockIdx.x - (of_z ? chunks : 0)) * PHIT_COLS;
   if (c0 >= d.nc) return;
+  const double *M = of_z ? Z : Phi;
+  double *out = of_z ? zts : rcs;
   const int NI = d.NI;
   if (STAGE) {
     for (int i = threadIdx.x; i < NI; i += 256) {
@@ -912,7 +972,7 @@ __global__ __launch_bounds__(256) void k_phit(const SubDesc *__restrict__ subs,
 #pragma unroll
   for (int k = 0; k < CPW; k++) {
     const int c = min(c0 + wave + 4 * k, cend - 1);  // a column past the end reads a valid one
-    pc[k] = Phi + d.zoff + (size_t)c * NI;
+    pc[k] = M + d.zoff + (size_t)c * NI;
     s[k] = 0.0;
   }
   for (int i = lane; i < NI; i += 64) {
@@ -930,7 +990,7 @@ __global__ __launch_bounds__(256) void k_phit(const SubDesc *__restrict__ subs,
   for (int k = 0; k < CPW; k++) {
     const double t = wave_sum(s[k]);
     const int c = c0 + wave + 4 * k;
-    if (lane == 0 && c < cend) rcs[d.coff + c] = t;
+    if (lane == 0 && c < cend) out[d.coff + c] = t;
   }
 }
 
@@ -953,7 +1013,7 @@ __global__ __launch_bounds__(KA_THR) void k_kapply(
     const T *__restrict__ pool, const SubDesc *__restrict__ subs, const int *__restrict__ map,
     const double *__restrict__ w, const double *__restrict__ rin, const double *__restrict__ Phi,
     const double *__restrict__ Z, const int *__restrict__ cmap, const double *__restrict__ uc,
-    const double *__restrict__ ysym, double *zl) {
+    double *zl) {
   extern __shared__ double smem[];
   const SubDesc d = subs[blockIdx.x];
   const int NI = d.NI, nc = d.nc, n = d.nti;
@@ -976,12 +1036,6 @@ __global__ __launch_bounds__(KA_THR) void k_kapply(
     s = wave_sum(s);
     if (l == 0) cc[c] = uc[cmap[d.coff + c]] - s;
   }
-  if (ysym) {
-    // S'^{-1} x already applied (explicit inverse, symmetric GEMV): no sweeps
-    publish_sync<GV>();
-    for (int i = tid; i < NI; i += KA_THR) xs[i] = ysym[d.loff + i];
-    publish_sync<GV>();
-  } else {
   // forward sweep x_I <- Linv_I (x_I - sum_{k<I} L_Ik x_k); lane = tile row.
   // The Linv_I entries are loaded before the row sum (they do not depend on
   // it), and four tiles of the row are in flight at a time.
@@ -1085,7 +1139,6 @@ __global__ __launch_bounds__(KA_THR) void k_kapply(
     }
     publish_sync<GV>();
   }
-  }
   publish_sync<GV>();
   for (int i = tid; i < NI; i += KA_THR) {
     double s = xs[i];
@@ -1099,16 +1152,20 @@ void launch_assemble(hipStream_t st, int n, const int *ptr, const int64_t *src, 
   if (n <= 0) return;
   hipLaunchKernelGGL(k_assemble, dim3((n + 255) / 256), dim3(256), 0, st, n, ptr, src, w, ylocal, y);
 }
-void launch_phit(hipStream_t st, const SubDesc *subs, int nsub, const double *Phi, const int *map,
-                 const double *w, const double *x, double *rcs, int maxnc, int maxNI) {
+void launch_phit(hipStream_t st, const SubDesc *subs, int nsub, const double *Phi, const double *Z,
+                 const int *map, const double *w, const double *x, double *rcs, double *zts,
+                 int maxnc, int maxNI) {
   if (nsub <= 0 || maxnc <= 0) return;
   const size_t sh = (size_t)std::max(maxNI, 1) * sizeof(double);
-  const dim3 grid((maxnc + PHIT_COLS - 1) / PHIT_COLS, nsub);
+  const int chunks = (maxnc + PHIT_COLS - 1) / PHIT_COLS;
+  const dim3 grid(Z ? 2 * chunks : chunks, nsub);
   if (sh <= max_dynamic_lds() && !g_trsv_global) {
     lds_request((const void *)k_phit<true>, sh, "coarse residual");
-    hipLaunchKernelGGL(k_phit<true>, grid, dim3(256), sh, st, subs, Phi, map, w, x, rcs);
+    hipLaunchKernelGGL(k_phit<true>, grid, dim3(256), sh, st, subs, Phi, Z, chunks, map, w, x, rcs,
+                       zts);
   } else {
-    hipLaunchKernelGGL(k_phit<false>, grid, dim3(256), 0, st, subs, Phi, map, w, x, rcs);
+    hipLaunchKernelGGL(k_phit<false>, grid, dim3(256), 0, st, subs, Phi, Z, chunks, map, w, x, rcs,
+                       zts);
   }
 }
 void launch_coarse_gather(hipStream_t st, int n, const int *ptr, const int *src,
@@ -1119,8 +1176,7 @@ void launch_coarse_gather(hipStream_t st, int n, const int *ptr, const int *src,
 template <typename T>
 void launch_kapply(hipStream_t st, const T *pool, const SubDesc *subs, int nsub, const int *map,
                    const double *w, const double *r, const double *Phi, const double *Z,
-                   const int *cmap, const double *uc, const double *ysym, double *zl, int maxNI,
-                   int maxnc, bool deep) {
+                   const int *cmap, const double *uc, double *zl, int maxNI, int maxnc, bool deep) {
   if (nsub <= 0) return;
   const size_t sh = (size_t)(maxNI + 1024 + 64 + maxnc) * sizeof(double);
   const size_t sg = (size_t)(1024 + 64 + maxnc) * sizeof(double);
@@ -1128,24 +1184,23 @@ void launch_kapply(hipStream_t st, const T *pool, const SubDesc *subs, int nsub,
   auto go = [&](auto kernel, size_t bytes) {
     lds_request((const void *)kernel, bytes, "preconditioner apply");
     hipLaunchKernelGGL(kernel, dim3(nsub), dim3(KA_THR), bytes, st, pool, subs, map, w, r, Phi, Z,
-                       cmap, uc, ysym, zl);
+                       cmap, uc, zl);
   };
   if (gv) {
-    if (deep && !ysym) go(k_kapply<T, true, true>, sg);
+    if (deep) go(k_kapply<T, true, true>, sg);
     else go(k_kapply<T, false, true>, sg);
   } else {
-    if (deep && !ysym) go(k_kapply<T, true, false>, sh);
+    if (deep) go(k_kapply<T, true, false>, sh);
     else go(k_kapply<T, false, false>, sh);
   }
 }
 template void launch_kapply<double>(hipStream_t, const double *, const SubDesc *, int, const int *,
                                     const double *, const double *, const double *,
-                                    const double *, const int *, const double *, const double *,
-                                    double *, int, int, bool);
+                                    const double *, const int *, const double *, double *, int, int,
+                                    bool);
 template void launch_kapply<float>(hipStream_t, const float *, const SubDesc *, int, const int *,
                                    const double *, const double *, const double *, const double *,
-                                   const int *, const double *, const double *, double *, int, int,
-                                   bool);
+                                   const int *, const double *, double *, int, int, bool);
 
 // ------------------------------------------------------------ vector ops
 __global__ __launch_bounds__(256) void k_dots(int n, DotArgs a, double *__restrict__ partial) {
