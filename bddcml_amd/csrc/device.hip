@@ -312,9 +312,10 @@ struct Device {
   Phase a_schur, cinv, phi, kinv;
   // explicit inverse of S': planned (W tiles in the factor space, task
   // lists, GEMV columns), formed (W = L^{-1}, W^T W: the apply is a GEMV),
-  // automatic (formed once the preconditioner has been applied
-  // kInverseAfterApplies times on this setup)
+  // automatic (formed once the preconditioner has been applied inv_after
+  // times on this setup)
   bool inv_planned = false, explicit_inv = false, inv_auto = false;
+  double inv_after = 0.0;
   int pc_count = 0;
   std::vector<SeqPhase> cseq;  // coarse factorization and inverse
   Arena plan0;  // scatter tables and tiles to clear (uploaded first)
@@ -1408,6 +1409,42 @@ static double interface_rho(const Sub &s) {
   return rho > 0.0 ? rho : 1.0;
 }
 
+// Applies after which the explicit inverse of S' has paid for itself: the
+// time of forming it over what an apply saves, from the tile counts (tile
+// rows n of each subdomain's S', its factor's element size).  The constants
+// were fitted on one MI355X over Poisson, elasticity and uneven boxes, 8 to
+// 512 subdomains, n = 1 to 76:
+//  - forming: tile products at 50 / 95 TFLOP/s (FP64 / FP32) behind one
+//    launch per tile row (10 us) whose longest task is a chain of products
+//    (2.6 / 1.9 us each);
+//  - an apply by sweeps: the larger of the slowest workgroup (3.4 us per
+//    tile row and direction, 0.7 / 0.4 us per tile) and both reads of the
+//    factors at 5.5 TB/s; by the inverse: one read at 4.7 TB/s and 15 us.
+// FP64, ms formed / sweeps / inverse: 64 subdomains n = 25: 2.9 / 0.60 / 0.10
+// (pays after 6); 36 boxes n <= 49: 8.7 / 2.25 / 0.17 (4); 60 boxes n <= 76:
+// 35.6 / 5.1 / 0.50 (8); 216 subdomains n = 25: 9.5 / 0.76 / 0.36 (23); 512:
+// 24 / 1.57 / 0.92 (37).
+static double inverse_pays_after(const std::vector<SubTiles> &sub, bool f32) {
+  double prods = 0.0, tiles = 0.0;
+  int nmax = 0;
+  for (const SubTiles &T : sub) {
+    const double n = T.nti;
+    prods += n * (n + 1.0) * (n + 2.0) / 6.0 + n * (n - 1.0) * (n + 4.0) / 6.0;
+    tiles += 0.5 * n * (n + 1.0);
+    nmax = std::max(nmax, T.nti);
+  }
+  const double n = nmax, bytes = tiles * TILE_ELEMS * (f32 ? 4.0 : 8.0);
+  const double form = prods * kTileGemm / (f32 ? 95e12 : 50e12) + n * 10e-6 +
+                      0.5 * n * (n - 1.0) * (f32 ? 1.9e-6 : 2.6e-6);
+  const double sweeps = std::max(2.0 * n * 3.4e-6 + n * (n + 1.0) * (f32 ? 0.4e-6 : 0.7e-6),
+                                 2.0 * bytes / 5.5e12);
+  const double saved = sweeps - (bytes / 4.7e12 + 15e-6);
+  return saved > 0.0 ? form / saved : 1e30;
+}
+// a solve rarely takes fewer applies than this: an inverse that pays for
+// itself within it is formed at setup
+constexpr double kInverseAtSetup = 8.0;
+
 // Second half of the setup, first part: everything that needs the
 // constraints but not the interface numbering, the weights or the
 // right-hand side -- the factor space, the S' / Z / Phi lists, the
@@ -1441,6 +1478,11 @@ void device_setup_interface(Solver &S) {
     D.inv_planned = S.explicit_inverse != 0 || S.adapt_pass;
     D.inv_auto = S.explicit_inverse == 2 && !S.adapt_pass;
     D.explicit_inv = false;
+    D.pc_count = 0;
+    D.inv_after = inverse_pays_after(D.sub, D.mixed);
+    // (a caller that sets the form of the sweeps gets sweeps first)
+    if (D.inv_auto && D.inv_after <= kInverseAtSetup && S.pc_form == 0 && launch_forms() == 0)
+      D.inv_auto = false;
     for (int is = 0; is < nsub; is++) assign_factor(D.sub[is], S.subs[is].nconstr, nf, D.inv_planned);
     if (nf >= INT32_MAX) fatal("BDDCML_DEVICE_PLAN", "too many factor tiles");
     D.ntilesf = nf;
@@ -2664,17 +2706,13 @@ static void level2_apply(Solver &S, const double *rc, double *uc) {
   launch_level_gather(st, S.ndofc, D.l2pos.p, E.vec.p, uc);
 }
 
-// applies after which the automatic mode forms the explicit inverse: about
-// the number whose saving (roughly half an apply each) pays for forming it
-constexpr int kInverseAfterApplies = 40;
-
 // automatic explicit inverse, at a solve boundary only (so that one Krylov
 // run sees one preconditioner): formed on every level whose preconditioner
-// has been applied kInverseAfterApplies times on this setup
+// has been applied as often as pays for it on this setup
 static void inverse_at_solve_start(Solver &S) {
   for (Solver *L = &S; L && L->dev; L = L->lev2.get()) {
     Device &D = *L->dev;
-    if (D.inv_auto && !D.explicit_inv && D.pc_count >= kInverseAfterApplies) form_inverse(*L);
+    if (D.inv_auto && !D.explicit_inv && D.pc_count >= D.inv_after) form_inverse(*L);
   }
 }
 

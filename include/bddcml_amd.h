@@ -120,10 +120,10 @@ int bddcml_amd_timings(double *out, int n);
  *   "explicit_inverse" (S'^{-1} formed, W = L^{-1} and W^T W on the tile
  *     GEMM, so that each preconditioner apply reads it once in a symmetric
  *     GEMV instead of sweeping the factor twice: 0 never; 1 at setup; 2, the
- *     default, at the start of the first solve after the preconditioner has
- *     been applied 40 times on the same setup, where the saved apply time
- *     has about paid for forming it; a solve never changes its
- *     preconditioner while it runs) */
+ *     default, at setup where about eight applies pay for forming it (few or
+ *     large subdomains, estimated from the tile counts), else at the start of
+ *     the first solve after as many applies as pay for it have run on the
+ *     same setup; a solve never changes its preconditioner while it runs) */
 int bddcml_amd_set_option(const char *key, double value);
 /* per subdomain (isub in numbase): out[0]=ndofi out[1]=nconstr out[2]=ndofo */
 int bddcml_amd_sub_info(int isub, int *out);
