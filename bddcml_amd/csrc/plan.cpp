@@ -418,7 +418,7 @@ struct Fnv {
   }
   // size and every 61st element: enough to separate classes cheaply, since
   // candidates are confirmed by a full comparison
-  template <class T> void sample(const std::vector<T> &v) {
+  template <class T, class A> void sample(const std::vector<T, A> &v) {
     add((uint64_t)v.size());
     for (size_t k = 0; k < v.size(); k += 61) add((uint64_t)v[k]);
     if (!v.empty()) add((uint64_t)v.back());
@@ -612,8 +612,8 @@ static void eliminate_bc(Sub &s) {
     std::sort(o.begin(), o.end(), [&](size_t a, size_t b) {
       return s.ai[a] != s.ai[b] ? s.ai[a] < s.ai[b] : s.aj[a] < s.aj[b];
     });
-    std::vector<int> ai(o.size()), aj(o.size());
-    std::vector<double> av(o.size());
+    RawInts ai(o.size()), aj(o.size());
+    RawVec<double> av(o.size());
     for (size_t k = 0; k < o.size(); k++) ai[k] = s.ai[o[k]], aj[k] = s.aj[o[k]], av[k] = s.av[o[k]];
     s.ai.swap(ai);
     s.aj.swap(aj);

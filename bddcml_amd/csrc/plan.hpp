@@ -8,10 +8,27 @@
 #pragma once
 
 #include <cstdint>
+#include <memory>
 #include <stdexcept>
 #include <utility>
 #include <string>
 #include <vector>
+
+// std::vector whose resize leaves new elements uninitialized (the assembled
+// triplets and the large node tables are filled in parallel right after)
+template <class T, class A = std::allocator<T>>
+struct NoInitAlloc : A {
+  using A::A;
+  template <class U> struct rebind {
+    using other = NoInitAlloc<U, typename std::allocator_traits<A>::template rebind_alloc<U>>;
+  };
+  template <class U> void construct(U *p) noexcept { ::new (static_cast<void *>(p)) U; }
+  template <class U, class... Args> void construct(U *p, Args &&...args) {
+    std::allocator_traits<A>::construct(static_cast<A &>(*this), p, std::forward<Args>(args)...);
+  }
+};
+template <class T> using RawVec = std::vector<T, NoInitAlloc<T>>;
+using RawInts = RawVec<int>;
 
 namespace bddc {
 
@@ -44,8 +61,8 @@ struct Sub {
   int nuser_c = 0;
   int find_components = 0, use_dual = 0, neighbouring = 1;
   // assembled upper triangle (sorted by row, col; duplicates summed)
-  std::vector<int> ai, aj;
-  std::vector<double> av;
+  RawInts ai, aj;
+  RawVec<double> av;
 
   // ---- topology --------------------------------------------------------
   std::vector<int> kdof;    // first dof of each node (nnods+1)

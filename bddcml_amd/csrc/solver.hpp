@@ -12,22 +12,6 @@
 
 #include "plan.hpp"
 
-// std::vector whose resize leaves new elements uninitialized (the large
-// node tables are filled in parallel right after)
-template <class T, class A = std::allocator<T>>
-struct NoInitAlloc : A {
-  using A::A;
-  template <class U> struct rebind {
-    using other = NoInitAlloc<U, typename std::allocator_traits<A>::template rebind_alloc<U>>;
-  };
-  template <class U> void construct(U *p) noexcept { ::new (static_cast<void *>(p)) U; }
-  template <class U, class... Args> void construct(U *p, Args &&...args) {
-    std::allocator_traits<A>::construct(static_cast<A &>(*this), p, std::forward<Args>(args)...);
-  }
-};
-template <class T> using RawVec = std::vector<T, NoInitAlloc<T>>;
-using RawInts = RawVec<int>;
-
 namespace bddc {
 
 struct Device;       // device-side plan and buffers (device.hip)
