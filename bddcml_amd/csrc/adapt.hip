@@ -54,6 +54,7 @@
 #include <string>
 #include <vector>
 
+#include "devmem.hpp"
 #include "kernels.hpp"
 #include "solver.hpp"
 
@@ -558,12 +559,12 @@ template <class T> struct ABuf {
   ABuf(const ABuf &) = delete;
   ABuf &operator=(const ABuf &) = delete;
   ~ABuf() {
-    if (p) (void)hipFree(p);
+    dev_free(p);
   }
   void alloc(size_t cnt) {
-    if (p) (void)hipFree(p);
+    dev_free(p);
     n = cnt;
-    AD_CHECK(hipMalloc(&p, std::max<size_t>(cnt, 1) * sizeof(T)));
+    p = static_cast<T *>(dev_alloc(std::max<size_t>(cnt, 1) * sizeof(T)));
   }
   void swap(ABuf &o) {
     std::swap(p, o.p);

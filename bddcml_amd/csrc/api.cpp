@@ -23,10 +23,12 @@ Solver &solver() {
 }
 void reset_solver() {
   if (g_solver) {
+    const bool held = g_solver->initialised;
     device_release(*g_solver);
     delete g_solver;
+    g_solver = nullptr;
+    if (held) device_end_of_problem(false);
   }
-  g_solver = nullptr;
 }
 
 static std::string g_last_error;
@@ -650,7 +652,11 @@ catch (const Error &e) {
   record_error(e);
 }
 
-void bddcml_finalize_c() try { reset_solver(); }
+void bddcml_finalize_c() try {
+  const bool held = g_solver && g_solver->initialised;
+  reset_solver();
+  if (!held) device_end_of_problem(true);  // nothing to end: kept memory goes back
+}
 catch (const Error &e) {
   record_error(e);
 }

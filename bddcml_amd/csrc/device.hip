@@ -32,6 +32,7 @@
 #include <thread>
 #include <unordered_map>
 
+#include "devmem.hpp"
 #include "kernels.hpp"
 #include "solver.hpp"
 
@@ -85,7 +86,7 @@ struct DBuf {
   }
   ~DBuf() { release(); }
   void release() {
-    if (p && owned) (void)hipFree(p);
+    if (p && owned) dev_free(p);
     p = nullptr;
     n = 0;
     owned = true;
@@ -108,7 +109,7 @@ struct DBuf {
     const double t = wall_time();
     release();
     n = cnt;
-    HIPCHECK(hipMalloc(&p, std::max<size_t>(cnt, 1) * sizeof(T)));
+    p = static_cast<T *>(dev_alloc(std::max<size_t>(cnt, 1) * sizeof(T)));
     g_alloc_s += wall_time() - t;
   }
   void upload(const std::vector<T> &v, hipStream_t st) {
@@ -535,6 +536,8 @@ void device_upload_entries(Solver &S, int is) {
 
 void device_release_input(Solver &S) { S.din.reset(); }
 
+void device_end_of_problem(bool nothing_held) { devmem_end_of_problem(nothing_held); }
+
 void device_release(Solver &S) {
   if (S.lev2) {  // borrows this level's stream: released first
     device_release(*S.lev2);
@@ -546,7 +549,7 @@ void device_release(Solver &S) {
     Device &D = *S.dev;
     if (D.st) (void)hipStreamSynchronize(D.st);
     if (D.up) (void)hipStreamSynchronize(D.up);
-    if (D.hrr) (void)hipHostFree(D.hrr), D.hrr = nullptr;
+    pinned_free(D.hrr), D.hrr = nullptr;
     if (D.pcg_exec) (void)hipGraphExecDestroy(D.pcg_exec), D.pcg_exec = nullptr;
     if (D.pcg_graph) (void)hipGraphDestroy(D.pcg_graph), D.pcg_graph = nullptr;
     for (hipEvent_t &e : D.ev)
@@ -557,8 +560,8 @@ void device_release(Solver &S) {
       if (e) (void)hipEventDestroy(e), e = nullptr;
     if (D.ev_up) (void)hipEventDestroy(D.ev_up), D.ev_up = nullptr;
     if (D.ev_rhs) (void)hipEventDestroy(D.ev_rhs), D.ev_rhs = nullptr;
-    if (D.st && !D.borrowed_st) (void)hipStreamDestroy(D.st);
-    if (D.up) (void)hipStreamDestroy(D.up);
+    if (!D.borrowed_st) stream_put(D.st);
+    stream_put(D.up);
     D.st = D.up = nullptr;
     S.dev.reset();
   }
@@ -825,8 +828,8 @@ void device_setup_begin(Solver &S) {
   device_release(S);
   S.dev.reset(new Device());
   Device &D = *S.dev;
-  HIPCHECK(hipStreamCreateWithFlags(&D.st, hipStreamNonBlocking));
-  HIPCHECK(hipStreamCreateWithFlags(&D.up, hipStreamNonBlocking));
+  D.st = stream_get();
+  D.up = stream_get();
   hipStream_t st = D.st;
   const int nsub = S.nsub;
   double t0 = wall_time();
@@ -2652,7 +2655,7 @@ void device_link_levels(Solver &S) {
   HIPCHECK(hipStreamSynchronize(E.st));
   HIPCHECK(hipStreamSynchronize(E.up));  // its own reduced rhs (unused) is done
   E.rhs_pending = false;
-  if (!E.borrowed_st) HIPCHECK(hipStreamDestroy(E.st));
+  if (!E.borrowed_st) stream_put(E.st);
   E.st = D.st;
   E.borrowed_st = true;
   // the levels below it borrowed its stream: they run on this one too
@@ -3126,11 +3129,10 @@ static void krylov(Solver &S, const double *rhs, int method, double tol, int max
     const size_t mc = D.pcg.n / 3;
     double *rz = D.pcg.p, *pap = D.pcg.p + mc, *rr = D.pcg.p + 2 * mc;
     if (D.hrr_n < m) {
-      if (D.hrr) (void)hipHostFree(D.hrr), D.hrr = nullptr;
+      pinned_free(D.hrr), D.hrr = nullptr;
       // mapped and coherent: the graph's dot kernel writes r.r here and the
       // host polls it
-      HIPCHECK(hipHostMalloc((void **)&D.hrr, m * sizeof(double),
-                             hipHostMallocMapped | hipHostMallocCoherent));
+      D.hrr = static_cast<double *>(pinned_alloc(m * sizeof(double)));
       HIPCHECK(hipHostGetDevicePointer((void **)&D.hrr_dev, D.hrr, 0));
       D.hrr_n = m;
     }

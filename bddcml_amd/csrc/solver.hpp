@@ -274,6 +274,9 @@ void device_element_gradient_noalloc(Solver &S, const double *ae, int nke, bool 
 void device_selftest_tile(int op, int npairs, const double *A, const double *B, const double *C,
                           const double *X, double alpha, double beta, double *out);
 void device_release(Solver &S);
+// device memory kept for the next problem (devmem.hpp): what the problem
+// that ends did not use goes back, with nothing_held all of it
+void device_end_of_problem(bool nothing_held);
 
 double wall_time();
 // ask the runtime to spin (not sleep) in host waits on the device; called
