@@ -1789,7 +1789,7 @@ void device_setup_interface(Solver &S) {
     D.plan2.add(D.cvals, cvalv);
     D.plan2.add(D.comega, omegav);
   }
-  // limits of the kernels: G^{-1} in place with one LDS row buffer (k_ginv),
+  // limits of the kernels: G^{-1} with a row and a column in LDS (k_ginv),
   // the whole interface vector of a subdomain in LDS (k_kapply), the coarse
   // matrix as full tiles
   if (D.maxnc > 1024) fatal("BDDCML_SETUP_PRECONDITIONER", "more than 1024 constraints per subdomain");
@@ -1934,8 +1934,8 @@ void device_setup_interface(Solver &S) {
   if (D.mixed) factor_phase(D.pool32.p);
   else factor_phase(D.fpool.p);
   launch_g(st, D.desc.p, nsub, D.cptr.p, D.cdof.p, D.gen_constraints ? D.cvals.p : nullptr, D.Z.p,
-           D.G.p);
-  launch_ginv(st, D.desc.p, nsub, D.G.p, nullptr, D.err.p);
+           D.G.p, D.maxnc);
+  launch_ginv(st, D.desc.p, nsub, D.G.p, D.err.p, D.maxnc);
   if (D.mixed) phi_phase(D.pool32.p);
   else phi_phase(D.fpool.p);
   if (D.inv_planned && !D.inv_auto) form_inverse(S);

@@ -135,8 +135,8 @@ void launch_ct_init_gen(hipStream_t st, T *pool, const SubDesc *subs, int nsub, 
 // G = C Z (row values cval, 1 when null), Ginv = G^{-1} (in place
 // Gauss-Jordan, SPD), Acs = Ginv - Omega (Omega_c = rho/|D_c|, or omega[c])
 void launch_g(hipStream_t st, const SubDesc *subs, int nsub, const int *cptr, const int *cdof,
-              const double *cval, const double *Z, double *G);
-void launch_ginv(hipStream_t st, const SubDesc *subs, int nsub, double *G, double *work, int *err);
+              const double *cval, const double *Z, double *G, int maxnc);
+void launch_ginv(hipStream_t st, const SubDesc *subs, int nsub, double *G, int *err, int maxnc);
 
 void launch_acs(hipStream_t st, const SubDesc *subs, int nsub, const int *cptr,
                 const double *omega, const double *G, double *Acs);

@@ -252,14 +252,18 @@ __global__ void k_y_to_z(const T *__restrict__ pool, const SubDesc *__restrict__
     Z[d.zoff + (size_t)c * d.NI + i] = (double)Y[(size_t)(c >> 6) * TILE_ELEMS + (c & 63) * 64];
 }
 
-// G = C Z over the constraint rows (values 1 when cval is null)
+// G = C Z over the constraint rows (values 1 when cval is null); a workgroup
+// takes KG_COLS columns of one subdomain (a whole subdomain per workgroup
+// left 12 to 64 of 256 CUs busy: 2.07 ms for 12 adaptive elasticity boxes on
+// average of the two setups, 0.13 ms now)
+constexpr int KG_COLS = 8;
 __global__ void k_g(const SubDesc *__restrict__ subs, const int *__restrict__ cptr,
                     const int *__restrict__ cdof, const double *__restrict__ cval,
                     const double *__restrict__ Z, double *__restrict__ G) {
   const SubDesc d = subs[blockIdx.x];
-  const int nc = d.nc;
-  for (int e = threadIdx.x; e < nc * nc; e += blockDim.x) {
-    int c = e / nc, k = e % nc;
+  const int nc = d.nc, k0 = blockIdx.y * KG_COLS, nk = min(KG_COLS, nc - k0);
+  for (int e = threadIdx.x; e < nc * nk; e += blockDim.x) {
+    const int c = e / nk, k = k0 + e % nk;
     double s = 0.0;
     for (int q = cptr[d.coff + c]; q < cptr[d.coff + c + 1]; q++)
       s += (cval ? cval[q] : 1.0) * Z[d.zoff + (size_t)k * d.NI + cdof[q]];
@@ -267,37 +271,106 @@ __global__ void k_g(const SubDesc *__restrict__ subs, const int *__restrict__ cp
   }
 }
 
-// in-place Gauss-Jordan inverse of the SPD matrices G (no pivoting)
-__global__ void k_ginv(const SubDesc *__restrict__ subs, double *__restrict__ G,
-                       int *__restrict__ err) {
-  __shared__ double F[1024];
-  __shared__ double inv;
+// In-place Gauss-Jordan inverse of the SPD matrices G (no pivoting), one
+// workgroup of 32 x 32 threads per matrix.  Thread (ty, tx) keeps the entries
+// (ty + 32 a, tx + 32 b) in registers; each of the n steps publishes the
+// scaled pivot row and the pivot column in LDS and updates every entry, two
+// barriers a step.  The n steps are a serial chain: with the matrix in global
+// memory and 256 threads 12 matrices of n = 129 to 160 took 2.19 ms, 64 of n
+// = 65 to 96 (elasticity, 32^3) 0.50 ms; now 0.24 and 0.079 ms.
+// M: rows and columns per thread, n <= 32 M; 36 entries still fit the 128
+// registers that 16 waves leave.
+template <int M>
+__global__ __launch_bounds__(1024) void k_ginv(const SubDesc *__restrict__ subs,
+                                               double *__restrict__ G, int *__restrict__ err) {
+  __shared__ double row[32 * M], col[32 * M];
   const SubDesc d = subs[blockIdx.x];
-  const int n = d.nc;
+  const int n = d.nc, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  if (n == 0) return;
   double *A = G + d.goff;  // A[i*n + j]
+  double v[M][M];
+#pragma unroll
+  for (int a = 0; a < M; a++)
+#pragma unroll
+    for (int b = 0; b < M; b++) {
+      const int i = ty + 32 * a, j = tx + 32 * b;
+      v[a][b] = i < n && j < n ? A[i * n + j] : 0.0;
+    }
+  for (int k = 0; k < n; k++) {
+    // column k and the unscaled row k (the pivot among both)
+#pragma unroll
+    for (int a = 0; a < M; a++) {
+      if (a == (k >> 5)) {
+        if (ty == (k & 31)) {
+#pragma unroll
+          for (int b = 0; b < M; b++) row[tx + 32 * b] = v[a][b];
+        }
+        if (tx == (k & 31)) {
+#pragma unroll
+          for (int b = 0; b < M; b++) col[ty + 32 * b] = v[b][a];
+        }
+      }
+    }
+    __syncthreads();
+    double p = row[k];
+    if (!(p > 0.0)) {
+      if (threadIdx.x == 0) atomicOr(err, 2);
+      p = 1.0;
+    }
+    const double inv = 1.0 / p;
+    double r[M], f[M];
+#pragma unroll
+    for (int b = 0; b < M; b++) {
+      const int j = tx + 32 * b;
+      r[b] = (j == k ? 1.0 : row[j]) * inv;
+    }
+#pragma unroll
+    for (int a = 0; a < M; a++) f[a] = col[ty + 32 * a];
+    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < M; a++) {
+      const int i = ty + 32 * a;
+#pragma unroll
+      for (int b = 0; b < M; b++) {
+        const int j = tx + 32 * b;
+        const double old = j == k ? 0.0 : v[a][b];
+        v[a][b] = i == k ? r[b] : old - f[a] * r[b];
+      }
+    }
+  }
+#pragma unroll
+  for (int a = 0; a < M; a++)
+#pragma unroll
+    for (int b = 0; b < M; b++) {
+      const int i = ty + 32 * a, j = tx + 32 * b;
+      if (i < n && j < n) A[i * n + j] = v[a][b];
+    }
+}
+// the same steps with the matrix in global memory (L2) and a row and a column
+// in LDS, for n above 192 (12 adaptive boxes: 8.2 -> 2.4 ms)
+__global__ __launch_bounds__(1024) void k_ginv_large(const SubDesc *__restrict__ subs,
+                                                     double *__restrict__ G,
+                                                     int *__restrict__ err) {
+  __shared__ double row[1024], col[1024];
+  const SubDesc d = subs[blockIdx.x];
+  const int n = d.nc, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  double *A = G + d.goff;
   for (int k = 0; k < n; k++) {
     __syncthreads();
-    if (threadIdx.x == 0) {
-      double p = A[k * n + k];
-      if (!(p > 0.0)) {
-        atomicOr(err, 2);
-        p = 1.0;
+    const double q = A[(size_t)k * n + k];
+    const double p = q > 0.0 ? q : 1.0;
+    if (!(q > 0.0) && threadIdx.x == 0) atomicOr(err, 2);
+    const double inv = 1.0 / p;
+    for (int j = threadIdx.x; j < n; j += 1024) {
+      row[j] = (j == k ? 1.0 : A[(size_t)k * n + j]) * inv;
+      col[j] = A[(size_t)j * n + k];
+    }
+    __syncthreads();
+    for (int i = ty; i < n; i += 32)
+      for (int j = tx; j < n; j += 32) {
+        const double old = j == k ? 0.0 : A[(size_t)i * n + j];
+        A[(size_t)i * n + j] = i == k ? row[j] : old - col[i] * row[j];
       }
-      inv = 1.0 / p;
-    }
-    __syncthreads();
-    for (int j = threadIdx.x; j < n; j += blockDim.x) {
-      double v = (j == k) ? 1.0 : A[k * n + j];
-      A[k * n + j] = v * inv;
-    }
-    for (int i = threadIdx.x; i < n; i += blockDim.x) F[i] = (i == k) ? 0.0 : A[i * n + k];
-    __syncthreads();
-    for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
-      int i = e / n, j = e % n;
-      if (i == k) continue;
-      double v = (j == k) ? 0.0 : A[i * n + j];
-      A[i * n + j] = v - F[i] * A[k * n + j];
-    }
   }
 }
 
@@ -372,14 +445,25 @@ template void launch_y_to_z<double>(hipStream_t, const double *, const SubDesc *
 template void launch_y_to_z<float>(hipStream_t, const float *, const SubDesc *, int, double *, int,
                                    int);
 void launch_g(hipStream_t st, const SubDesc *subs, int nsub, const int *cptr, const int *cdof,
-              const double *cval, const double *Z, double *G) {
-  if (nsub <= 0) return;
-  hipLaunchKernelGGL(k_g, dim3(nsub), dim3(256), 0, st, subs, cptr, cdof, cval, Z, G);
+              const double *cval, const double *Z, double *G, int maxnc) {
+  if (nsub <= 0 || maxnc <= 0) return;
+  hipLaunchKernelGGL(k_g, dim3(nsub, (maxnc + KG_COLS - 1) / KG_COLS), dim3(256), 0, st, subs, cptr,
+                     cdof, cval, Z, G);
 }
-void launch_ginv(hipStream_t st, const SubDesc *subs, int nsub, double *G, double *work, int *err) {
-  (void)work;
-  if (nsub <= 0) return;
-  hipLaunchKernelGGL(k_ginv, dim3(nsub), dim3(256), 0, st, subs, G, err);
+void launch_ginv(hipStream_t st, const SubDesc *subs, int nsub, double *G, int *err, int maxnc) {
+  if (nsub <= 0 || maxnc <= 0) return;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nsub), dim3(1024), 0, st, subs, G, err);
+  };
+  switch ((maxnc + 31) / 32) {
+    case 1: go(k_ginv<1>); break;
+    case 2: go(k_ginv<2>); break;
+    case 3: go(k_ginv<3>); break;
+    case 4: go(k_ginv<4>); break;
+    case 5: go(k_ginv<5>); break;
+    case 6: go(k_ginv<6>); break;
+    default: go(k_ginv_large);
+  }
 }
 void launch_acs(hipStream_t st, const SubDesc *subs, int nsub, const int *cptr,
                 const double *omega, const double *G, double *Acs) {
