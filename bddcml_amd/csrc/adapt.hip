@@ -88,18 +88,25 @@ __device__ __forceinline__ double *pcol(double *b, const PairDesc &p, bool wide,
 }
 
 // x <- x - sum_c q_c (q_c . x) on columns [c0, c0 + ncol) of every active
-// pair; one thread per projection column (disjoint supports)
-__global__ void k_ad_project(const PairDesc *__restrict__ pairs, const int *__restrict__ qptr,
-                             const int *__restrict__ qpos, const double *__restrict__ qval,
-                             double *buf, int wide, int c0) {
+// pair; 16 lanes per projection column (disjoint supports), their partial
+// sums met in a fixed butterfly.  Latency-bound: one thread per projection
+// column walked rows of 100 and more entries (101 us a launch for 24^3
+// elasticity in 12 boxes, 12.5 us now).
+constexpr int AD_PROJ_THR = 512;
+__global__ __launch_bounds__(AD_PROJ_THR) void k_ad_project(
+    const PairDesc *__restrict__ pairs, const int *__restrict__ qptr, const int *__restrict__ qpos,
+    const double *__restrict__ qval, double *buf, int wide, int c0) {
   const PairDesc p = pairs[blockIdx.x];
-  const int col = blockIdx.y;
+  const int col = blockIdx.y, grp = threadIdx.x >> 4, l = threadIdx.x & 15;
   if (!p.active || col >= p.k) return;
   double *x = pcol(buf, p, wide, c0 + col);
-  for (int c = p.q0 + threadIdx.x; c < p.q1; c += blockDim.x) {
+  for (int c = p.q0 + grp; c < p.q1; c += AD_PROJ_THR / 16) {
+    const int e0 = qptr[c], e1 = qptr[c + 1];
     double t = 0.0;
-    for (int e = qptr[c]; e < qptr[c + 1]; e++) t += qval[e] * x[qpos[e]];
-    for (int e = qptr[c]; e < qptr[c + 1]; e++) x[qpos[e]] -= t * qval[e];
+    for (int e = e0 + l; e < e1; e += 16) t += qval[e] * x[qpos[e]];
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) t += __shfl_xor(t, o, 16);
+    for (int e = e0 + l; e < e1; e += 16) x[qpos[e]] -= t * qval[e];
   }
 }
 
@@ -176,8 +183,12 @@ __global__ __launch_bounds__(256) void k_ad_resid(const PairDesc *__restrict__ p
 //   y_s += Phi_s (R_s u - Z_s^T r_s),   u = K^+ sum_s R_s^T Phi_s^T r_s,
 // since Z_s G_s^{-1} Z_s^T r_s = Phi_s Z_s^T r_s.  R_s maps the constraints
 // of s to the pair's coarse dofs (cmap); K^+ is symmetric.  LDS: the coarse
-// vectors g, u (ncp each) and Phi^T r, Z^T r (nci + ncj each).
-__global__ __launch_bounds__(256) void k_ad_coarse_pc(const PairDesc *__restrict__ pairs,
+// vectors g, u (ncp each) and Phi^T r, Z^T r (nci + ncj each).  One workgroup
+// per pair and column reads Phi and Z of both sides; 16 waves and unrolled
+// loops keep enough of those loads in flight (4 waves: 0.90 ms a launch for
+// 24^3 elasticity in 12 boxes, 0.40 ms now).
+constexpr int AD_PC_THR = 1024;
+__global__ __launch_bounds__(AD_PC_THR) void k_ad_coarse_pc(const PairDesc *__restrict__ pairs,
                                                       const double *__restrict__ Z,
                                                       const double *__restrict__ Phi,
                                                       const int *__restrict__ cmap,
@@ -193,12 +204,13 @@ __global__ __launch_bounds__(256) void k_ad_coarse_pc(const PairDesc *__restrict
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const double *x = in + p.woff + (int64_t)col * p.n;
   // Phi^T r and Z^T r, one wave per constraint
-  for (int e = wv; e < nc2; e += 4) {
+  for (int e = wv; e < nc2; e += AD_PC_THR / 64) {
     const int side = e >= p.nci, c = side ? e - p.nci : e;
     const int NI = side ? NIj : p.NIi;
     const int64_t zo = (side ? p.zoj : p.zoi) + (int64_t)c * NI;
     const double *xs = x + (side ? p.NIi : 0);
     double a = 0.0, b = 0.0;
+#pragma unroll 4
     for (int r = lane; r < NI; r += 64) {
       a += Phi[zo + r] * xs[r];
       b += Z[zo + r] * xs[r];
@@ -209,30 +221,32 @@ __global__ __launch_bounds__(256) void k_ad_coarse_pc(const PairDesc *__restrict
     }
     if (lane == 0) gp[e] = a, zr[e] = b;
   }
-  for (int q = threadIdx.x; q < p.ncp; q += 256) g[q] = 0.0;
+  for (int q = threadIdx.x; q < p.ncp; q += AD_PC_THR) g[q] = 0.0;
   __syncthreads();
   // assemble side by side: within a side the coarse dofs are distinct
   const int *cm = cmap + p.cm0;
-  for (int c = threadIdx.x; c < p.nci; c += 256) g[cm[c]] += gp[c];
+  for (int c = threadIdx.x; c < p.nci; c += AD_PC_THR) g[cm[c]] += gp[c];
   __syncthreads();
-  for (int c = threadIdx.x; c < p.ncj; c += 256) g[cm[p.nci + c]] += gp[p.nci + c];
+  for (int c = threadIdx.x; c < p.ncj; c += AD_PC_THR) g[cm[p.nci + c]] += gp[p.nci + c];
   __syncthreads();
   const double *K = Kp + p.kc0;
-  for (int q = threadIdx.x; q < p.ncp; q += 256) {
+  for (int q = threadIdx.x; q < p.ncp; q += AD_PC_THR) {
     double s = 0.0;
+#pragma unroll 8
     for (int t = 0; t < p.ncp; t++) s += K[(int64_t)t * p.ncp + q] * g[t];
     u[q] = s;
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < nc2; e += 256) gp[e] = u[cm[e]] - zr[e];
+  for (int e = threadIdx.x; e < nc2; e += AD_PC_THR) gp[e] = u[cm[e]] - zr[e];
   __syncthreads();
   double *y = out + p.woff + (int64_t)col * p.n;
-  for (int i = threadIdx.x; i < p.n; i += 256) {
+  for (int i = threadIdx.x; i < p.n; i += AD_PC_THR) {
     const int side = i >= p.NIi, r = side ? i - p.NIi : i;
     const int NI = side ? NIj : p.NIi, nc = side ? p.ncj : p.nci;
     const double *ph = Phi + (side ? p.zoj : p.zoi) + r;
     const double *w = gp + (side ? p.nci : 0);
     double s = 0.0;
+#pragma unroll 8
     for (int c = 0; c < nc; c++) s += ph[(int64_t)c * NI] * w[c];
     y[i] += s;
   }
@@ -243,41 +257,70 @@ struct Blocks {
 };
 
 // Gram matrices GA = V^T (A V), GB = V^T (B V) of the nb blocks of V, each
-// of k columns (row major, order nb k, stride 3 kmax); one workgroup per
-// pair, one wave per entry at a time
+// of k columns (row major, order nb k, stride 3 kmax).  One wave per 4 x 4
+// block of entries on and above the diagonal: 12 column reads for 32 sums
+// (entry by entry in one workgroup per pair: 96 reads and at most 4 waves a
+// pair, 1.72 ms a launch for 24^3 elasticity in 12 boxes;
+// 0.064 ms now).
 __global__ __launch_bounds__(256) void k_ad_gram(const PairDesc *__restrict__ pairs, Blocks b,
                                                  int nb, int kmax, double *__restrict__ GA,
                                                  double *__restrict__ GB) {
   const PairDesc p = pairs[blockIdx.x];
   if (!p.active) return;
-  const int m = nb * p.k, ld = 3 * kmax;
+  const int m = nb * p.k, ld = 3 * kmax, ng = (m + 3) / 4;
+  int task = blockIdx.y * 4 + (threadIdx.x >> 6);
+  if (task >= ng * (ng + 1) / 2) return;
+  int g0 = 0;  // block row; its blocks (g0, g0 .. ng - 1) follow each other
+  while (task >= ng - g0) task -= ng - g0, g0++;
+  const int a0 = 4 * g0, c0 = 4 * (g0 + task);
   double *ga = GA + (int64_t)blockIdx.x * ld * ld, *gb = GB + (int64_t)blockIdx.x * ld * ld;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  for (int e = wave; e < m * m; e += 4) {
-    const int a = e / m, c = e % m;
-    if (c < a) continue;
-    const double *va = pcol(b.v[a / p.k], p, false, a % p.k);
-    const double *ac = pcol(b.av[c / p.k], p, false, c % p.k);
-    const double *bc = pcol(b.bv[c / p.k], p, false, c % p.k);
-    double sa = 0.0, sb = 0.0;
-    for (int i = lane; i < p.n; i += 64) {
-      sa += va[i] * ac[i];
-      sb += va[i] * bc[i];
-    }
-    for (int o = 32; o > 0; o >>= 1) {
-      sa += __shfl_xor(sa, o);
-      sb += __shfl_xor(sb, o);
-    }
-    if (lane == 0) {
-      ga[a * ld + c] = ga[c * ld + a] = sa;
-      gb[a * ld + c] = gb[c * ld + a] = sb;
-    }
+  const int lane = threadIdx.x & 63;
+  const double *va[4], *ac[4], *bc[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {  // columns past the end read a valid one
+    const int a = min(a0 + q, m - 1), c = min(c0 + q, m - 1);
+    va[q] = pcol(b.v[a / p.k], p, false, a % p.k);
+    ac[q] = pcol(b.av[c / p.k], p, false, c % p.k);
+    bc[q] = pcol(b.bv[c / p.k], p, false, c % p.k);
   }
+  double sa[4][4] = {}, sb[4][4] = {};
+#pragma unroll 2
+  for (int i = lane; i < p.n; i += 64) {
+    double x[4], y[4], z[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) x[q] = va[q][i], y[q] = ac[q][i], z[q] = bc[q][i];
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        sa[q][r] += x[q] * y[r];
+        sb[q][r] += x[q] * z[r];
+      }
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      double s = sa[q][r], t = sb[q][r];
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        s += __shfl_xor(s, o);
+        t += __shfl_xor(t, o);
+      }
+      const int a = a0 + q, c = c0 + r;
+      if (lane == 0 && c < m && a <= c) {
+        ga[a * ld + c] = ga[c * ld + a] = s;
+        gb[a * ld + c] = gb[c * ld + a] = t;
+      }
+    }
 }
 
 // X' = V C, P' = V C without the X block (the W and P parts), and the same
 // combinations of A V and B V; C is (nb k) x k per pair, row major with
-// stride kmax; one thread per row
+// stride kmax; one thread per row, which reads each of its values once for
+// all k sums (at most AD_MAXK; one read per sum before: 216 us a launch for
+// 24^3 elasticity in 12 boxes, 82 us now)
+constexpr int AD_MAXK = 16;
 __global__ __launch_bounds__(256) void k_ad_combine(const PairDesc *__restrict__ pairs, Blocks b,
                                                     int nb, int kmax, const double *__restrict__ C,
                                                     Blocks o) {
@@ -299,17 +342,26 @@ __global__ __launch_bounds__(256) void k_ad_combine(const PairDesc *__restrict__
   for (int which = 0; which < 3; which++) {
     double *const *src = which == 0 ? b.v : (which == 1 ? b.av : b.bv);
     double *const *dst = which == 0 ? o.v : (which == 1 ? o.av : o.bv);
-    for (int c = 0; c < p.k; c++) {
-      double sx = 0.0, sp = 0.0;
-      for (int blk = 0; blk < nb; blk++)
-        for (int j = 0; j < p.k; j++) {
-          const double v = pcol(src[blk], p, false, j)[i] * cf[(blk * p.k + j) * kmax + c];
-          sx += v;
-          if (blk > 0) sp += v;
-        }
-      pcol(dst[0], p, false, c)[i] = sx;  // new X (or AX, BX)
-      pcol(dst[2], p, false, c)[i] = sp;  // new P (or AP, BP)
-    }
+    double sx[AD_MAXK] = {}, sp[AD_MAXK] = {};
+    for (int blk = 0; blk < nb; blk++)
+#pragma unroll 2
+      for (int j = 0; j < p.k; j++) {
+        const double x = pcol(src[blk], p, false, j)[i];
+        const double *cr = cf + (blk * p.k + j) * kmax;
+#pragma unroll
+        for (int c = 0; c < AD_MAXK; c++)
+          if (c < p.k) {
+            const double v = x * cr[c];
+            sx[c] += v;
+            if (blk > 0) sp[c] += v;
+          }
+      }
+#pragma unroll
+    for (int c = 0; c < AD_MAXK; c++)
+      if (c < p.k) {
+        pcol(dst[0], p, false, c)[i] = sx[c];  // new X (or AX, BX)
+        pcol(dst[2], p, false, c)[i] = sp[c];  // new P (or AP, BP)
+      }
   }
 }
 
@@ -808,17 +860,17 @@ void adaptive_constraints(Solver &S) {
   auto apply = [&](int b, int ab, int bb) {
     if (np == 0) return;
     hipLaunchKernelGGL(k_ad_copy, pk, dim3(256), 0, st, dpairs.p, blk[b].p, 0, 0, win.p, 1, kmax);
-    hipLaunchKernelGGL(k_ad_project, pk, dim3(64), 0, st, dpairs.p, dqptr.p, dqpos.p, dqval.p,
+    hipLaunchKernelGGL(k_ad_project, pk, dim3(AD_PROJ_THR), 0, st, dpairs.p, dqptr.p, dqpos.p, dqval.p,
                        win.p, 1, kmax);
     hipLaunchKernelGGL(k_ad_jump, pk, dim3(256), 0, st, dpairs.p, dma.p, dmb.p, dmwa.p, dmwb.p,
                        win.p, 1, kmax, win.p, 1, 0, 0);
     launch_symm_cols<double>(st, pool, dsubA.p, dtaskA.p, (int)taskA.size(), dcolA.p, win.p, wout.p);
     hipLaunchKernelGGL(k_ad_jump, pk, dim3(256), 0, st, dpairs.p, dma.p, dmb.p, dmwa.p, dmwb.p,
                        wout.p, 1, 0, blk[ab].p, 0, 0, 1);
-    hipLaunchKernelGGL(k_ad_project, pk, dim3(64), 0, st, dpairs.p, dqptr.p, dqpos.p, dqval.p,
+    hipLaunchKernelGGL(k_ad_project, pk, dim3(AD_PROJ_THR), 0, st, dpairs.p, dqptr.p, dqpos.p, dqval.p,
                        blk[ab].p, 0, 0);
     hipLaunchKernelGGL(k_ad_copy, pk, dim3(256), 0, st, dpairs.p, wout.p, 1, kmax, blk[bb].p, 0, 0);
-    hipLaunchKernelGGL(k_ad_project, pk, dim3(64), 0, st, dpairs.p, dqptr.p, dqpos.p, dqval.p,
+    hipLaunchKernelGGL(k_ad_project, pk, dim3(AD_PROJ_THR), 0, st, dpairs.p, dqptr.p, dqpos.p, dqval.p,
                        blk[bb].p, 0, 0);
   };
   // preconditioner: W = P T W on the k columns of W (W already projected)
@@ -837,14 +889,14 @@ void adaptive_constraints(Solver &S) {
       AD_CHECK(hipStreamSynchronize(st));
       t0 = wall_time();
     }
-    hipLaunchKernelGGL(k_ad_coarse_pc, pk, dim3(256), pc_lds, st, dpairs.p, pcs.Z, pcs.Phi, dcmap.p,
+    hipLaunchKernelGGL(k_ad_coarse_pc, pk, dim3(AD_PC_THR), pc_lds, st, dpairs.p, pcs.Z, pcs.Phi, dcmap.p,
                        dkp.p, win.p, wout.p);
     if (S.verbose >= 3) {
       AD_CHECK(hipStreamSynchronize(st));
       t_pc_coarse += wall_time() - t0;
     }
     hipLaunchKernelGGL(k_ad_copy, pk, dim3(256), 0, st, dpairs.p, wout.p, 1, 0, blk[W].p, 0, 0);
-    hipLaunchKernelGGL(k_ad_project, pk, dim3(64), 0, st, dpairs.p, dqptr.p, dqpos.p, dqval.p,
+    hipLaunchKernelGGL(k_ad_project, pk, dim3(AD_PROJ_THR), 0, st, dpairs.p, dqptr.p, dqpos.p, dqval.p,
                        blk[W].p, 0, 0);
   };
   std::vector<double> hGA((size_t)np * ld * ld), hGB((size_t)np * ld * ld), hC((size_t)np * ld * kmax, 0.0),
@@ -854,8 +906,9 @@ void adaptive_constraints(Solver &S) {
   double t_rr = 0.0;  // host part of the Rayleigh-Ritz steps
   auto rr_update = [&](int nb) {
     Blocks in{{blk[X].p, blk[W].p, blk[P].p}, {blk[AX].p, blk[AW].p, blk[AP].p}, {blk[BX].p, blk[BW].p, blk[BP].p}};
-    hipLaunchKernelGGL(k_ad_gram, dim3(std::max(np, 1)), dim3(256), 0, st, dpairs.p, in, nb, kmax,
-                       dGA.p, dGB.p);
+    const int ng = (nb * kmax + 3) / 4;
+    hipLaunchKernelGGL(k_ad_gram, dim3(std::max(np, 1), (ng * (ng + 1) / 2 + 3) / 4), dim3(256), 0, st,
+                       dpairs.p, in, nb, kmax, dGA.p, dGB.p);
     AD_CHECK(hipMemcpyAsync(hGA.data(), dGA.p, hGA.size() * 8, hipMemcpyDeviceToHost, st));
     AD_CHECK(hipMemcpyAsync(hGB.data(), dGB.p, hGB.size() * 8, hipMemcpyDeviceToHost, st));
     AD_CHECK(hipStreamSynchronize(st));
@@ -894,7 +947,7 @@ void adaptive_constraints(Solver &S) {
         }
     }
     AD_CHECK(hipMemcpyAsync(blk[X].p, x0.data(), x0.size() * 8, hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL(k_ad_project, pk, dim3(64), 0, st, dpairs.p, dqptr.p, dqpos.p, dqval.p,
+    hipLaunchKernelGGL(k_ad_project, pk, dim3(AD_PROJ_THR), 0, st, dpairs.p, dqptr.p, dqpos.p, dqval.p,
                        blk[X].p, 0, 0);
     apply(X, AX, BX);
     rr_update(1);
@@ -936,7 +989,7 @@ void adaptive_constraints(Solver &S) {
       if (nactive == 0) break;
       AD_CHECK(hipMemcpyAsync(dpairs.p, pd.data(), pd.size() * sizeof(PairDesc), hipMemcpyHostToDevice, st));
       // W = P T P R (the residual kernel wrote R)
-      hipLaunchKernelGGL(k_ad_project, pk, dim3(64), 0, st, dpairs.p, dqptr.p, dqpos.p, dqval.p,
+      hipLaunchKernelGGL(k_ad_project, pk, dim3(AD_PROJ_THR), 0, st, dpairs.p, dqptr.p, dqpos.p, dqval.p,
                          blk[W].p, 0, 0);
       timed(1, [&] { precondition(); });
       timed(2, [&] { apply(W, AW, BW); });

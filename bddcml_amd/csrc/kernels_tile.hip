@@ -666,15 +666,10 @@ void launch_scatter_ones(hipStream_t st, double *pool, const int64_t *idx, int64
 // One workgroup per (subdomain, tile row I, 64 columns): out_I = sum_J M_IJ
 // in_J on the f64 matrix cores, the M tile and the 64 x 64 input block
 // staged in LDS (the upper tiles as transposes of the stored lower ones).
-template <typename TP>
-__device__ __forceinline__ void tile_to_lds_f64(const TP *__restrict__ t, double *lds, bool trans) {
-  for (int e = threadIdx.x; e < TILE_ELEMS; e += NTHR) {
-    const int row = e & 63, col = e >> 6;
-    const double x = (double)t[e];
-    if (!trans) lds[col * LDL + row] = x;
-    else lds[row * LDL + col] = x;
-  }
-}
+// The next tile and input block are loaded into registers while the matrix
+// cores work on the current ones (loaded between the barriers, a step of the
+// 25 to 32 took 15 us: 458 us a launch for 12 subdomains; 200 us
+// now).
 template <typename TP>
 __global__ __launch_bounds__(NTHR) void k_symm_cols(const TP *__restrict__ pool,
                                                     const SymmSub *__restrict__ subs,
@@ -687,33 +682,48 @@ __global__ __launch_bounds__(NTHR) void k_symm_cols(const TP *__restrict__ pool,
   __shared__ int64_t cl[64];
   const SymmTask t = tasks[blockIdx.x];
   const SymmSub d = subs[t.sub];
+  const int r = threadIdx.x & 63, c0 = threadIdx.x >> 6;  // entries (r, c0 + 4 i)
   if (threadIdx.x < 64) cl[threadIdx.x] = cols[d.col0 + t.c0 + threadIdx.x];
+  __syncthreads();
   typename Mfma<double>::v4 acc[2][2];
   zero_acc<double>(acc);
-  for (int J = 0; J < d.nt; J++) {
-    const bool low = J <= t.I;
-    const int I0 = low ? t.I : J, J0 = low ? J : t.I;
+  constexpr int NE = TILE_ELEMS / NTHR;
+  TP m[NE];
+  double x[NE];
+  auto load = [&](int J) {
+    const int I0 = max(t.I, J), J0 = min(t.I, J);
     const TP *T = pool + (size_t)(d.tile0 + J0 * d.nt - J0 * (J0 - 1) / 2 + (I0 - J0)) * TILE_ELEMS;
+#pragma unroll
+    for (int i = 0; i < NE; i++) m[i] = T[threadIdx.x + NTHR * i];
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+      const int64_t o = cl[c0 + 4 * i];
+      x[i] = o >= 0 ? in[o + J * 64 + r] : 0.0;
+    }
+  };
+  load(0);
+  for (int J = 0; J < d.nt; J++) {
     __syncthreads();
     // As[q][r] = M(I, J)(r, q): the stored tile itself (I >= J) or the
-    // transpose of tile (J, I)
-    tile_to_lds_f64(T, As, !low);
-    // Bs[q][c] = in(J*64 + q, column c)
-    for (int e = threadIdx.x; e < TILE_ELEMS; e += NTHR) {
-      const int q = e & 63, c = e >> 6;
-      const int64_t o = cl[c];
-      Bs[q * LDL + c] = o >= 0 ? in[o + J * 64 + q] : 0.0;
+    // transpose of tile (J, I); Bs[q][c] = in(J*64 + q, column c)
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+      const int c = c0 + 4 * i;
+      if (J <= t.I) As[c * LDL + r] = (double)m[i];
+      else As[r * LDL + c] = (double)m[i];
+      Bs[r * LDL + c] = x[i];
     }
     __syncthreads();
+    if (J + 1 < d.nt) load(J + 1);
     mfma_accumulate<double>(As, Bs, acc);
   }
   __syncthreads();
   acc_to_lds<double>(acc, As);  // As[c*LDL + r] = out(I*64 + r, column c)
   __syncthreads();
   for (int e = threadIdx.x; e < TILE_ELEMS; e += NTHR) {
-    const int r = e & 63, c = e >> 6;
+    const int q = e & 63, c = e >> 6;
     const int64_t o = cl[c];
-    if (o >= 0) out[o + t.I * 64 + r] = As[c * LDL + r];
+    if (o >= 0) out[o + t.I * 64 + q] = As[c * LDL + q];
   }
 }
 template <typename TP>
