@@ -41,6 +41,14 @@ static Sub &local_sub(Solver &S, int isub, const char *routine) {
   return S.subs[is];
 }
 
+[[noreturn]] static void bad_triplet(int i, int j, int matrixtype) {
+  const char *R = "LEVELS_UPLOAD_SUBDOMAIN_DATA";
+  if (matrixtype != 0 && i > j)
+    fatal(R, "Matrix in wrong format - only upper triangle is expected for symmetric problems, matrixtype = " +
+                 std::to_string(matrixtype));
+  fatal(R, "matrix index out of range");
+}
+
 // Assembled triplets of one subdomain (s.ai, s.aj, s.av: sorted by row and
 // column, duplicates summed in input order; src/module_sm.f90:630-685) from
 // la input triplets with indices from b.  Returns whether a fixed dof may
@@ -54,7 +62,6 @@ static Sub &local_sub(Solver &S, int isub, const char *routine) {
 // waking another thread.
 static bool assemble_triplets(Sub &s, int la, const int *is, const int *js, const double *as, int b,
                               int matrixtype) {
-  const char *R = "LEVELS_UPLOAD_SUBDOMAIN_DATA";
   const int nd = s.ndofs;
   const bool full = matrixtype == 0;
   const int nt = std::max(1, std::min({omp_get_max_threads(), la / 8192, 64}));
@@ -169,12 +176,7 @@ static bool assemble_triplets(Sub &s, int la, const int *is, const int *js, cons
         }
     }
   }
-  if (bad < la) {
-    if (!full && is[bad] > js[bad])
-      fatal(R, "Matrix in wrong format - only upper triangle is expected for symmetric problems, matrixtype = " +
-                   std::to_string(matrixtype));
-    fatal(R, "matrix index out of range");
-  }
+  if (bad < la) bad_triplet(is[bad], js[bad], matrixtype);
   return full || std::any_of(nodiag.begin(), nodiag.end(), [](int v) { return v != 0; });
 }
 
@@ -318,6 +320,16 @@ void bddcml_upload_subdomain_data_c(
   if (s.kdof[*nnods] != *ndofs) fatal(R, "sum of NNDF differs from NDOFS");
   const int nd = *ndofs;
   const bool full = *matrixtype == 0;
+  // the triplets of a large subdomain are assembled on the device, in the
+  // background of the next uploads; below that one or two host threads take
+  // less time (16,384 triplets: 0.06 ms) than the launches and the read-back
+  if (!S.plan_only && !full && *la >= 16384) {
+    s.on_host = false;
+    const int bad = device_assemble_entries(S, s.isub, *la, i_sparse, j_sparse, a_sparse, b);
+    if (bad < *la) bad_triplet(i_sparse[bad], j_sparse[bad], *matrixtype);
+    s.uploaded = true;
+    return;
+  }
   const bool no_diag = assemble_triplets(s, *la, i_sparse, j_sparse, a_sparse, b, *matrixtype);
   if (full) {
     // both triangles assembled: every (i, j) needs its mirror (j, i) with the
@@ -369,6 +381,7 @@ void bddcml_upload_subdomain_data_c(
       s.ai.swap(ai), s.aj.swap(aj), s.av.swap(av);
     }
   }
+  s.nnz = (int)s.ai.size();
   // the assembled values go to HBM now; setup permutes and eliminates them there
   if (!S.plan_only) device_upload_entries(S, s.isub);
   s.uploaded = true;
@@ -416,6 +429,10 @@ void bddcml_setup_preconditioner_c(int *matrixtype, int *use_defaults_int,
   };
   // what the interior factorization needs: the interior / interface split
   // and the orderings; globs and constraints follow while the device factors
+  if (!S.plan_only) {
+    device_finish_uploads(S);
+    phase("uploads finished");
+  }
   build_topology(S);
   phase("topology");
   build_orderings(S);

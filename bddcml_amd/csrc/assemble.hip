@@ -1,0 +1,233 @@
+// assemble.hip -- triplet assembly of uploaded subdomain matrices on the
+// device (src/module_sm.f90:630-685): entries sorted by row and column,
+// duplicates summed in input order, so that the result has the bits of the
+// host assembly.  Batched over the subdomains of a flush (blockIdx.y).
+//
+// A counting sort places (column, input index) keys row by row -- in any
+// order within a row, by integer atomics -- and a rank sort orders each row's
+// few keys (they are distinct, so the ranks do not depend on that order).
+// One wave per row: rows are 30 to 200 entries long.  Eight subdomains of
+// 147,456 triplets take 0.33 ms (latency-bound: scattered 8-byte accesses and
+// integer atomics), while the host copies the next ones: an upload takes 0.15
+// ms of host time where its assembly by 16 host threads took 0.30 ms.
+#include "kernels.hpp"
+
+namespace bddc {
+
+constexpr int ASM_THR = 256;    // 4 waves
+constexpr int ASM_LDS = 512;    // keys of a row staged in LDS (longer rows: global memory)
+
+__global__ void k_asm_zero(const AsmSub *__restrict__ subs) {
+  const AsmSub d = subs[blockIdx.y];
+  for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < d.nd; r += gridDim.x * blockDim.x) d.cur[r] = 0;
+}
+
+__global__ void k_asm_count(const AsmSub *__restrict__ subs) {
+  const AsmSub d = subs[blockIdx.y];
+  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < d.n; k += gridDim.x * blockDim.x)
+    atomicAdd(&d.cur[d.i[k] - d.b], 1);
+}
+
+// ptr = exclusive sums of cur over the nd rows (ptr[nd] the total), one
+// workgroup of 1024 threads per subdomain; which 0: ptr = rowp and cur is
+// set to it (the next free place of each row); 1: ptr = uptr, the total is
+// info->nnz; 2: ptr = bptr, the total is info->nbc
+__global__ __launch_bounds__(1024) void k_asm_scan(const AsmSub *__restrict__ subs, int which) {
+  __shared__ int wsum[16];
+  __shared__ int carry;
+  const AsmSub d = subs[blockIdx.x];
+  int *ptr = which == 0 ? d.rowp : which == 1 ? d.uptr : d.bptr;
+  if (!ptr) return;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (threadIdx.x == 0) carry = 0;
+  for (int r0 = 0; r0 < d.nd; r0 += 1024) {
+    const int r = r0 + threadIdx.x;
+    const int v = r < d.nd ? d.cur[r] : 0;
+    int s = v;  // inclusive sum over the wave
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_up(s, o);
+      if (lane >= o) s += t;
+    }
+    if (lane == 63) wsum[w] = s;
+    __syncthreads();
+    int base = carry;
+    for (int q = 0; q < w; q++) base += wsum[q];
+    if (r < d.nd) {
+      ptr[r] = base + s - v;
+      if (which == 0) d.cur[r] = base + s - v;
+    }
+    __syncthreads();
+    if (threadIdx.x == 1023) carry = base + s;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    ptr[d.nd] = carry;
+    if (which == 1) d.info->nnz = carry, d.info->hash = 0;
+    if (which == 2) d.info->nbc = carry;
+  }
+}
+
+__global__ void k_asm_place(const AsmSub *__restrict__ subs) {
+  const AsmSub d = subs[blockIdx.y];
+  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < d.n; k += gridDim.x * blockDim.x) {
+    const int p = atomicAdd(&d.cur[d.i[k] - d.b], 1);
+    d.key[p] = (uint64_t)(uint32_t)(d.j[k] - d.b) << 32 | (uint32_t)k;
+  }
+}
+
+// every row's keys ordered by rank into key2; cur[row] = its distinct columns
+__global__ __launch_bounds__(ASM_THR) void k_asm_sort(const AsmSub *__restrict__ subs) {
+  __shared__ uint64_t sh[ASM_THR / 64][ASM_LDS];
+  const AsmSub d = subs[blockIdx.y];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int step = gridDim.x * (ASM_THR / 64);
+  // every wave of the workgroup takes the same number of rounds (barriers)
+  for (int r0 = blockIdx.x * (ASM_THR / 64); r0 < d.nd; r0 += step) {
+    const int r = r0 + w;
+    const int p0 = r < d.nd ? d.rowp[r] : 0, len = r < d.nd ? d.rowp[r + 1] - p0 : 0;
+    const uint64_t *K = d.key + p0;
+    const bool staged = len <= ASM_LDS;
+    __syncthreads();
+    if (staged)
+      for (int q = lane; q < len; q += 64) sh[w][q] = K[q];
+    __syncthreads();
+    int heads = 0;
+    for (int q0 = 0; q0 < len; q0 += 64) {
+      const int q = q0 + lane;
+      const bool live = q < len;
+      const uint64_t own = live ? (staged ? sh[w][q] : K[q]) : ~0ull;
+      int rank = 0;
+      bool first = true;  // no smaller key of the same column
+      if (staged) {
+        for (int t = 0; t < len; t++) {
+          const uint64_t k = sh[w][t];
+          const bool less = k < own;
+          rank += less;
+          first = first && !(less && (k >> 32) == (own >> 32));
+        }
+      } else {
+        for (int t = 0; t < len; t++) {
+          const uint64_t k = K[t];
+          const bool less = k < own;
+          rank += less;
+          first = first && !(less && (k >> 32) == (own >> 32));
+        }
+      }
+      if (live) d.key2[p0 + rank] = own;
+      heads += __popcll(__ballot(live && first));
+    }
+    if (r < d.nd && lane == 0) d.cur[r] = heads;
+  }
+}
+
+__device__ __forceinline__ uint64_t mix64(uint64_t z) {
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  return z ^ (z >> 31);
+}
+
+// the assembled entries: one wave per row, the first lane of each column
+// sums its duplicates in input order; info->hash = sum of a hash of every
+// (row, column), whatever the order of the rows
+__global__ __launch_bounds__(ASM_THR) void k_asm_sum(const AsmSub *__restrict__ subs) {
+  const AsmSub d = subs[blockIdx.y];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  uint64_t h = 0;
+  for (int r = blockIdx.x * (ASM_THR / 64) + w; r < d.nd; r += gridDim.x * (ASM_THR / 64)) {
+    const int p0 = d.rowp[r], p1 = d.rowp[r + 1];
+    int o = d.uptr[r];
+    for (int q0 = p0; q0 < p1; q0 += 64) {
+      const int q = q0 + lane;
+      const bool live = q < p1;
+      const uint64_t k = live ? d.key2[q] : 0;
+      const uint32_t j = (uint32_t)(k >> 32);
+      const bool head = live && (q == p0 || (uint32_t)(d.key2[q - 1] >> 32) != j);
+      const unsigned long long m = __ballot(head);
+      if (head) {
+        double s = d.a[(uint32_t)k];
+        for (int t = q + 1; t < p1; t++) {
+          const uint64_t kt = d.key2[t];
+          if ((uint32_t)(kt >> 32) != j) break;
+          s += d.a[(uint32_t)kt];
+        }
+        const int e = o + __popcll(m & ((1ull << lane) - 1));
+        d.ai[e] = r;
+        d.aj[e] = (int)j;
+        d.av[e] = s;
+        h += mix64((uint64_t)(uint32_t)r << 32 | j);
+      }
+      o += __popcll(m);
+    }
+  }
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1) h += __shfl_xor((unsigned long long)h, s);
+  if (lane == 0 && h) atomicAdd((unsigned long long *)&d.info->hash, (unsigned long long)h);
+}
+
+// what the host keeps of the assembled matrix: the diagonal (diag, 0 where a
+// row has none: it leads its row in the upper triangle) and, where the
+// subdomain has fixed dofs, the entries that touch one, in order
+__global__ __launch_bounds__(ASM_THR) void k_asm_diag(const AsmSub *__restrict__ subs) {
+  const AsmSub d = subs[blockIdx.y];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  for (int r = blockIdx.x * (ASM_THR / 64) + w; r < d.nd; r += gridDim.x * (ASM_THR / 64)) {
+    const int p0 = d.uptr[r], p1 = d.uptr[r + 1];
+    if (lane == 0) d.diag[r] = p0 < p1 && d.aj[p0] == r ? d.av[p0] : 0.0;
+    if (!d.bptr) continue;
+    const bool fr = d.fix[r] != 0;
+    int n = 0;
+    for (int q = p0 + lane; q < p1; q += 64) n += fr || d.fix[d.aj[q]] != 0;
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) n += __shfl_xor(n, s);
+    if (lane == 0) d.cur[r] = n;
+  }
+}
+__global__ __launch_bounds__(ASM_THR) void k_asm_fixed(const AsmSub *__restrict__ subs) {
+  const AsmSub d = subs[blockIdx.y];
+  if (!d.bptr) return;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  for (int r = blockIdx.x * (ASM_THR / 64) + w; r < d.nd; r += gridDim.x * (ASM_THR / 64)) {
+    const int p0 = d.uptr[r], p1 = d.uptr[r + 1];
+    const bool fr = d.fix[r] != 0;
+    int o = d.bptr[r];
+    for (int q0 = p0; q0 < p1; q0 += 64) {
+      const int q = q0 + lane;
+      const bool in = q < p1 && (fr || d.fix[d.aj[q]] != 0);
+      const unsigned long long m = __ballot(in);
+      if (in) {
+        const int e = o + __popcll(m & ((1ull << lane) - 1));
+        d.bi[e] = r;
+        d.bj[e] = d.aj[q];
+        d.ba[e] = d.av[q];
+      }
+      o += __popcll(m);
+    }
+  }
+}
+
+void launch_assemble_triplets(hipStream_t st, const AsmSub *subs, int nsub, int maxn, int maxnd) {
+  if (nsub <= 0) return;
+  const unsigned gn = (unsigned)std::min((maxn + 1023) / 1024, 256);
+  const unsigned gr = (unsigned)std::min((maxnd + 15) / 16, 1024);  // 4 rows a wave or more
+  hipLaunchKernelGGL(k_asm_zero, dim3((maxnd + 255) / 256, nsub), dim3(256), 0, st, subs);
+  hipLaunchKernelGGL(k_asm_count, dim3(gn, nsub), dim3(256), 0, st, subs);
+  hipLaunchKernelGGL(k_asm_scan, dim3(nsub), dim3(1024), 0, st, subs, 0);
+  hipLaunchKernelGGL(k_asm_place, dim3(gn, nsub), dim3(256), 0, st, subs);
+  hipLaunchKernelGGL(k_asm_sort, dim3(gr, nsub), dim3(ASM_THR), 0, st, subs);
+  hipLaunchKernelGGL(k_asm_scan, dim3(nsub), dim3(1024), 0, st, subs, 1);
+  hipLaunchKernelGGL(k_asm_sum, dim3(gr, nsub), dim3(ASM_THR), 0, st, subs);
+}
+void launch_assembled_diag(hipStream_t st, const AsmSub *subs, int nsub, int maxnd) {
+  if (nsub <= 0) return;
+  const unsigned gr = (unsigned)std::min((maxnd + 15) / 16, 1024);
+  hipLaunchKernelGGL(k_asm_diag, dim3(gr, nsub), dim3(ASM_THR), 0, st, subs);
+  hipLaunchKernelGGL(k_asm_scan, dim3(nsub), dim3(1024), 0, st, subs, 2);
+}
+void launch_assembled_fixed(hipStream_t st, const AsmSub *subs, int nsub, int maxnd) {
+  if (nsub <= 0) return;
+  const unsigned gr = (unsigned)std::min((maxnd + 15) / 16, 1024);
+  hipLaunchKernelGGL(k_asm_fixed, dim3(gr, nsub), dim3(ASM_THR), 0, st, subs);
+}
+
+}  // namespace bddc

@@ -433,6 +433,15 @@ struct DeviceInput {
   std::vector<View<double>> av;
   std::vector<DBuf<char>> chunks;
   size_t used = 0;  // bytes taken of the last chunk
+  // assemblies on the device: queued ones, their work space, row starts and
+  // Dirichlet flags of the assembled matrices
+  std::vector<AsmSub> pending;
+  DBuf<char> work;
+  size_t work_used = 0;
+  DBuf<AsmInfo> info;
+  std::vector<View<int>> uptr;
+  std::vector<View<char>> fix;
+  bool fetched = true;
   DBuf<char> cmp;   // pointer tables and flags of the pattern comparison
   template <class T> void carve(View<T> &v, size_t n) {
     const size_t bytes = (std::max<size_t>(n, 1) * sizeof(T) + 255) / 256 * 256;
@@ -464,10 +473,10 @@ bool device_same_patterns(Solver &S, const std::vector<int> &cand, std::vector<c
   std::vector<int> c2(cand);
   for (int i = 0; i < n; i++) {
     const Sub &s = S.subs[i];
-    if (I.ai[i].n != s.ai.size() || I.aj[i].n != s.aj.size() || s.ai.size() != s.aj.size()) return false;
+    if (I.ai[i].n != (size_t)s.nnz || I.aj[i].n != (size_t)s.nnz) return false;
     pa[i] = (uint64_t)(uintptr_t)I.ai[i].p;
     pb[i] = (uint64_t)(uintptr_t)I.aj[i].p;
-    cnt[i] = (int64_t)s.ai.size();
+    cnt[i] = (int64_t)s.nnz;
   }
   eq.assign(n, 1);
   for (int i = 0; i < n; i++)
@@ -498,24 +507,20 @@ bool device_same_patterns(Solver &S, const std::vector<int> &cand, std::vector<c
 Solver::Solver() = default;
 Solver::~Solver() = default;
 
-void device_upload_entries(Solver &S, int is) {
+static DeviceInput &device_input(Solver &S) {
   if (!S.din) {
     S.din.reset(new DeviceInput());
     S.din->ai.resize(S.nsub);
     S.din->aj.resize(S.nsub);
     S.din->av.resize(S.nsub);
   }
-  const Sub &s = S.subs[is];
-  DeviceInput &I = *S.din;
-  const size_t n = s.ai.size();
-  I.carve(I.ai[is], n);
-  I.carve(I.aj[is], n);
-  I.carve(I.av[is], n);
-  if (!n) return;
-  // the three arrays in the pinned staging area of the uploads, which starts
-  // over (waiting for the copies in flight) when it is full and grows to
-  // several subdomains, 32 MB at most beyond the largest one
-  const size_t bi = n * sizeof(int), bytes = 2 * bi + n * sizeof(double);
+  return *S.din;
+}
+
+// `bytes` of the pinned staging area of the uploads (offset returned), which
+// starts over (waiting for the copies in flight) when it is full and grows to
+// several subdomains, 32 MB at most beyond the largest one
+static char *upload_room(size_t bytes) {
   Staging &h = upload_staging();
   size_t o = (h.used + 255) / 256 * 256;
   if (o + bytes > h.cap) {
@@ -525,13 +530,243 @@ void device_upload_entries(Solver &S, int is) {
       h.grow(std::max<size_t>(bytes, std::min<size_t>(4 * bytes, (size_t)32 << 20)));
   }
   h.used = o + bytes;
+  return h.p + o;
+}
+
+void device_upload_entries(Solver &S, int is) {
+  const Sub &s = S.subs[is];
+  DeviceInput &I = device_input(S);
+  const size_t n = s.ai.size();
+  I.carve(I.ai[is], n);
+  I.carve(I.aj[is], n);
+  I.carve(I.av[is], n);
+  if (!n) return;
+  const size_t bi = n * sizeof(int);
+  char *h = upload_room(2 * bi + n * sizeof(double));
   const size_t ch = (size_t)64 << 10;
-  copy_par(h.p + o, reinterpret_cast<const char *>(s.av.data()), n * sizeof(double), ch);
-  copy_par(h.p + o + 8 * n, reinterpret_cast<const char *>(s.ai.data()), bi, ch);
-  copy_par(h.p + o + 12 * n, reinterpret_cast<const char *>(s.aj.data()), bi, ch);
-  HIPCHECK(hipMemcpyAsync(I.av[is].p, h.p + o, 8 * n, hipMemcpyHostToDevice, nullptr));
-  HIPCHECK(hipMemcpyAsync(I.ai[is].p, h.p + o + 8 * n, bi, hipMemcpyHostToDevice, nullptr));
-  HIPCHECK(hipMemcpyAsync(I.aj[is].p, h.p + o + 12 * n, bi, hipMemcpyHostToDevice, nullptr));
+  copy_par(h, reinterpret_cast<const char *>(s.av.data()), n * sizeof(double), ch);
+  copy_par(h + 8 * n, reinterpret_cast<const char *>(s.ai.data()), bi, ch);
+  copy_par(h + 12 * n, reinterpret_cast<const char *>(s.aj.data()), bi, ch);
+  HIPCHECK(hipMemcpyAsync(I.av[is].p, h, 8 * n, hipMemcpyHostToDevice, nullptr));
+  HIPCHECK(hipMemcpyAsync(I.ai[is].p, h + 8 * n, bi, hipMemcpyHostToDevice, nullptr));
+  HIPCHECK(hipMemcpyAsync(I.aj[is].p, h + 12 * n, bi, hipMemcpyHostToDevice, nullptr));
+}
+
+// launches the assemblies queued so far
+static void flush_assemblies(DeviceInput &I) {
+  if (I.pending.empty()) return;
+  int maxn = 0, maxnd = 0;
+  for (const AsmSub &a : I.pending) maxn = std::max(maxn, a.n), maxnd = std::max(maxnd, a.nd);
+  const size_t bytes = I.pending.size() * sizeof(AsmSub);
+  char *h = upload_room(bytes);
+  std::memcpy(h, I.pending.data(), bytes);
+  View<char> v;
+  I.carve(v, bytes);
+  HIPCHECK(hipMemcpyAsync(v.p, h, bytes, hipMemcpyHostToDevice, nullptr));
+  launch_assemble_triplets(nullptr, reinterpret_cast<const AsmSub *>(v.p), (int)I.pending.size(), maxn,
+                           maxnd);
+  HIPCHECK(hipGetLastError());
+  I.pending.clear();
+  I.work_used = 0;  // reused in stream order
+}
+
+// Unassembled triplets into pinned memory (by all threads, which check them
+// on the way), to the device and into the queue of assemblies; a flush takes
+// as many subdomains as fit the work space.
+int device_assemble_entries(Solver &S, int is, int la, const int *ii, const int *jj, const double *aa,
+                            int b) {
+  DeviceInput &I = device_input(S);
+  Sub &s = S.subs[is];
+  const int nd = s.ndofs;
+  // a fixed dof without a diagonal entry gets an explicit zero one (appended)
+  const size_t cap = (size_t)la + (s.has_fix ? nd : 0);
+  const size_t oi = 8 * cap, oj = oi + 4 * cap, ofx = oj + 4 * cap, raw = (ofx + nd + 255) / 256 * 256;
+  // work space: the input and the keys and counts of its assembly (before the
+  // staging area is taken: a flush stages its descriptors there)
+  const size_t keys = (cap * 8 + 255) / 256 * 256, rows = ((size_t)(nd + 1) * 4 + 255) / 256 * 256;
+  const size_t need = raw + 2 * keys + 2 * rows;
+  if (I.work_used + need > I.work.n) {
+    flush_assemblies(I);
+    if (need > I.work.n) I.work.alloc(std::min(std::max<size_t>(need, (size_t)96 << 20), 8 * need));
+  }
+  char *h = upload_room(raw);
+  double *ha = reinterpret_cast<double *>(h);
+  int *hi = reinterpret_cast<int *>(h + oi), *hj = reinterpret_cast<int *>(h + oj);
+  char *hf = h + ofx;
+  std::vector<char> diag(s.has_fix ? nd : 0, 0);
+  char *dg = s.has_fix ? diag.data() : nullptr;
+  constexpr int CH = 4096;
+  const int nch = (la + CH - 1) / CH;
+  int bad = la;
+#pragma omp parallel for schedule(static) reduction(min : bad)
+  for (int c = 0; c < nch; c++) {
+    const int k0 = c * CH, k1 = std::min(la, k0 + CH);
+    int wrong = 0;
+    for (int k = k0; k < k1; k++) {
+      const int i = ii[k] - b, j = jj[k] - b;
+      wrong |= (i > j) | (i < 0) | (j >= nd);
+      hi[k] = ii[k];
+      hj[k] = jj[k];
+      ha[k] = aa[k];
+    }
+    if (wrong) {
+      int k = k0;
+      while (ii[k] <= jj[k] && ii[k] >= b && jj[k] - b < nd) k++;
+      bad = std::min(bad, k);
+    } else if (dg) {
+      for (int k = k0; k < k1; k++)
+        if (ii[k] == jj[k]) __atomic_store_n(dg + (ii[k] - b), (char)1, __ATOMIC_RELAXED);
+    }
+  }
+  if (bad < la) return bad;
+  int n = la;
+  for (int d = 0; d < nd; d++) {
+    hf[d] = s.ifix[d] != 0;
+    if (dg && hf[d] && !dg[d]) hi[n] = hj[n] = d + b, ha[n] = 0.0, n++;
+  }
+  char *w = I.work.p + I.work_used;
+  I.work_used += need;
+  HIPCHECK(hipMemcpyAsync(w, h, raw, hipMemcpyHostToDevice, nullptr));
+  if (I.info.n < (size_t)S.nsub) I.info.alloc(S.nsub);
+  if (I.uptr.empty()) I.uptr.resize(S.nsub), I.fix.resize(S.nsub);
+  I.carve(I.ai[is], n);
+  I.carve(I.aj[is], n);
+  I.carve(I.av[is], n);
+  I.carve(I.uptr[is], nd + 1);
+  I.carve(I.fix[is], nd);
+  HIPCHECK(hipMemcpyAsync(I.fix[is].p, h + ofx, nd, hipMemcpyHostToDevice, nullptr));
+  AsmSub t{};
+  t.a = reinterpret_cast<const double *>(w);
+  t.i = reinterpret_cast<const int *>(w + oi);
+  t.j = reinterpret_cast<const int *>(w + oj);
+  t.n = n, t.nd = nd, t.b = b;
+  t.key = reinterpret_cast<uint64_t *>(w + raw);
+  t.key2 = reinterpret_cast<uint64_t *>(w + raw + keys);
+  t.rowp = reinterpret_cast<int *>(w + raw + 2 * keys);
+  t.cur = reinterpret_cast<int *>(w + raw + 2 * keys + rows);
+  t.uptr = I.uptr[is].p, t.ai = I.ai[is].p, t.aj = I.aj[is].p, t.av = I.av[is].p;
+  t.info = I.info.p + is;
+  I.pending.push_back(t);
+  I.fetched = false;
+  return la;
+}
+
+void device_finish_uploads(Solver &S) {
+  if (!S.din || S.din->fetched) return;
+  DeviceInput &I = *S.din;
+  flush_assemblies(I);
+  std::vector<int> subs;
+  int maxnd = 0;
+  size_t rows = 0;
+  for (int is = 0; is < S.nsub; is++)
+    if (!S.subs[is].on_host) {
+      subs.push_back(is);
+      maxnd = std::max(maxnd, S.subs[is].ndofs);
+      rows += S.subs[is].ndofs;
+    }
+  const int n = (int)subs.size();
+  // diagonals, and the couplings of each subdomain with fixed dofs: counted,
+  // then written to one buffer
+  DBuf<double> diag;
+  DBuf<int> cnt, bptr;
+  diag.alloc(rows);
+  cnt.alloc(rows);
+  bptr.alloc(rows + n);
+  std::vector<AsmSub> t(n);
+  std::vector<size_t> ro(n + 1, 0);
+  for (int k = 0; k < n; k++) {
+    const int is = subs[k];
+    const Sub &s = S.subs[is];
+    ro[k + 1] = ro[k] + s.ndofs;
+    AsmSub &a = t[k];
+    a = AsmSub{};
+    a.nd = s.ndofs;
+    a.cur = cnt.p + ro[k];
+    a.uptr = I.uptr[is].p, a.ai = I.ai[is].p, a.aj = I.aj[is].p, a.av = I.av[is].p;
+    a.info = I.info.p + is;
+    a.fix = I.fix[is].p;
+    a.diag = diag.p + ro[k];
+    a.bptr = s.has_fix ? bptr.p + ro[k] + k : nullptr;
+  }
+  DBuf<AsmSub> dt;
+  dt.upload(t, nullptr);
+  launch_assembled_diag(nullptr, dt.p, n, maxnd);
+  HIPCHECK(hipGetLastError());
+  std::vector<AsmInfo> info(S.nsub);
+  HIPCHECK(hipMemcpy(info.data(), I.info.p, S.nsub * sizeof(AsmInfo), hipMemcpyDeviceToHost));
+  std::vector<size_t> bo(n + 1, 0);
+  for (int k = 0; k < n; k++) {
+    Sub &s = S.subs[subs[k]];
+    const AsmInfo &f = info[subs[k]];
+    if (f.nnz < 0 || (size_t)f.nnz > I.ai[subs[k]].n || (s.has_fix && (f.nbc < 0 || f.nbc > f.nnz)))
+      fatal("BDDCML_DEVICE", "invalid triplet assembly");
+    s.nnz = f.nnz;
+    s.pat_hash = f.hash;
+    I.ai[subs[k]].n = I.aj[subs[k]].n = I.av[subs[k]].n = f.nnz;
+    bo[k + 1] = bo[k] + (s.has_fix ? f.nbc : 0);
+  }
+  // one read-back: diagonals, coupling values, rows, columns
+  DBuf<char> bc;
+  const size_t nb = bo[n];
+  bc.alloc(16 * nb);
+  for (int k = 0; k < n; k++) {
+    t[k].ba = reinterpret_cast<double *>(bc.p) + bo[k];
+    t[k].bi = reinterpret_cast<int *>(bc.p + 8 * nb) + bo[k];
+    t[k].bj = reinterpret_cast<int *>(bc.p + 12 * nb) + bo[k];
+  }
+  HIPCHECK(hipMemcpyAsync(dt.p, t.data(), n * sizeof(AsmSub), hipMemcpyHostToDevice, nullptr));
+  launch_assembled_fixed(nullptr, dt.p, n, maxnd);
+  HIPCHECK(hipGetLastError());
+  Staging &h = staging();
+  h.used = 0;
+  h.grow(8 * rows + 16 * nb);
+  HIPCHECK(hipMemcpyAsync(h.p, diag.p, 8 * rows, hipMemcpyDeviceToHost, nullptr));
+  if (nb) HIPCHECK(hipMemcpyAsync(h.p + 8 * rows, bc.p, 16 * nb, hipMemcpyDeviceToHost, nullptr));
+  HIPCHECK(hipStreamSynchronize(nullptr));
+  const double *hd = reinterpret_cast<const double *>(h.p), *hb = hd + rows;
+  const int *hi = reinterpret_cast<const int *>(hb + nb), *hj = hi + nb;
+#pragma omp parallel for schedule(dynamic, 4)
+  for (int k = 0; k < n; k++) {
+    Sub &s = S.subs[subs[k]];
+    s.diag.assign(hd + ro[k], hd + ro[k + 1]);
+    s.bc_a.assign(hb + bo[k], hb + bo[k + 1]);
+    s.bc_i.assign(hi + bo[k], hi + bo[k + 1]);
+    s.bc_j.assign(hj + bo[k], hj + bo[k + 1]);
+  }
+  I.work.release();
+  I.work_used = 0;
+  I.fetched = true;
+}
+
+void device_fetch_patterns(Solver &S, const std::vector<int> &subs) {
+  if (!S.din) return;
+  DeviceInput &I = *S.din;
+  Staging &h = staging();
+  size_t total = 0;
+  for (int is : subs)
+    if (!S.subs[is].on_host && S.subs[is].ai.empty()) total += 8 * (size_t)S.subs[is].nnz;
+  if (!total) return;
+  h.used = 0;
+  h.grow(total);
+  std::vector<std::pair<int, size_t>> got;
+  size_t o = 0;
+  for (int is : subs) {
+    const Sub &s = S.subs[is];
+    if (s.on_host || !s.ai.empty()) continue;
+    const size_t b = 4 * (size_t)s.nnz;
+    HIPCHECK(hipMemcpyAsync(h.p + o, I.ai[is].p, b, hipMemcpyDeviceToHost, nullptr));
+    HIPCHECK(hipMemcpyAsync(h.p + o + b, I.aj[is].p, b, hipMemcpyDeviceToHost, nullptr));
+    got.push_back({is, o});
+    o += 2 * b;
+  }
+  HIPCHECK(hipStreamSynchronize(nullptr));
+#pragma omp parallel for schedule(dynamic)
+  for (int k = 0; k < (int)got.size(); k++) {
+    Sub &s = S.subs[got[k].first];
+    const int *p = reinterpret_cast<const int *>(h.p + got[k].second);
+    s.ai.assign(p, p + s.nnz);
+    s.aj.assign(p + s.nnz, p + 2 * (size_t)s.nnz);
+  }
 }
 
 void device_release_input(Solver &S) { S.din.reset(); }
@@ -579,7 +814,7 @@ static void symbolic(const Sub &s, SubTiles &T) {
   const int nt = s.nto + s.nti, nw = (nt + 63) / 64;
   T.col.assign(nt, std::vector<uint64_t>(nw, 0ull));
   for (int J = 0; J < nt; J++) bs_set(T.col[J], J);
-  for (size_t k = 0; k < s.av.size(); k++) {
+  for (size_t k = 0; k < s.ai.size(); k++) {
     int a = s.perm[s.ai[k]], b = s.perm[s.aj[k]];
     int I = std::max(a, b) / TILE, J = std::min(a, b) / TILE;
     bs_set(T.col[J], I);
@@ -1152,7 +1387,7 @@ void device_setup_begin(Solver &S) {
                           (int)S.din->ai[is].n, (int)foff[is], (int)poff[c], (int)toff[c],
                           (int)doff[c], (int)(doff[c + 1] - doff[c]), T.base};
       D.perm_off[is] = (int)poff[c];
-      if ((int64_t)S.din->ai[is].n != (int64_t)s.ai.size()) bad |= 1;
+      if ((int64_t)S.din->ai[is].n != (int64_t)s.nnz) bad |= 1;
       if (T.base != T.pat.tile.front() || s.ndofs != S.subs[oreps[c]].ndofs) bad |= 4;
       if ((int64_t)T.base + (int64_t)T.pat.tile.size() > D.ntiles) bad |= 4;
       for (int d = 0; d < s.ndofs; d++) fix[foff[is] + d] = s.ifix[d] != 0;
@@ -1416,8 +1651,7 @@ static void build_resid_index(Solver &S) {
   int64_t foff = 0;
   for (int is = 0; is < nsub; is++) {
     const int c = ocls[is];
-    if (S.subs[is].ai.size() != S.subs[oreps[c]].ai.size() ||
-        (int64_t)S.din->av[is].n != (int64_t)S.subs[is].ai.size())
+    if (S.subs[is].nnz != S.subs[oreps[c]].nnz || (int64_t)S.din->av[is].n != (int64_t)S.subs[is].nnz)
       fatal("BDDCML_DEVICE_PLAN", "triplet structure differs within a class");
     if (foff != D.hodesc[is].poff) fatal("BDDCML_DEVICE_PLAN", "local-order offsets");
     rs[is] = ResidSub{S.din->av[is].p, foff, (int64_t)eno[c], (int)rpo[c], (int)foff,
@@ -1436,6 +1670,14 @@ static void build_resid_index(Solver &S) {
 // triplets before that elimination runs on the host
 static double interface_rho(const Sub &s) {
   double rho = 0.0;
+  if (!s.on_host) {
+    for (int i = 0; i < s.ndofs; i++) {
+      if (s.perm[i] < s.NO) continue;
+      const double v = std::fabs(s.diag[i]);
+      rho = std::max(rho, s.ifix[i] && v < 1e-12 ? 1.0 : v);
+    }
+    return rho > 0.0 ? rho : 1.0;
+  }
   std::vector<char> seen(s.has_fix ? s.ndofs : 0, 0);
   for (size_t k = 0; k < s.av.size(); k++) {
     const int i = s.ai[k];
@@ -3345,7 +3587,7 @@ static void refine_solution(Solver &S, int method, double tol, int maxit, int nd
       // triplet values, flags, f, u and r of every dof (the class indices
       // are shared by the subdomains of a class)
       double nnz = 0;
-      for (int is = 0; is < S.nsub; is++) nnz += (double)S.subs[is].ai.size();
+      for (int is = 0; is < S.nsub; is++) nnz += (double)S.subs[is].nnz;
       S.t.resid_bytes = 8.0 * nnz + 25.0 * (double)D.ndofs_total;
     }
     const double rel = std::sqrt(sc[0]) / normres0;

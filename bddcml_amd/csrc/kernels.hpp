@@ -77,6 +77,36 @@ void launch_scatter_sub(hipStream_t st, T *pool, const ScatterSub *subs, int nsu
 // pool[idx[k]] = 1.0
 void launch_scatter_ones(hipStream_t st, double *pool, const int64_t *idx, int64_t n);
 
+// One subdomain of a batched triplet assembly (assemble.hip).  Input: n
+// triplets (i, j, a; indices from b) and nd rows; work: row counts and places
+// (rowp nd + 1, cur nd), keys (n each); result: the assembled entries (room
+// for n) with their row starts uptr (nd + 1) and info.
+struct AsmInfo {
+  int nnz, nbc;  // assembled entries; those touching a fixed dof
+  uint64_t hash;  // of the assembled pattern
+};
+struct AsmSub {
+  const double *a;
+  const int *i, *j;
+  int n, nd, b;
+  int *rowp, *cur;
+  uint64_t *key, *key2;
+  int *uptr, *ai, *aj;
+  double *av;
+  AsmInfo *info;
+  // diagonal and Dirichlet couplings (launch_assembled_diag / _fixed):
+  // Dirichlet flags, row starts of the couplings (null: none wanted), lists
+  const char *fix;
+  double *diag;
+  int *bptr, *bi, *bj;
+  double *ba;
+};
+void launch_assemble_triplets(hipStream_t st, const AsmSub *subs, int nsub, int maxn, int maxnd);
+// diag, and with bptr the number of couplings per row and info->nbc
+void launch_assembled_diag(hipStream_t st, const AsmSub *subs, int nsub, int maxnd);
+// the couplings (bi, bj, ba), sorted by row and column
+void launch_assembled_fixed(hipStream_t st, const AsmSub *subs, int nsub, int maxnd);
+
 // diff[i] = 1 where the triplet pattern (ai, aj: device pointers) of
 // subdomain i differs from that of cand[i] (equal lengths cnt)
 void launch_same_pattern(hipStream_t st, const uint64_t *pai, const uint64_t *paj, const int *cand,

@@ -186,6 +186,7 @@ static bool level2_subdomain(const Solver &S, const std::vector<int> &elems,
     else
       t.ai.push_back(x.i), t.aj.push_back(x.j), t.av.push_back(x.a);
   }
+  t.nnz = (int)t.ai.size();
   t.uploaded = true;
   return true;
 }

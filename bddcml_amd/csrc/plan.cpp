@@ -573,9 +573,8 @@ static void exchange_sum(Solver &S, std::vector<std::vector<double>> &v) {
 // at free dofs, a_ii g_i (diagonal kept, 1 if tiny) at fixed dofs
 static void bc_from_stored(Sub &s) {
   s.bc.assign(s.ndofs, 0.0);
-  for (size_t q = 0; q < s.bc_k.size(); q++) {
-    const size_t k = s.bc_k[q];
-    const int i = s.ai[k], j = s.aj[k];
+  for (size_t q = 0; q < s.bc_a.size(); q++) {
+    const int i = s.bc_i[q], j = s.bc_j[q];
     double a = s.bc_a[q];
     if (i != j) {
       if (s.ifix[i] && !s.ifix[j]) s.bc[j] -= a * s.fixv[i];
@@ -591,7 +590,12 @@ static void bc_from_stored(Sub &s) {
 // couplings to fixed dofs are zeroed after their values are stored
 static void eliminate_bc(Sub &s) {
   s.bc.assign(s.ndofs, 0.0);
-  s.bc_k.clear();
+  if (!s.on_host) {  // the couplings came with the assembly
+    if (s.has_fix) bc_from_stored(s);
+    return;
+  }
+  s.bc_i.clear();
+  s.bc_j.clear();
   s.bc_a.clear();
   if (!s.has_fix) return;
   // every fixed dof needs a diagonal entry
@@ -618,11 +622,13 @@ static void eliminate_bc(Sub &s) {
     s.ai.swap(ai);
     s.aj.swap(aj);
     s.av.swap(av);
+    s.nnz = (int)s.av.size();
   }
   for (size_t k = 0; k < s.av.size(); k++) {
     const int i = s.ai[k], j = s.aj[k];
     if (!s.ifix[i] && !s.ifix[j]) continue;
-    s.bc_k.push_back(k);
+    s.bc_i.push_back(i);
+    s.bc_j.push_back(j);
     s.bc_a.push_back(s.av[k]);
     if (i != j) s.av[k] = 0.0;
     else if (std::fabs(s.av[k]) < 1e-12) s.av[k] = 1.0;
@@ -658,9 +664,8 @@ void build_reactions(Solver &S) {
     Sub &s = S.subs[is];
     s.rea.assign(s.ndofs, 0.0);
     if (!s.has_fix) continue;
-    for (size_t q = 0; q < s.bc_k.size(); q++) {
-      const size_t k = s.bc_k[q];
-      const int i = s.ai[k], j = s.aj[k];
+    for (size_t q = 0; q < s.bc_a.size(); q++) {
+      const int i = s.bc_i[q], j = s.bc_j[q];
       const double a = s.bc_a[q];
       s.rea[i] += a * s.sol[j];
       if (i != j) s.rea[j] += a * s.sol[i];
@@ -712,8 +717,13 @@ bool weight_coefficients(const Solver &S, int is, std::vector<double> &rho) {
   rho.assign(ni, 1.0);
   if (S.weights_type == 1) {
     std::vector<double> dg(s.ndofs, 0.0);
-    for (size_t k = 0; k < s.av.size(); k++)
-      if (s.ai[k] == s.aj[k]) dg[s.ai[k]] += s.av[k];
+    if (s.on_host) {
+      for (size_t k = 0; k < s.av.size(); k++)
+        if (s.ai[k] == s.aj[k]) dg[s.ai[k]] += s.av[k];
+    } else {  // as the Dirichlet elimination leaves it
+      for (int d = 0; d < s.ndofs; d++)
+        dg[d] = s.ifix[d] && std::fabs(s.diag[d]) < 1e-12 ? 1.0 : s.diag[d];
+    }
     for (size_t k = 0; k < ni; k++) {
       rho[k] = dg[s.ifc_dof[k]];
       if (rho[k] == 0.0) rho[k] = 1.0;
@@ -966,7 +976,7 @@ void build_unique_interface(Solver &S) {
 // neighbours by ascending degree).
 static std::vector<int> order_rcm(const Sub &s, const std::vector<int> &loc, int no) {
   std::vector<std::vector<int>> g(no);
-  for (size_t k = 0; k < s.av.size(); k++) {
+  for (size_t k = 0; k < s.ai.size(); k++) {
     int i = loc[s.ai[k]], j = loc[s.aj[k]];
     if (i >= 0 && j >= 0 && i != j) g[i].push_back(j), g[j].push_back(i);
   }
@@ -1108,7 +1118,7 @@ static void order_subdomain(Sub &s, int method, int leaf_dofs, int ndim) {
     // symmetric node adjacency by counting sort (repeated neighbours of
     // multi-dof nodes are harmless to the separator test)
     std::vector<int> ptr(nn + 1, 0);
-    for (size_t k = 0; k < s.av.size(); k++) {
+    for (size_t k = 0; k < s.ai.size(); k++) {
       int a = nloc[dnode[s.ai[k]]], b = nloc[dnode[s.aj[k]]];
       if (a >= 0 && b >= 0 && a != b) ptr[a + 1]++, ptr[b + 1]++;
     }
@@ -1116,7 +1126,7 @@ static void order_subdomain(Sub &s, int method, int leaf_dofs, int ndim) {
     std::vector<int> adj(ptr[nn]);
     {
       std::vector<int> fill(ptr.begin(), ptr.end() - 1);
-      for (size_t k = 0; k < s.av.size(); k++) {
+      for (size_t k = 0; k < s.ai.size(); k++) {
         int a = nloc[dnode[s.ai[k]]], b = nloc[dnode[s.aj[k]]];
         if (a >= 0 && b >= 0 && a != b) adj[fill[a]++] = b, adj[fill[b]++] = a;
       }
@@ -1144,7 +1154,7 @@ static void order_subdomain(Sub &s, int method, int leaf_dofs, int ndim) {
   std::vector<int> iloc(n, -1);
   for (int k = 0; k < ni; k++) iloc[s.ifc_dof[k]] = k;
   std::vector<int> first(ni, NO);
-  for (size_t k = 0; k < s.av.size(); k++) {
+  for (size_t k = 0; k < s.ai.size(); k++) {
     int i = s.ai[k], j = s.aj[k];
     if (loc[i] >= 0 && iloc[j] >= 0) first[iloc[j]] = std::min(first[iloc[j]], ipos[loc[i]]);
     if (loc[j] >= 0 && iloc[i] >= 0) first[iloc[i]] = std::min(first[iloc[i]], ipos[loc[j]]);
@@ -1188,7 +1198,9 @@ void build_orderings(Solver &S) {
         const Sub &s = S.subs[i];
         Fnv f;
         f.add((uint64_t)s.ndofs), f.add((uint64_t)s.nnods), f.sample(s.kdof);
-        f.sample(s.ai), f.sample(s.aj), f.add(s.int_dof), f.add(s.ifc_dof);
+        if (s.on_host) f.sample(s.ai), f.sample(s.aj);
+        else f.add((uint64_t)s.nnz), f.add(s.pat_hash);
+        f.add(s.int_dof), f.add(s.ifc_dof);
         return f.h;
       },
       [&](int a, int b) {
@@ -1196,7 +1208,9 @@ void build_orderings(Solver &S) {
         const bool known = !pat_eq.empty() && cand_of[b] == a;
         return x.ndofs == y.ndofs && x.nnods == y.nnods && x.kdof == y.kdof &&
                x.int_dof == y.int_dof && x.ifc_dof == y.ifc_dof &&
-               (known ? pat_eq[b] != 0 : (x.ai == y.ai && x.aj == y.aj)) && same_shape(x, y, S.ndim);
+               (known ? pat_eq[b] != 0
+                      : (x.on_host && y.on_host && x.ai == y.ai && x.aj == y.aj)) &&
+               same_shape(x, y, S.ndim);
       },
       S.ord_cls, S.ord_reps,
       [&](const std::vector<int> &cand) {
@@ -1204,6 +1218,7 @@ void build_orderings(Solver &S) {
         if (!device_same_patterns(S, cand, pat_eq)) pat_eq.clear();
       });
   phase("classes");
+  if (!S.plan_only) device_fetch_patterns(S, S.ord_reps);
 #pragma omp parallel for schedule(dynamic)
   for (int k = 0; k < (int)S.ord_reps.size(); k++)
     order_subdomain(S.subs[S.ord_reps[k]], S.ordering, S.nd_leaf, S.ndim);

@@ -60,9 +60,17 @@ struct Sub {
   std::vector<double> user_c;
   int nuser_c = 0;
   int find_components = 0, use_dual = 0, neighbouring = 1;
-  // assembled upper triangle (sorted by row, col; duplicates summed)
+  // assembled upper triangle (sorted by row, col; duplicates summed): nnz
+  // entries.  on_host: in ai, aj, av.  Otherwise assembled on the device; the
+  // host has a hash of the pattern, the diagonal (0 where a row has none) and
+  // the Dirichlet couplings (bc_*) from the start of the setup on, and ai, aj
+  // (not av) where the ordering stage asked for them
+  int nnz = 0;
+  bool on_host = true;
   RawInts ai, aj;
   RawVec<double> av;
+  uint64_t pat_hash = 0;
+  RawVec<double> diag;
 
   // ---- topology --------------------------------------------------------
   std::vector<int> kdof;    // first dof of each node (nnods+1)
@@ -98,8 +106,8 @@ struct Sub {
   std::vector<double> bc;   // eliminated Dirichlet values, ndofs
   // triplet entries touching fixed dofs with their values before the
   // elimination, kept to eliminate new Dirichlet values later
-  std::vector<size_t> bc_k;
-  std::vector<double> bc_a;
+  RawInts bc_i, bc_j;
+  RawVec<double> bc_a;
   std::vector<double> rea;  // reactions of the last solve (ndofs)
   std::vector<double> w;    // interface weights (reference order)
   std::vector<double> fmod; // right-hand side used for condensation, ndofs

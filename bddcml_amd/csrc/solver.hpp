@@ -178,6 +178,16 @@ void change_global_data(const int *ifix, int lifix, const double *fixv, int lfix
 
 // device steps (device.hip)
 void device_upload_entries(Solver &S, int is);
+// the same for unassembled triplets (la of them, indices from b, upper
+// triangle), assembled on the device; returns la, or the first entry that is
+// out of range or below the diagonal (then nothing was sent)
+int device_assemble_entries(Solver &S, int is, int la, const int *i, const int *j, const double *a,
+                            int b);
+// start of the setup: the assemblies finished, their counts, pattern hashes,
+// diagonals and Dirichlet couplings on the host
+void device_finish_uploads(Solver &S);
+// ai, aj of device-assembled subdomains to the host
+void device_fetch_patterns(Solver &S, const std::vector<int> &subs);
 void device_release_input(Solver &S);
 // triplet patterns of subdomain i and cand[i] compared in HBM (eq[i] = 1:
 // equal); false when not available (then eq is untouched)

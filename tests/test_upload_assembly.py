@@ -1,6 +1,7 @@
-"""Triplet assembly of bddcml_upload_subdomain_data_c at sizes where one and
-several host threads share it: any input order gives the same matrix, and a
-bad entry is refused with its message wherever it stands."""
+"""Triplet assembly of bddcml_upload_subdomain_data_c, on the host (small
+subdomains, full storage) and on the device (from 16,384 triplets): any input
+order gives the same matrix, and a bad entry is refused with its message
+wherever it stands."""
 import numpy as np
 import pytest
 
@@ -20,8 +21,8 @@ def _shuffled(d, seed, full=False):
                 matrixtype=0 if full else d["matrixtype"])
 
 
-# 2,304 triplets: one thread; 18,432 and 62,208: two and seven shares;
-# elasticity rows of up to 648 triplets (the long-row sort)
+# 2,304 triplets: one host thread; 18,432: device; 62,208 in full storage:
+# several host threads; elasticity: device, rows of up to 192 triplets
 @pytest.mark.gpu
 @pytest.mark.parametrize("nel,kind,full", [(4, "poisson", False), (8, "poisson", False),
                                            (12, "poisson", True), (6, "elasticity", False)])
@@ -42,6 +43,91 @@ def test_input_order_does_not_matter(nel, kind, full):
         assert np.abs(x - y).max() <= 1e-12 * np.abs(x).max()
 
 
+def _matrices(p, change, matrixtype=1):
+    b = bddcml_amd.Bddcml()
+    b.init(2, [p.nsub, 1], numbase=p.numbase)
+    for k, d in enumerate(p.subdomains()):
+        b.upload_subdomain_data(change(d, k))
+    b.setup_preconditioner(matrixtype)
+    it, reason, _ = b.solve(0, 1e-10, 200, 50)
+    assert reason == 0
+    out = [b.sub_matrix(s + p.numbase) for s in range(p.nsub)], b.download_global_solution(p.ndof)
+    b.finalize()
+    return out
+
+
+@pytest.mark.gpu
+def test_long_rows_on_the_device():
+    """Every triplet in 20 parts: rows of up to 1,280 entries, beyond what the
+    device sort stages in LDS (512)."""
+    print("case long rows", flush=True)
+    p = CubeProblem(4, 2, rhs="random", seed=3)  # 46,080 triplets
+
+    def parts(d, k):
+        o = np.random.RandomState(k).permutation(20 * len(d["a_sparse"]))
+        rep = lambda x: np.tile(x, 20)[o].copy()
+        return dict(d, i_sparse=rep(d["i_sparse"]), j_sparse=rep(d["j_sparse"]),
+                    a_sparse=rep(d["a_sparse"] / 20.0))
+
+    (x, u), (y, v) = _matrices(p, lambda d, k: d), _matrices(p, parts)
+    for a, b in zip(x, y):
+        # sums of 160 terms in another order: 160 eps of the entries' sum of moduli
+        assert np.abs(a - b).max() <= 1e-12 * np.abs(a).max()
+    assert np.abs(u - v).max() <= 1e-9 * np.abs(u).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nel", [4, 8, 9])
+def test_fixed_dofs_without_diagonal(nel):
+    """Missing diagonals of fixed dofs become 1, nonzero fixed values move to
+    the right-hand side: device assembly against the host's full storage."""
+    print("case missing diagonals", nel, flush=True)
+    p = CubeProblem(nel, 2, rhs="random", seed=3, dirichlet="random")
+
+    def drop(d, k):
+        b = p.numbase
+        keep = (d["i_sparse"] != d["j_sparse"]) | (d["ifix"][d["i_sparse"] - b] == 0)
+        return dict(d, **{n: d[n][keep].copy() for n in ("i_sparse", "j_sparse", "a_sparse")})
+
+    (x, u) = _matrices(p, drop)
+    (y, v) = _matrices(p, lambda d, k: _shuffled(drop(d, k), k, full=True), matrixtype=0)
+    for a, b in zip(x, y):
+        assert np.abs(a - b).max() <= 1e-12 * np.abs(a).max()
+    assert np.abs(u - v).max() <= 1e-8 * np.abs(u).max()
+    # fixed values come back as given
+    for d in p.subdomains():
+        g = d["isvgvn"][d["ifix"] > 0] - p.numbase
+        assert np.allclose(u[g], d["fixv"][d["ifix"] > 0], rtol=1e-12, atol=0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["poisson", "elasticity"])
+def test_stiffness_weights_and_reactions(kind):
+    """The diagonal and the Dirichlet couplings read back from the device
+    assembly: stiffness weights and reactions against the host's assembly of
+    the same matrix in full storage."""
+    print("case weights, reactions", kind, flush=True)
+    n = 6 if kind == "elasticity" else 9
+    p = CubeProblem(n, 2, kind=kind, rhs="random", seed=3, dirichlet="random",
+                    coef=lambda e: 1.0 + (e % 7))
+    out = []
+    for full in (False, True):
+        b = bddcml_amd.Bddcml()
+        b.init(2, [p.nsub, 1], numbase=p.numbase)
+        for k, d in enumerate(p.subdomains()):
+            b.upload_subdomain_data(_shuffled(d, k, True) if full else d)
+        b.setup_preconditioner(0 if full else 1, weights_type=1)
+        it, reason, _ = b.solve(0, 1e-11, 200, 50)
+        assert reason == 0
+        r = np.random.RandomState(1).rand(b.counts()["nig"])
+        out.append((it, b.apply_pc(r), b.download_global_solution(p.ndof),
+                    b.download_global_reactions(p.ndof)))
+        b.finalize()
+    assert out[0][0] == out[1][0]
+    for x, y in zip(out[0][1:], out[1][1:]):
+        assert np.abs(x - y).max() <= 1e-8 * np.abs(x).max()
+
+
 @pytest.mark.parametrize("nel", [4, 12])
 @pytest.mark.parametrize("place", [0, 0.4, 1.0])
 def test_bad_entries_are_refused(nel, place):
@@ -59,6 +145,31 @@ def test_bad_entries_are_refused(nel, place):
             b.upload_subdomain_data(bad)
         b.upload_subdomain_data(d)
         b.finalize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("place", [0, 0.4, 1.0])
+def test_bad_entries_are_refused_before_the_device(place):
+    """The same on the device path: refused by the upload, on the host, and
+    the next upload of the subdomain is taken."""
+    print("case bad entries", place, flush=True)
+    p = CubeProblem(8, 2, rhs="random", seed=3)
+    subs = list(p.subdomains())
+    d = subs[0]
+    k = int(place * (len(d["a_sparse"]) - 1))
+    b = bddcml_amd.Bddcml()
+    b.init(2, [p.nsub, 1], numbase=p.numbase)
+    for i, j, text in ((5, 3, "upper triangle"), (1, d["ndofs"] + 1, "out of range"),
+                       (0, 3, "out of range")):
+        bad = dict(d, i_sparse=d["i_sparse"].copy(), j_sparse=d["j_sparse"].copy())
+        bad["i_sparse"][k], bad["j_sparse"][k] = i, j
+        with pytest.raises(RuntimeError, match=text):
+            b.upload_subdomain_data(bad)
+    for s in subs:
+        b.upload_subdomain_data(s)
+    b.setup_preconditioner()
+    assert b.solve(0, 1e-8, 100, 50)[1] == 0
+    b.finalize()
 
 
 def test_first_bad_entry_names_the_error():
