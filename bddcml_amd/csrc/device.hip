@@ -358,12 +358,13 @@ struct Device {
   int maxNI = 0, maxnc = 0, maxnti = 0, maxnt = 1, maxncT = 0;
   bool kapply_deep = false;  // form of the local preconditioner launch
   int64_t LV = 0;
-  View<SymvCol> scols;
-  View<SymvCol> pcols;  // the same columns over the explicit S'^{-1} tiles
+  SymvPlan symv;
+  View<SymvGroup> sgrps;
+  View<SymvGroup> pgrps;  // the same groups over the explicit S'^{-1} tiles
   View<SymvRow> srows;
-  DBuf<double> spart;  // partial slots of the symmetric S GEMV
+  DBuf<double> spart;  // the groups' vectors of the symmetric S GEMV
   DBuf<double> cpart;  // partial slots of the coarse GEMV
-  int nscols = 0, nsrows = 0;
+  int nsgrps = 0, nsrows = 0;
   View<int> aptr;
   View<int64_t> asrc;
   View<int> cgptr, cgsrc;
@@ -2070,40 +2071,33 @@ void device_setup_interface(Solver &S) {
   D.Phi.alloc(std::max<int64_t>(zo, 1));
   D.G.alloc(std::max<int64_t>(go, 1));
   D.Acs.alloc(std::max<int64_t>(go, 1));
-  // symmetric S GEMV: tile columns, longest first, and reduce rows; coarse
-  // GEMV rows
-  std::vector<SymvCol> sc;
+  // symmetric S GEMV: groups of tile columns and reduce rows; coarse GEMV rows
+  std::vector<SymvGroup> sg;
   std::vector<SymvRow> sr;
   {
-    int64_t ps = 0;
+    std::vector<int> nti(nsub);
+    for (int is = 0; is < nsub; is++) nti[is] = D.sub[is].nti;
+    D.symv = symv_plan(nti);
+    int64_t po = 0;
     for (int is = 0; is < nsub; is++) {
       const SubTiles &T = D.sub[is];
-      for (int I = 0; I < T.nti; I++) sr.push_back({is, I, (int)ps, T.nti});
-      ps += (int64_t)T.nti * (T.nti + 1) / 2;
+      const int n = T.nti, P = D.symv.groups[is];
+      if (T.slow < 0 || (int64_t)T.slow + (int64_t)n * (n + 1) / 2 > D.ntiles || P < 1 || P > n)
+        fatal("BDDCML_DEVICE_PLAN", "invalid GEMV group");
+      for (int I = 0; I < n; I++) sr.push_back({is, I, n, P, po});
+      for (int g = 0; g < P; g++) sg.push_back({T.slow, n, is, g, P, po + (int64_t)g * n * 64});
+      po += (int64_t)P * n * 64;
     }
-    if (ps >= INT32_MAX) fatal("BDDCML_DEVICE_PLAN", "too many interface tiles");
-    for (int J = 0; J < D.maxnti; J++)
-      for (int is = 0; is < nsub; is++) {
-        const SubTiles &T = D.sub[is];
-        if (J < T.nti)
-          sc.push_back({T.slow + lowidx(T.nti, J, J), T.nti - J, is, J,
-                        0});  // pslot set below
-      }
-    std::vector<int> psub(nsub);
-    for (const SymvRow &r : sr) psub[r.mat] = r.psub;
-    for (SymvCol &c : sc) c.pslot = psub[c.mat] + lowidx(D.sub[c.mat].nti, c.J, c.J);
-    std::stable_sort(sc.begin(), sc.end(), [](const SymvCol &a, const SymvCol &b) { return a.nt > b.nt; });
-    for (const SymvCol &c : sc)
-      if (c.tile0 < 0 || (int64_t)c.tile0 + c.nt > D.ntiles) fatal("BDDCML_DEVICE_PLAN", "invalid GEMV column");
     if (D.inv_planned) {
-      std::vector<SymvCol> pc(sc);
-      for (SymvCol &c : pc) {
-        c.tile0 = D.sub[c.mat].pbase + lowidx(D.sub[c.mat].nti, c.J, c.J);
-        if (c.tile0 < 0 || (int64_t)c.tile0 + c.nt > D.ntilesf) fatal("BDDCML_DEVICE_PLAN", "invalid GEMV column");
+      std::vector<SymvGroup> pg(sg);
+      for (SymvGroup &g : pg) {
+        g.tile0 = D.sub[g.mat].pbase;
+        if (g.tile0 < 0 || (int64_t)g.tile0 + (int64_t)g.n * (g.n + 1) / 2 > D.ntilesf)
+          fatal("BDDCML_DEVICE_PLAN", "invalid GEMV group");
       }
-      D.plan2.add(D.pcols, pc);
+      D.plan2.add(D.pgrps, pg);
     }
-    D.spart.alloc((size_t)std::max<int64_t>(ps, 1) * 64);
+    D.spart.alloc((size_t)std::max<int64_t>(po, 1));
   }
   // coarse inverse GEMV over the full-storage tiles
   if (D.dense_coarse) {
@@ -2111,10 +2105,10 @@ void device_setup_interface(Solver &S) {
       fatal("BDDCML_DEVICE_PLAN", "invalid coarse GEMV tiles");
     D.cpart.alloc((size_t)D.ntc * D.ntc * 64);
   }
-  D.plan2.add(D.scols, sc);
+  D.plan2.add(D.sgrps, sg);
   D.plan2.add(D.srows, sr);
   D.nsrows = (int)sr.size();
-  D.nscols = (int)sc.size();
+  D.nsgrps = (int)sg.size();
   ph("interface maps");
   // coarse gather CSR: coarse dof -> constraint rows (subdomain order)
   {
@@ -2923,11 +2917,11 @@ static void op_schur(Solver &S, const double *x, double *y, bool timed = false) 
     HIPCHECK(hipEventRecord(D.ev_apply[0], D.st));
   }
   if (D.f32i)
-    launch_symv(D.st, (const float *)D.ipool32.p, D.scols.p, D.nscols, D.srows.p, D.nsrows,
-                D.loff.p, D.map.p, x, D.spart.p, D.yl.p);
+    launch_symv(D.st, (const float *)D.ipool32.p, D.sgrps.p, D.nsgrps, D.symv, D.srows.p,
+                D.nsrows, D.loff.p, D.map.p, x, D.spart.p, D.yl.p);
   else
-    launch_symv(D.st, (const double *)D.pool.p, D.scols.p, D.nscols, D.srows.p, D.nsrows,
-                D.loff.p, D.map.p, x, D.spart.p, D.yl.p);
+    launch_symv(D.st, (const double *)D.pool.p, D.sgrps.p, D.nsgrps, D.symv, D.srows.p,
+                D.nsrows, D.loff.p, D.map.p, x, D.spart.p, D.yl.p);
   if (timed) {
     HIPCHECK(hipEventRecord(D.ev_apply[1], D.st));
     double tiles = 0;
@@ -3023,8 +3017,8 @@ static void op_pc(Solver &S, const double *r, double *z, bool timed) {
   }
   auto local = [&](const auto *fp) {
     if (D.explicit_inv)
-      launch_inverse_apply(st, fp, D.pcols.p, D.nscols, D.srows.p, D.nsrows, D.desc.p, D.loff.p,
-                           D.map.p, D.w.p, r, D.spart.p, D.Phi.p, D.cmap.p, D.uc.p, D.zts.p,
+      launch_inverse_apply(st, fp, D.pgrps.p, D.nsgrps, D.symv, D.srows.p, D.nsrows, D.desc.p,
+                           D.loff.p, D.map.p, D.w.p, r, D.spart.p, D.Phi.p, D.cmap.p, D.uc.p, D.zts.p,
                            D.zl.p, D.maxnc);
     else
       launch_kapply(st, fp, D.desc.p, S.nsub, D.map.p, D.w.p, r, D.Phi.p, D.Z.p, D.cmap.p, D.uc.p,

@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <vector>
 
 #include "plan.hpp"
 
@@ -246,21 +247,28 @@ void launch_ifc_scatter(hipStream_t st, int n, const int *ptr, const int64_t *po
 // ---- iteration kernels ---------------------------------------------------
 // Symmetric tile GEMV over the packed lower tiles of each subdomain's S:
 // y_local[loff + I*64 + r] = sum_J S(I,J) x_J with x_J[r] = xin[map[loff + J*64 + r]]
-// (0 where map < 0).  One workgroup per tile column (SymvCol) writes partial
-// slots (I, J) of `part` (64 doubles each, packed like the tiles); the reduce
-// sums each row's slots in a fixed order.
-struct SymvCol {
-  int tile0;  // tile (J, J); the column's tiles (I, J), I = J..nti-1, follow
-  int nt;     // nti - J
+// (0 where map < 0).  One workgroup per group of tile columns (SymvGroup)
+// writes its sums over the whole subdomain to its vector in `part`; the
+// reduce adds the groups' vectors in order.
+struct SymvGroup {
+  int tile0;  // tile (0, 0) of the packed lower tiles
+  int n;      // tile rows
   int mat;    // subdomain
-  int J;
-  int pslot;  // partial slot of (J, J)
+  int J0, P;  // this group and their number (P = n: single columns)
+  int64_t poff;  // its vector (64 n doubles) in part
 };
 struct SymvRow {
   int mat, I;
-  int psub;   // partial slot of the subdomain's (0, 0)
-  int nti;
+  int n, P;
+  int64_t poff;  // the vector of the subdomain's first group
 };
+// groups per subdomain, and how the launch uses LDS (bytes; input staged)
+struct SymvPlan {
+  std::vector<int> groups;
+  size_t lds = 0;
+  bool stage = false;
+};
+SymvPlan symv_plan(const std::vector<int> &n);
 // block-sparse tile GEMV: per task y[yoff..yoff+64) = (b ? b[boff..] : 0) +
 // sign * sum over its pairs of op(tile) x[xoff..xoff+64), op the tile or
 // (trans) its transpose; tiles column major in pool.  A task may write the
@@ -277,7 +285,7 @@ void launch_tile_gemv(hipStream_t st, const double *pool, const GemvTask *tasks,
                       const GemvPair *pairs, const double *x, const double *b, double *y, int trans,
                       double sign);
 template <typename T>
-void launch_symv(hipStream_t st, const T *pool, const SymvCol *cols, int ncols,
+void launch_symv(hipStream_t st, const T *pool, const SymvGroup *grps, int ngrps, const SymvPlan &pl,
                  const SymvRow *rows, int nrows, const int64_t *loff, const int *map,
                  const double *xin, double *part, double *yout);
 // y = A x for a dense nt x nt tile matrix in full storage (tile (I, J) at
@@ -303,14 +311,14 @@ void launch_kapply(hipStream_t st, const T *pool, const SubDesc *subs, int nsub,
                    const double *w, const double *r, const double *Phi, const double *Z,
                    const int *cmap, const double *uc, double *zl, int maxNI, int maxnc, bool deep);
 // The same local part through the explicit inverse: z = S'^{-1} x by the
-// symmetric tile GEMV over cols (tiles of the factor pool), summed per tile
+// symmetric tile GEMV over grps (tiles of the factor pool), summed per tile
 // row together with Phi (uc(indrowc) - zts); zts = Z^T x from launch_phit.
 template <typename T>
-void launch_inverse_apply(hipStream_t st, const T *pool, const SymvCol *cols, int ncols,
-                          const SymvRow *rows, int nrows, const SubDesc *subs, const int64_t *loff,
-                          const int *map, const double *wts, const double *xin, double *part,
-                          const double *Phi, const int *cmap, const double *uc, const double *zts,
-                          double *zl, int maxnc);
+void launch_inverse_apply(hipStream_t st, const T *pool, const SymvGroup *grps, int ngrps,
+                          const SymvPlan &pl, const SymvRow *rows, int nrows, const SubDesc *subs,
+                          const int64_t *loff, const int *map, const double *wts, const double *xin,
+                          double *part, const double *Phi, const int *cmap, const double *uc,
+                          const double *zts, double *zl, int maxnc);
 
 // deterministic reductions and vector updates on unique vectors
 constexpr int DOT_BLOCKS = 240;

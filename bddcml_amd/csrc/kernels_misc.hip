@@ -719,84 +719,155 @@ template void launch_trsv_bwd<float>(hipStream_t, const float *, const TrsvDesc 
                                      const int *, const int *, double *, int);
 
 // -------------------------------------------------------- iteration kernels
-// y = S x for symmetric S held as its lower tiles.  Workgroup = tile column
-// J of one subdomain; wave w reads columns 16w..16w+15 of each tile (lane =
-// row, one coalesced 512-byte column per load), the next tile prefetched.
-// Slot (I, J), I > J, receives S_IJ x_J; slot (J, J) receives S_JJ x_J plus
-// sum_{I>J} S_IJ^T x_I (lane products summed over rows by butterflies).
-// T: element type of the tiles (double: S; float or double: an explicit
-// S'^{-1} in the factor space).  wts (may be null): per local entry weight
-// applied to the gathered input.
-template <typename T>
+__device__ __forceinline__ int packed_lower(int n, int I, int J) {
+  return J * n - J * (J - 1) / 2 + (I - J);
+}
+
+// y = S x for symmetric S held as its lower tiles, read once.  A workgroup
+// walks the tile columns of one group (J0, 2P-1-J0, 2P+J0, ... of P groups:
+// equal tile counts) and adds S_IJ x_J to row I and S_IJ^T x_I to row J of a
+// vector in LDS, written to part once; the groups' vectors are summed by
+// k_symv_reduce.  A single-column group (P = n: few or very large subdomains)
+// needs no LDS vector and writes every row as it comes.
+//
+// HBM-bound, by the one read of the tiles.  What kept the form with one
+// workgroup per tile column at 5.2 (FP64) and 4.4 TB/s (FP32) was not the
+// reads: 512 bytes of partial sums written per tile (1.6 % of the bytes) cost
+// 16 %, and tiles passing through the caches as if they were read again
+// another 9 %.  So the row sums stay in LDS, the tiles are read with
+// nontemporal 16-byte loads, and there are two workgroups per CU, no more
+// (symv_groups): 512 subdomains of 25 tile rows 1.07 -> 0.80 ms FP64 (6.8
+// TB/s; a plain read of the same bytes 0.87), 216 in FP32 0.272 -> 0.207 ms,
+// 36 of 35 rows 0.156 -> 0.120 ms.
+//
+// Wave w takes columns 16w..16w+15 of each tile, a lane RPL consecutive rows
+// of every CPI-th of them; the next tile is loaded ahead.  T: element type of
+// the tiles.  wts (may be null): weight of each local entry, applied to the
+// gathered input; XL: the subdomain's input staged in LDS, else gathered tile
+// by tile.
+template <typename T, bool XL>
 __global__ __launch_bounds__(256) void k_symv(const T *__restrict__ pool,
-                                              const SymvCol *__restrict__ cols,
+                                              const SymvGroup *__restrict__ grps,
                                               const int64_t *__restrict__ loff,
                                               const int *__restrict__ map,
                                               const double *__restrict__ wts,
                                               const double *__restrict__ xin,
                                               double *__restrict__ part) {
-  __shared__ double xj[64];
+  constexpr int RPL = 16 / (int)sizeof(T), LPC = 64 / RPL, CPI = 64 / LPC, NQ = 16 / CPI;
+  typedef T vec __attribute__((ext_vector_type(RPL)));
+  extern __shared__ double sm[];
   __shared__ double red[2][4][64];
   __shared__ double dg[64];
-  const SymvCol col = cols[blockIdx.x];
-  const int64_t lo = loff[col.mat];
-  const int tid = threadIdx.x, w = tid >> 6, r = tid & 63;
+  const SymvGroup g = grps[blockIdx.x];
+  const int n = g.n, P = g.P, NI = 64 * n;
+  const bool direct = P == n;
+  const int64_t lo = loff[g.mat];
+  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, h = l / LPC, r = RPL * (l % LPC);
   const int *mp = map + lo;
-  if (tid < 64) {
-    const int g = mp[col.J * 64 + tid];
-    xj[tid] = g >= 0 ? (wts ? wts[lo + col.J * 64 + tid] * xin[g] : xin[g]) : 0.0;
-  }
+  double *xs = sm, *ra = XL ? sm + NI : sm;
+  auto gather = [&](int e) {
+    const int q = mp[e];
+    return q >= 0 ? (wts ? wts[lo + e] * xin[q] : xin[q]) : 0.0;
+  };
+  auto xval = [&](int e) { return XL ? xs[e] : gather(e); };
+  if (XL)
+    for (int e = tid; e < NI; e += 256) xs[e] = gather(e);
+  if (!direct)
+    for (int e = tid; e < NI; e += 256) ra[e] = 0.0;
   __syncthreads();
-  double xc[16], acc[16], cur[16], nxt[16];
+  double *out = part + g.poff;
+  int b = 0;
+  for (int m = 0; m * P < n; m++) {
+    const int J = (m & 1) ? (m + 1) * P - 1 - g.J0 : m * P + g.J0;
+    if (J >= n) continue;
+    const int nt = n - J;
+    const T *T0 = pool + (size_t)(g.tile0 + packed_lower(n, J, J)) * TILE_ELEMS + (16 * w + h) * 64 + r;
+    double xc[NQ], acc[NQ], xi[RPL], xn[RPL];
+    vec cur[NQ], nxt[NQ];
 #pragma unroll
-  for (int c = 0; c < 16; c++) xc[c] = xj[16 * w + c], acc[c] = 0.0;
-  const T *T0 = pool + (size_t)col.tile0 * TILE_ELEMS + (16 * w) * 64 + r;
+    for (int q = 0; q < NQ; q++)
+      cur[q] = __builtin_nontemporal_load(reinterpret_cast<const vec *>(T0 + q * CPI * 64));
 #pragma unroll
-  for (int c = 0; c < 16; c++) cur[c] = (double)T0[c * 64];
-  double xi = 0.0;  // x_I[r] of the current tile (I > J)
-  for (int k = 0; k < col.nt; k++) {
-    double xn = 0.0;
-    if (k + 1 < col.nt) {
-      const T *Tn = T0 + (size_t)(k + 1) * TILE_ELEMS;
+    for (int q = 0; q < NQ; q++) xc[q] = xval(J * 64 + 16 * w + CPI * q + h), acc[q] = 0.0;
 #pragma unroll
-      for (int c = 0; c < 16; c++) nxt[c] = (double)Tn[c * 64];
-      const int g = mp[(col.J + k + 1) * 64 + r];
-      xn = g >= 0 ? (wts ? wts[lo + (col.J + k + 1) * 64 + r] * xin[g] : xin[g]) : 0.0;
+    for (int i = 0; i < RPL; i++) xi[i] = 0.0;  // the diagonal tile adds no transpose
+    for (int k = 0; k < nt; k++, b ^= 1) {
+      if (k + 1 < nt) {
+        const T *Tn = T0 + (size_t)(k + 1) * TILE_ELEMS;
+#pragma unroll
+        for (int q = 0; q < NQ; q++)
+          nxt[q] = __builtin_nontemporal_load(reinterpret_cast<const vec *>(Tn + q * CPI * 64));
+#pragma unroll
+        for (int i = 0; i < RPL; i++) xn[i] = xval((J + k + 1) * 64 + r + i);
+      }
+      double s[RPL];
+#pragma unroll
+      for (int i = 0; i < RPL; i++) s[i] = 0.0;
+#pragma unroll
+      for (int q = 0; q < NQ; q++) {
+        double t = 0.0;
+#pragma unroll
+        for (int i = 0; i < RPL; i++) {
+          const double e = (double)cur[q][i];
+          s[i] += e * xc[q];
+          t += e * xi[i];
+        }
+        acc[q] += t;
+      }
+#pragma unroll
+      for (int o = LPC; o < 64; o <<= 1)
+#pragma unroll
+        for (int i = 0; i < RPL; i++) s[i] += __shfl_xor(s[i], o);
+      if (h == 0) {
+#pragma unroll
+        for (int i = 0; i < RPL; i++) red[b][w][r + i] = s[i];
+      }
+      __syncthreads();
+      if (w == (k & 3)) {
+        const double v = (red[b][0][l] + red[b][1][l]) + (red[b][2][l] + red[b][3][l]);
+        if (!direct) ra[(J + k) * 64 + l] += v;
+        else if (k == 0) dg[l] = v;
+        else out[(J + k) * 64 + l] = v;
+      }
+#pragma unroll
+      for (int q = 0; q < NQ; q++) cur[q] = nxt[q];
+#pragma unroll
+      for (int i = 0; i < RPL; i++) xi[i] = xn[i];
     }
-    double s0 = 0.0, s1 = 0.0;
+    // S_IJ^T x_I: each column's sum over its LPC lanes
+    double mine = 0.0;
 #pragma unroll
-    for (int c = 0; c < 16; c += 2) s0 += cur[c] * xc[c], s1 += cur[c + 1] * xc[c + 1];
-    if (k > 0) {
+    for (int q = 0; q < NQ; q++) {
+      double v = acc[q];
 #pragma unroll
-      for (int c = 0; c < 16; c++) acc[c] += cur[c] * xi;
+      for (int o = LPC / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
+      if (l % LPC == q) mine = v;
     }
-    red[k & 1][w][r] = s0 + s1;
     __syncthreads();
-    if (w == 0) {
-      const double v = (red[k & 1][0][r] + red[k & 1][1][r]) + (red[k & 1][2][r] + red[k & 1][3][r]);
-      if (k == 0)
-        dg[r] = v;
-      else
-        part[(size_t)(col.pslot + k) * 64 + r] = v;
+    if (l % LPC < NQ) {
+      const int c = 16 * w + CPI * (l % LPC) + h;
+      if (direct) out[J * 64 + c] = dg[c] + mine;
+      else ra[J * 64 + c] += mine;
     }
-#pragma unroll
-    for (int c = 0; c < 16; c++) cur[c] = nxt[c];
-    xi = xn;
+    __syncthreads();
   }
-  double mine = 0.0;
-#pragma unroll
-  for (int c = 0; c < 16; c++) {
-    double v = acc[c];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    if (r == c) mine = v;
-  }
-  __syncthreads();
-  if (r < 16) part[(size_t)col.pslot * 64 + 16 * w + r] = dg[16 * w + r] + mine;
+  if (!direct)
+    for (int e = tid; e < NI; e += 256) out[e] = ra[e];
 }
 
-// y_local[loff + I*64 + r] = sum_{J <= I} slot(I, J)[r], J ascending; one
-// wave per row
+// sum of the groups' vectors at row tile I, entry r (a single-column group J
+// holds rows I >= J only); the groups p0, p0 + step, ...
+__device__ __forceinline__ double symv_sum(const SymvRow &R, const double *__restrict__ part, int r,
+                                           int p0, int step) {
+  const int np = R.P == R.n ? R.I + 1 : R.P;
+  const double *q = part + R.poff + R.I * 64 + r;
+  double s = 0.0;
+#pragma unroll 4
+  for (int p = p0; p < np; p += step) s += q[(size_t)p * R.n * 64];
+  return s;
+}
+
+// y_local[loff + I*64 + r], one wave per row tile
 __global__ __launch_bounds__(256) void k_symv_reduce(const SymvRow *__restrict__ rows, int nrows,
                                                      const int64_t *__restrict__ loff,
                                                      const double *__restrict__ part,
@@ -804,11 +875,7 @@ __global__ __launch_bounds__(256) void k_symv_reduce(const SymvRow *__restrict__
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6), r = threadIdx.x & 63;
   if (row >= nrows) return;
   const SymvRow R = rows[row];
-  double s = 0.0;
-#pragma unroll 8
-  for (int J = 0; J <= R.I; J++)
-    s += part[(size_t)(R.psub + J * R.nti - J * (J - 1) / 2 + (R.I - J)) * 64 + r];
-  yout[loff[R.mat] + R.I * 64 + r] = s;
+  yout[loff[R.mat] + R.I * 64 + r] = symv_sum(R, part, r, 0, 1);
 }
 
 // The same sums with the coarse-basis part of the local preconditioner
@@ -829,10 +896,7 @@ __global__ __launch_bounds__(256) void k_symv_reduce_phi(
   const SubDesc d = subs[R.mat];
   const int w = threadIdx.x >> 6, r = threadIdx.x & 63;
   for (int c = threadIdx.x; c < d.nc; c += 256) cc[c] = uc[cmap[d.coff + c]] - zts[d.coff + c];
-  double s = 0.0;
-#pragma unroll 4
-  for (int J = w; J <= R.I; J += 4)
-    s += part[(size_t)(R.psub + J * R.nti - J * (J - 1) / 2 + (R.I - J)) * 64 + r];
+  double s = symv_sum(R, part, r, w, 4);
   __syncthreads();
   const double *P = Phi + d.zoff + R.I * 64 + r;
 #pragma unroll 4
@@ -842,44 +906,79 @@ __global__ __launch_bounds__(256) void k_symv_reduce_phi(
   if (w == 0) zl[d.loff + R.I * 64 + r] = (red[0][r] + red[1][r]) + (red[2][r] + red[3][r]);
 }
 
+// Groups of every subdomain's tile columns (tile counts n): about two
+// workgroups per CU in all, shared by tile count.  More of them lost (36
+// subdomains of 35 rows: 504 workgroups 0.120 ms, 720 0.129, 1,044 0.143; 64
+// of 25 rows: 512 0.108, 1,024 0.124), fewer left CUs idle (216: 0.131).
+// LDS holds the output vector of a subdomain, and its input where both fit
+// twice into a CU; a subdomain too large for the vector takes single-column
+// groups.
+SymvPlan symv_plan(const std::vector<int> &n) {
+  SymvPlan o;
+  double total = 0.0;
+  int nmax = 0;
+  for (int k : n) total += 0.5 * k * (k + 1.0), nmax = std::max(nmax, k);
+  const size_t room = max_dynamic_lds() - 8192;  // beside the static arrays
+  o.groups.resize(n.size());
+  for (size_t i = 0; i < n.size(); i++) {
+    const double share = total > 0.0 ? 512.0 * 0.5 * n[i] * (n[i] + 1.0) / total : 1.0;
+    int P = std::max(1, std::min(n[i], (int)(share + 0.5)));
+    if ((size_t)n[i] * 512 > room) P = n[i];
+    o.groups[i] = P;
+    if (P < n[i]) o.lds = std::max(o.lds, (size_t)n[i] * 512);
+  }
+  o.stage = o.lds + (size_t)nmax * 512 <= (size_t)72 << 10;
+  if (o.stage) o.lds += (size_t)nmax * 512;
+  return o;
+}
 template <typename T>
-void launch_symv(hipStream_t st, const T *pool, const SymvCol *cols, int ncols,
+static void symv_groups(hipStream_t st, const T *pool, const SymvGroup *grps, int ngrps,
+                        const SymvPlan &pl, const int64_t *loff, const int *map, const double *wts,
+                        const double *xin, double *part) {
+  auto go = [&](auto kernel) {
+    lds_request((const void *)kernel, pl.lds, "symmetric GEMV");
+    hipLaunchKernelGGL(kernel, dim3(ngrps), dim3(256), pl.lds, st, pool, grps, loff, map, wts, xin,
+                       part);
+  };
+  if (pl.stage) go(k_symv<T, true>);
+  else go(k_symv<T, false>);
+}
+template <typename T>
+void launch_symv(hipStream_t st, const T *pool, const SymvGroup *grps, int ngrps, const SymvPlan &pl,
                  const SymvRow *rows, int nrows, const int64_t *loff, const int *map,
                  const double *xin, double *part, double *yout) {
-  if (ncols <= 0 || nrows <= 0) return;
-  hipLaunchKernelGGL(k_symv<T>, dim3(ncols), dim3(256), 0, st, pool, cols, loff, map, nullptr, xin,
-                     part);
+  if (ngrps <= 0 || nrows <= 0) return;
+  symv_groups(st, pool, grps, ngrps, pl, loff, map, nullptr, xin, part);
   hipLaunchKernelGGL(k_symv_reduce, dim3((nrows + 3) / 4), dim3(256), 0, st, rows, nrows, loff,
                      part, yout);
 }
 template <typename T>
-void launch_inverse_apply(hipStream_t st, const T *pool, const SymvCol *cols, int ncols,
-                          const SymvRow *rows, int nrows, const SubDesc *subs, const int64_t *loff,
-                          const int *map, const double *wts, const double *xin, double *part,
-                          const double *Phi, const int *cmap, const double *uc, const double *zts,
-                          double *zl, int maxnc) {
-  if (ncols <= 0 || nrows <= 0) return;
-  hipLaunchKernelGGL(k_symv<T>, dim3(ncols), dim3(256), 0, st, pool, cols, loff, map, wts, xin,
-                     part);
+void launch_inverse_apply(hipStream_t st, const T *pool, const SymvGroup *grps, int ngrps,
+                          const SymvPlan &pl, const SymvRow *rows, int nrows, const SubDesc *subs,
+                          const int64_t *loff, const int *map, const double *wts, const double *xin,
+                          double *part, const double *Phi, const int *cmap, const double *uc,
+                          const double *zts, double *zl, int maxnc) {
+  if (ngrps <= 0 || nrows <= 0) return;
+  symv_groups(st, pool, grps, ngrps, pl, loff, map, wts, xin, part);
   hipLaunchKernelGGL(k_symv_reduce_phi, dim3(nrows), dim3(256), (size_t)maxnc * sizeof(double), st,
                      rows, subs, part, Phi, cmap, uc, zts, zl);
 }
-template void launch_inverse_apply<double>(hipStream_t, const double *, const SymvCol *, int,
-                                           const SymvRow *, int, const SubDesc *, const int64_t *,
-                                           const int *, const double *, const double *, double *,
-                                           const double *, const int *, const double *,
-                                           const double *, double *, int);
-template void launch_inverse_apply<float>(hipStream_t, const float *, const SymvCol *, int,
-                                          const SymvRow *, int, const SubDesc *, const int64_t *,
-                                          const int *, const double *, const double *, double *,
-                                          const double *, const int *, const double *,
-                                          const double *, double *, int);
-template void launch_symv<double>(hipStream_t, const double *, const SymvCol *, int,
-                                  const SymvRow *, int, const int64_t *, const int *,
-                                  const double *, double *, double *);
-template void launch_symv<float>(hipStream_t, const float *, const SymvCol *, int, const SymvRow *,
-                                 int, const int64_t *, const int *, const double *, double *,
-                                 double *);
+template void launch_symv<double>(hipStream_t, const double *, const SymvGroup *, int,
+                                  const SymvPlan &, const SymvRow *, int, const int64_t *,
+                                  const int *, const double *, double *, double *);
+template void launch_symv<float>(hipStream_t, const float *, const SymvGroup *, int,
+                                 const SymvPlan &, const SymvRow *, int, const int64_t *,
+                                 const int *, const double *, double *, double *);
+template void launch_inverse_apply<double>(hipStream_t, const double *, const SymvGroup *, int,
+                                           const SymvPlan &, const SymvRow *, int, const SubDesc *,
+                                           const int64_t *, const int *, const double *,
+                                           const double *, double *, const double *, const int *,
+                                           const double *, const double *, double *, int);
+template void launch_inverse_apply<float>(hipStream_t, const float *, const SymvGroup *, int,
+                                          const SymvPlan &, const SymvRow *, int, const SubDesc *,
+                                          const int64_t *, const int *, const double *,
+                                          const double *, double *, const double *, const int *,
+                                          const double *, const double *, double *, int);
 
 // Block-sparse tile GEMV, one workgroup per output segment of 64:
 // y[yoff..] = (b ? b[boff..] : 0) + sign * sum_p op(T_p) x[xoff_p..], op the
@@ -1008,9 +1107,6 @@ __global__ void k_coarse_gather(int n, const int *__restrict__ ptr, const int *_
 // ------------------------------------------------- local preconditioner apply
 constexpr int KA_THR = 1024;  // 16 waves per subdomain
 
-__device__ __forceinline__ int packed_lower(int n, int I, int J) {
-  return J * n - J * (J - 1) / 2 + (I - J);
-}
 
 
 // rcs = Phi_i^T (w .* r(map)) per subdomain, and with the explicit inverse

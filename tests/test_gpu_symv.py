@@ -1,0 +1,41 @@
+"""The symmetric tile GEMV against dense products with the subdomains' Schur
+complements, in each form its launch can take: single-column groups (few
+subdomains), grouped columns with the input in LDS (many), grouped columns
+with the input gathered tile by tile (interfaces of more than 72 tiles); FP64
+and FP32 tiles."""
+import numpy as np
+import pytest
+
+import bddcml_amd
+from bddcml_amd.cube import CubeProblem
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("refined", [0, 1])
+@pytest.mark.parametrize("nel,ns,kind", [(2, 2, "poisson"), (8, 4, "poisson"), (8, 6, "poisson"),
+                                         (5, 5, "elasticity"), (16, 3, "elasticity")])
+def test_schur_apply_equals_dense_products(nel, ns, kind, refined):
+    print("case symmetric GEMV", nel, ns, kind, refined, flush=True)
+    if nel == 16 and refined:
+        pytest.skip("the FP64 case covers the form; FP32 differs in the loads only")
+    p = CubeProblem(nel, ns, kind=kind, rhs="random", seed=3)
+    b = bddcml_amd.Bddcml()
+    b.init(2, [p.nsub, 1], numbase=p.numbase)
+    b.set_option("refinement", refined)
+    for d in p.subdomains():
+        b.upload_subdomain_data(d)
+    b.setup_preconditioner()
+    ig = b.interface_dofs()
+    pos = -np.ones(p.ndof, dtype=int)
+    pos[ig] = np.arange(len(ig))
+    x = np.random.RandomState(5).uniform(-1, 1, len(ig))
+    y = b.apply_schur(x)
+    ref = np.zeros_like(x)
+    for s in range(p.nsub):
+        g, _ = b.sub_maps(s + p.numbase)
+        k = pos[g]
+        np.add.at(ref, k, b.sub_matrix(s + p.numbase) @ x[k])
+    b.finalize()
+    # the same products summed in another order: n eps of the row sums of moduli
+    assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max()
