@@ -1024,13 +1024,24 @@ static std::vector<TaskList> merge_steps(const std::vector<Q> &sts, std::vector<
   return out;
 }
 
-// algorithmic work: 2*64^3 flops per tile product, 64^3/3 per tile Cholesky
-// plus 64^3/3 for its inverse, 2*64^3 per post multiply; pair lists are
-// shared between subdomains, so the pairs of each task are counted
+// work done: 2*64^3 flops per tile product, 64^3/3 per tile Cholesky plus
+// 64^3/3 for its inverse, 2*64^3 per post multiply; of products with masks
+// and of post multiplies by triangular tiles (kTilePost) the 16 x 16 blocks
+// that are computed.  Pair lists are shared between subdomains, so the pairs
+// of each task are counted.
 static const double kTileGemm = 2.0 * 64 * 64 * 64, kTileChol = 64.0 * 64 * 64 / 3.0;
+static const double kTilePost = kTileGemm * 10 / 16;
 static double tile_products(const TaskList &l) {
+  std::vector<double> upto(l.pairs.size() + 1, 0.0);
+  for (size_t p = 0; p < l.pairs.size(); p++) {
+    int blocks = 0;
+    for (int k = 0; k < 16; k += 4)
+      blocks += __builtin_popcount(l.pairs[p].m >> k & 15) *
+                __builtin_popcount(l.pairs[p].m >> (16 + k) & 15);
+    upto[p + 1] = upto[p] + blocks / 64.0;
+  }
   double n = 0;
-  for (const TileTask &t : l.tasks) n += t.p1 - t.p0;
+  for (const TileTask &t : l.tasks) n += upto[t.p1] - upto[t.p0];
   return n;
 }
 // tasks that end with a post multiply or a factorization (a task of its own
@@ -1184,6 +1195,48 @@ void device_setup_begin(Solver &S) {
     }
     Q.a_diag.resize(nlev);
     Q.a_off.resize(nlev);
+    // the factor's nonzero 16 x 16 blocks (symbolic elimination at that
+    // granularity, a bitset of block rows per block column), per tile of the
+    // factored columns bit 4 k + r for block (r, k)
+    std::vector<uint16_t> blocks(T.pat.tile.size(), 0);
+    {
+      const Sub &s = S.subs[reps[ic]];
+      const int nb = 4 * nt, nbo = 4 * nto, nw = (nb + 63) / 64;
+      std::vector<uint64_t> B((size_t)nb * nw, 0);
+      auto set = [&](int J, int I) { B[(size_t)J * nw + (I >> 6)] |= 1ull << (I & 63); };
+      for (int J = 0; J < nbo; J++) set(J, J);
+      for (size_t k = 0; k < s.ai.size(); k++) {
+        const int a = s.perm[s.ai[k]], b = s.perm[s.aj[k]];
+        set(std::min(a, b) >> 4, std::max(a, b) >> 4);
+      }
+      for (int J = 0; J < nbo; J++) {
+        // fill reaches the later columns through the first one (its parent in
+        // the elimination tree); columns of the interface are not needed
+        const uint64_t *c = B.data() + (size_t)J * nw;
+        int w = (J + 1) >> 6;
+        uint64_t v = w < nw ? c[w] & (~0ull << ((J + 1) & 63)) : 0;
+        while (!v && ++w < nw) v = c[w];
+        if (!v) continue;
+        const int I = 64 * w + __builtin_ctzll(v);
+        if (I >= nbo) continue;
+        uint64_t *o = B.data() + (size_t)I * nw;
+        o[w] |= v;
+        for (int x = w + 1; x < nw; x++) o[x] |= c[x];
+      }
+      for (int J = 0; J < nto; J++)
+        for (int q = T.pat.colptr[J]; q < T.pat.colptr[J + 1]; q++) {
+          const int I = T.pat.rowidx[q];
+          unsigned m = 0;
+          for (int k = 0; k < 4; k++) {
+            const uint64_t *c = B.data() + (size_t)(4 * J + k) * nw;
+            m |= (unsigned)((c[(4 * I) >> 6] >> ((4 * I) & 63)) & 15) << (4 * k);
+          }
+          blocks[q] = (uint16_t)m;
+        }
+    }
+    auto block_mask = [&](int ta, int tb) {
+      return (uint32_t)blocks[ta - T.base] | (uint32_t)blocks[tb - T.base] << 16;
+    };
     // pairs (L(I,k), L(J,k)) over the columns k < kmax both rows reach
     // (and that `keep` accepts)
     auto common = [&](int I, int J, int kmax, TaskList &L, auto keep) {
@@ -1194,7 +1247,10 @@ void device_setup_begin(Solver &S) {
         if (a[x] < b[y]) x++;
         else if (b[y] < a[x]) y++;
         else {
-          if (keep(a[x])) L.pairs.push_back({find(I, a[x]), find(J, b[y])});
+          if (keep(a[x])) {
+            const int ta = find(I, a[x]), tb = find(J, b[y]);
+            L.pairs.push_back({ta, tb, block_mask(ta, tb)});
+          }
           x++, y++;
         }
       }
@@ -1534,24 +1590,25 @@ void device_setup_begin(Solver &S) {
                 (size_t)D.sc_pads.n);
 
   S.t.schur_flops = kTileGemm * tile_products(a_schur);
-  S.t.interior_flops = tile_work(a_diag, 2 * kTileChol) + tile_work(a_off, kTileGemm) +
+  S.t.interior_flops = tile_work(a_diag, 2 * kTileChol) + tile_work(a_off, kTilePost) +
                        tile_work(m_rows, kTileGemm) + S.t.schur_flops;
   // ---- numerics, first half: Dirichlet elimination into the tiles,
   // interior factorization, Schur complements
   D.ev_gemm.assign(2 * D.a_off.size(), nullptr);
   for (hipEvent_t &e : D.ev_gemm) HIPCHECK(hipEventCreate(&e));
   D.gemm_flops.clear();
-  for (const TaskList &l : a_off) D.gemm_flops.push_back(kTileGemm * (tile_products(l) + posted_tasks(l)));
+  for (const TaskList &l : a_off)
+    D.gemm_flops.push_back(kTileGemm * tile_products(l) + kTilePost * posted_tasks(l));
   HIPCHECK(hipEventCreateWithFlags(&D.ev_up, hipEventDisableTiming));
   HIPCHECK(hipEventCreateWithFlags(&D.ev_rhs, hipEventDisableTiming));
   // element type of the subdomain tiles: FP64, or FP32 with refinement
   auto interior = [&](auto *pool) {
     for (size_t J = 0; J < D.a_diag.size(); J++) {
       launch_tile_potrf(st, pool, D.a_diag[J].tasks.p, D.a_diag[J].pairs.p, D.a_diag[J].ntask,
-                        D.err.p);
+                        D.err.p, true);
       HIPCHECK(hipEventRecord(D.ev_gemm[2 * J], st));
       launch_tile_gemm(st, pool, D.a_off[J].tasks.p, D.a_off[J].pairs.p, D.a_off[J].ntask, GEMM_NT,
-                       POST_RIGHT_XT, 1.0, -1.0);
+                       POST_RIGHT_XT, 1.0, -1.0, true);
       HIPCHECK(hipEventRecord(D.ev_gemm[2 * J + 1], st));
     }
     HIPCHECK(hipEventRecord(ev[1], st));
@@ -1570,6 +1627,14 @@ void device_setup_begin(Solver &S) {
   S.t.plan += wall_time() - t0;
 }
 
+// S' is dense: all that the skipping products can leave out is the upper half
+// of the inverse diagonal tile.  That pays in FP64 (interface phase of 512
+// subdomains of 16^3 19.58 -> 18.87 ms); the FP32 products, whose matrix
+// instructions take half the time, lose more to reading each operand block
+// once per product (9.64 -> 10.23 ms).
+template <typename P>
+constexpr bool skip_interface = std::is_same<P, double *>::value;
+
 // Explicit inverse of S' on the compute stream: W = L^{-1} row by row, then
 // S'^{-1} = W^T W over the factor tiles (the factor is not needed after
 // that: later applies use the GEMV).  Launches queued behind work already on
@@ -1578,9 +1643,10 @@ static void form_inverse(Solver &S) {
   Device &D = *S.dev;
   hipStream_t st = D.st;
   auto run = [&](auto *fp) {
+    constexpr bool skip = skip_interface<decltype(fp)>;
     for (size_t i = 0; i < D.w_rows.size(); i++)
       launch_tile_gemm(st, fp, D.w_rows[i].tasks.p, D.w_rows[i].pairs.p, D.w_rows[i].ntask, GEMM_NN,
-                       POST_LEFT_X, 1.0, -1.0);
+                       POST_LEFT_X, 1.0, -1.0, skip);
     launch_tile_gemm(st, fp, D.kinv.tasks.p, D.kinv.pairs.p, D.kinv.ntask, GEMM_TN, POST_NONE, 1.0,
                      1.0);
   };
@@ -2153,11 +2219,11 @@ void device_setup_interface(Solver &S) {
     for (size_t J = 0; J < D.p_diag.size(); J++) {
       launch_tile_potrf(st, fp, D.p_diag[J].tasks.p, D.p_diag[J].pairs.p, D.p_diag[J].ntask, D.err.p);
       launch_tile_gemm(st, fp, D.p_off[J].tasks.p, D.p_off[J].pairs.p, D.p_off[J].ntask, GEMM_NT,
-                       POST_RIGHT_XT, 1.0, -1.0);
+                       POST_RIGHT_XT, 1.0, -1.0, skip_interface<decltype(fp)>);
     }
     for (size_t i = 0; i < D.z_bwd.size(); i++)
       launch_tile_gemm(st, fp, D.z_bwd[i].tasks.p, D.z_bwd[i].pairs.p, D.z_bwd[i].ntask, GEMM_TN,
-                       POST_LEFT_XT, 1.0, -1.0);
+                       POST_LEFT_XT, 1.0, -1.0, skip_interface<decltype(fp)>);
     launch_y_to_z(st, fp, D.desc.p, nsub, D.Z.p, D.maxNI, 0);
   };
   // Phi = Z G^{-1} on the tile GEMM, in the factor space

@@ -19,10 +19,12 @@ enum GemmKind { GEMM_NT = 0, GEMM_NN = 1, GEMM_TN = 2 };
 // post operations on E after the sum
 enum GemmPost { POST_NONE = 0, POST_RIGHT_XT = 1, POST_LEFT_X = 2, POST_LEFT_XT = 3 };
 
-// T = double or float (tile pool element type)
+// T = double or float (tile pool element type).  skip: products follow the
+// pairs' masks (TilePair::m) and X of the post operations is lower triangular
+// (an inverse diagonal tile); without it both are taken as dense.
 template <typename T>
 void launch_tile_gemm(hipStream_t st, T *pool, const TileTask *tasks, const TilePair *pairs,
-                      int ntasks, int kind, int post, double alpha, double beta);
+                      int ntasks, int kind, int post, double alpha, double beta, bool skip = false);
 // a symmetric matrix per subdomain (packed lower tiles from tile0, nt tile
 // rows) times a set of columns scattered in memory (col0: first entry of the
 // subdomain's column offsets)
@@ -47,7 +49,7 @@ void launch_schur_gemm(hipStream_t st, float *pool, const TileTask *tasks, const
 // C = C - sum A B^T ; C = chol(C) (lower, upper zeroed) ; X = inv(C)
 template <typename T>
 void launch_tile_potrf(hipStream_t st, T *pool, const TileTask *tasks, const TilePair *pairs,
-                       int ntasks, int *err);
+                       int ntasks, int *err, bool skip = false);
 // tasks of mixed kinds in one launch: tile products with their own mode
 // (task_mode) and tile factorizations (mode kTaskPotrf, C and inverse tile x)
 void launch_tile_step(hipStream_t st, double *pool, const TileTask *tasks, const TilePair *pairs,

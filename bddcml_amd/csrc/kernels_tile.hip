@@ -1,8 +1,8 @@
 // kernels_tile.hip -- batched 64x64 tile algebra on CDNA4 matrix cores, FP64
 // (and FP32 for the preconditioner factors of the mixed-precision mode).
 //
-// One workgroup (4 waves) owns one output tile.  Each wave computes a 32x32
-// quadrant as 2x2 blocks of 16x16x4 MFMA accumulators; operand tiles
+// One workgroup (4 waves) owns one output tile.  Each wave computes 2x2 of
+// its 4x4 blocks of 16x16 in 16x16x4 MFMA accumulators; operand tiles
 // are staged through LDS with a padded leading dimension.  These kernels
 // carry every dense factorisation of the path: the partial Cholesky of the
 // subdomain matrices (Schur complements), the Cholesky / inverse of the
@@ -23,6 +23,7 @@ template <> struct Mfma<double> {
   typedef double v4 __attribute__((ext_vector_type(4)));
   typedef double2 vec;  // 16-byte global access
   static constexpr int VE = 2;
+  static constexpr int WPS = 2;  // waves per SIMD that the tiles' LDS allows
   __device__ static __forceinline__ v4 op(double a, double b, v4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
@@ -32,6 +33,7 @@ template <> struct Mfma<float> {
   typedef float v4 __attribute__((ext_vector_type(4)));
   typedef float4 vec;
   static constexpr int VE = 4;
+  static constexpr int WPS = 4;
   __device__ static __forceinline__ v4 op(float a, float b, v4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
@@ -105,20 +107,29 @@ template <typename T> __device__ __forceinline__ void lds_to_tile(const T *lds, 
   }
 }
 
-// acc(r,c) += sum_q As[q*LDL + r] * Bs[q*LDL + c] over this wave's 32x32
-// quadrant, as 2x2 blocks of 16x16
+// Each wave computes 2x2 of the output tile's 4x4 blocks of 16x16: rows
+// blocks wr and wr + 2, column blocks wc and wc + 2 (interleaved: blocks that
+// are skipped together then spread over the waves)
+__device__ __forceinline__ int wave_row() {
+  return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 1;
+}
+__device__ __forceinline__ int wave_col() {
+  return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >> 1;
+}
+
+// acc(r,c) += sum_q As[q*LDL + r] * Bs[q*LDL + c] over this wave's blocks
 template <typename T>
 __device__ __forceinline__ void mfma_accumulate(const T *As, const T *Bs,
                                                 typename Mfma<T>::v4 acc[2][2]) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int R0 = (wave & 1) * 32, C0 = (wave >> 1) * 32;
+  const int lane = threadIdx.x & 63;
+  const int R0 = wave_row() * 16, C0 = wave_col() * 16;
   const int li = lane & 15, lk = lane >> 4;
 #pragma unroll 4
   for (int q = 0; q < 64; q += 4) {
     const T *ar = As + (q + lk) * LDL + R0 + li;
     const T *br = Bs + (q + lk) * LDL + C0 + li;
-    const T a0 = ar[0], a1 = ar[16];
-    const T b0 = br[0], b1 = br[16];
+    const T a0 = ar[0], a1 = ar[32];
+    const T b0 = br[0], b1 = br[32];
     acc[0][0] = Mfma<T>::op(a0, b0, acc[0][0]);
     acc[0][1] = Mfma<T>::op(a0, b1, acc[0][1]);
     acc[1][0] = Mfma<T>::op(a1, b0, acc[1][0]);
@@ -126,11 +137,54 @@ __device__ __forceinline__ void mfma_accumulate(const T *As, const T *Bs,
   }
 }
 
+// the same without the blocks that m (TilePair) says are zero: their products
+// add zeros, so the sums keep their bits.  The factor's tiles are half empty
+// at this granularity where separators and the interface meet (16^3 Poisson
+// subdomains: 0.50 of the block products of the factorization and 0.62 of the
+// Schur update are nonzero, 0.62 / 0.69 for the busiest wave of a product).
+// 512 of them: interior factorization 44.2 -> 38.1 ms, its GEMM launches
+// 24.2 -> 20.4, Schur update 14.6 -> 12.2; on FP32 tiles 23.1 -> 21.3, 11.8 ->
+// 10.1 and 7.0 -> 5.9.  Each block product reads its own operands from LDS:
+// keeping a second, shared-read loop for full tiles beside it costs the FP64
+// kernels 16 spilled registers and the whole gain (46.3 ms).
+template <typename T>
+__device__ __forceinline__ void mfma_accumulate(const T *As, const T *Bs,
+                                                typename Mfma<T>::v4 acc[2][2], uint32_t m) {
+  const int lane = threadIdx.x & 63;
+  const int wr = wave_row(), wc = wave_col();
+  const int li = lane & 15, lk = lane >> 4;
+  uint32_t ma = m >> wr, mb = m >> (16 + wc);
+  const T *ar = As + lk * LDL + wr * 16 + li, *br = Bs + lk * LDL + wc * 16 + li;
+#pragma unroll 1
+  for (int k = 0; k < 4; k++, ma >>= 4, mb >>= 4, ar += 16 * LDL, br += 16 * LDL) {
+    const bool a0 = ma & 1, a1 = ma & 4, b0 = mb & 1, b1 = mb & 4;
+    if (a0 && b0) {
+#pragma unroll
+      for (int q = 0; q < 16 * LDL; q += 4 * LDL) acc[0][0] = Mfma<T>::op(ar[q], br[q], acc[0][0]);
+    }
+    if (a0 && b1) {
+#pragma unroll
+      for (int q = 0; q < 16 * LDL; q += 4 * LDL) acc[0][1] = Mfma<T>::op(ar[q], br[q + 32], acc[0][1]);
+    }
+    if (a1 && b0) {
+#pragma unroll
+      for (int q = 0; q < 16 * LDL; q += 4 * LDL) acc[1][0] = Mfma<T>::op(ar[q + 32], br[q], acc[1][0]);
+    }
+    if (a1 && b1) {
+#pragma unroll
+      for (int q = 0; q < 16 * LDL; q += 4 * LDL) acc[1][1] = Mfma<T>::op(ar[q + 32], br[q + 32], acc[1][1]);
+    }
+  }
+}
+// masks of a lower triangular operand X in the post multiplies: X(c, q) as B,
+// X(r, q) as A, X(q, r) as A
+constexpr uint32_t kLowerB = 0x8CEFFFFFu, kLowerA = 0xFFFF8CEFu, kLowerTA = 0xFFFFF731u;
+
 // tile coordinates of accumulator (bi, bj, v) of this lane
 template <typename T> __device__ __forceinline__ void acc_coord(int bi, int bj, int v, int &r, int &c) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  r = (wave & 1) * 32 + bi * 16 + Mfma<T>::row(lane, v);
-  c = (wave >> 1) * 32 + bj * 16 + (lane & 15);
+  const int lane = threadIdx.x & 63;
+  r = wave_row() * 16 + bi * 32 + Mfma<T>::row(lane, v);
+  c = wave_col() * 16 + bj * 32 + (lane & 15);
 }
 
 template <typename T> __device__ __forceinline__ void zero_acc(typename Mfma<T>::v4 acc[2][2]) {
@@ -143,7 +197,7 @@ template <typename T> __device__ __forceinline__ void zero_acc(typename Mfma<T>:
 // acc = sum over pairs of opA(A) opB(B) in the "r,q x c,q" form.  Software
 // pipelined two pairs deep: the tiles of pairs p+1 and p+2 are in flight in
 // registers while the matrix cores work on pair p from LDS.
-template <typename T>
+template <typename T, bool SKIP>
 __device__ __forceinline__ void gemm_sum(const T *__restrict__ pool, const TilePair *pairs, int p0,
                                          int p1, int base, int kind, T *As, T *Bs,
                                          typename Mfma<T>::v4 acc[2][2]) {
@@ -152,29 +206,33 @@ __device__ __forceinline__ void gemm_sum(const T *__restrict__ pool, const TileP
   const T *pb = pool + (size_t)base * TILE_ELEMS;
   if (p0 >= p1) return;
   TileRegs<T> ra0, rb0, ra1, rb1;
-  auto load = [&](int p, TileRegs<T> &ra, TileRegs<T> &rb) {
+  uint32_t m0 = 0, m1 = 0;
+  auto load = [&](int p, TileRegs<T> &ra, TileRegs<T> &rb, uint32_t &m) {
     const TilePair pr = pairs[p];
     tile_load(pb + (size_t)pr.a * TILE_ELEMS, ra);
     tile_load(pb + (size_t)pr.b * TILE_ELEMS, rb);
+    m = pr.m;
   };
   // one pair from registers: to LDS, refill the registers with pair p + 2,
   // multiply
-  auto step = [&](int p, TileRegs<T> &ra, TileRegs<T> &rb) {
+  auto step = [&](int p, TileRegs<T> &ra, TileRegs<T> &rb, uint32_t &mr) {
     __syncthreads();
     tile_store_lds(ra, As, ta);
     tile_store_lds(rb, Bs, tb);
     __syncthreads();
-    if (p + 2 < p1) load(p + 2, ra, rb);
-    mfma_accumulate<T>(As, Bs, acc);
+    const uint32_t m = mr;
+    if (p + 2 < p1) load(p + 2, ra, rb, mr);
+    if constexpr (SKIP) mfma_accumulate<T>(As, Bs, acc, m);
+    else mfma_accumulate<T>(As, Bs, acc);
   };
-  load(p0, ra0, rb0);
-  if (p0 + 1 < p1) load(p0 + 1, ra1, rb1);
+  load(p0, ra0, rb0, m0);
+  if (p0 + 1 < p1) load(p0 + 1, ra1, rb1, m1);
   int p = p0;
   for (; p + 1 < p1; p += 2) {
-    step(p, ra0, rb0);
-    step(p + 1, ra1, rb1);
+    step(p, ra0, rb0, m0);
+    step(p + 1, ra1, rb1, m1);
   }
-  if (p < p1) step(p, ra0, rb0);
+  if (p < p1) step(p, ra0, rb0, m0);
 }
 
 // E = alpha*C + beta*acc, left in As as element (r,c) at c*LDL + r
@@ -213,14 +271,14 @@ __device__ __forceinline__ void acc_to_lds(typename Mfma<T>::v4 acc[2][2], T *As
       }
 }
 
-template <typename T>
+template <typename T, bool SKIP>
 __device__ __forceinline__ void tile_gemm_task_lds(T *__restrict__ pool, const TileTask t,
                                                    const TilePair *__restrict__ pairs, int kind,
                                                    int post, double alpha, double beta, T *As,
                                                    T *Bs) {
   typename Mfma<T>::v4 acc[2][2];
   zero_acc<T>(acc);
-  gemm_sum<T>(pool, pairs, t.p0, t.p1, t.base, kind, As, Bs, acc);
+  gemm_sum<T, SKIP>(pool, pairs, t.p0, t.p1, t.base, kind, As, Bs, acc);
   T *C = pool + (size_t)t.c * TILE_ELEMS;
   form_e<T>(C, t.fresh ? 0.0 : alpha, beta, acc, As);  // E in As
   if (post == POST_NONE) {
@@ -243,19 +301,23 @@ __device__ __forceinline__ void tile_gemm_task_lds(T *__restrict__ pool, const T
   }
   __syncthreads();
   zero_acc<T>(acc);
-  mfma_accumulate<T>(As, Bs, acc);
+  if constexpr (SKIP)
+    mfma_accumulate<T>(As, Bs, acc,
+                       post == POST_RIGHT_XT ? kLowerB : post == POST_LEFT_X ? kLowerA : kLowerTA);
+  else
+    mfma_accumulate<T>(As, Bs, acc);
   __syncthreads();
   acc_to_lds<T>(acc, As);
   __syncthreads();
   lds_to_tile(As, C);
 }
-template <typename T>
+template <typename T, bool SKIP>
 __device__ __forceinline__ void tile_gemm_task(T *__restrict__ pool, const TileTask t,
                                                const TilePair *__restrict__ pairs, int kind,
                                                int post, double alpha, double beta) {
   __shared__ T As[64 * LDL];
   __shared__ T Bs[64 * LDL];
-  tile_gemm_task_lds<T>(pool, t, pairs, kind, post, alpha, beta, As, Bs);
+  tile_gemm_task_lds<T, SKIP>(pool, t, pairs, kind, post, alpha, beta, As, Bs);
 }
 
 // Logical task of this workgroup.  Workgroups reach the 8 XCDs round-robin
@@ -272,33 +334,33 @@ __device__ __forceinline__ int task_index(int chunked) {
 static int g_task_order = 1;
 void set_task_order(int chunked) { g_task_order = chunked != 0; }
 
-template <typename T>
-__global__ __launch_bounds__(NTHR) void k_tile_gemm(T *__restrict__ pool,
+template <typename T, bool SKIP>
+__global__ __launch_bounds__(NTHR, Mfma<T>::WPS) void k_tile_gemm(T *__restrict__ pool,
                                                     const TileTask *__restrict__ tasks,
                                                     const TilePair *__restrict__ pairs, int kind,
                                                     int post, double alpha, double beta,
                                                     int chunked) {
   const TileTask t = tasks[task_index(chunked)];
-  if (t.mode >= 0)
-    tile_gemm_task<T>(pool, t, pairs, t.mode & 3, (t.mode >> 2) & 3, 1.0, (t.mode & 16) ? -1.0 : 0.0);
-  else
-    tile_gemm_task<T>(pool, t, pairs, kind, post, alpha, beta);
+  // (one call: the sums and the post multiply are inlined once)
+  const bool own = t.mode >= 0;
+  tile_gemm_task<T, SKIP>(pool, t, pairs, own ? t.mode & 3 : kind, own ? (t.mode >> 2) & 3 : post,
+                    own ? 1.0 : alpha, own ? ((t.mode & 16) ? -1.0 : 0.0) : beta);
 }
 
 // the Schur-complement block update S = A22 - sum W^T W in a launch of its
 // own symbol, so that profiles separate it from the factorization steps
-__global__ __launch_bounds__(NTHR) void k_schur_gemm(double *__restrict__ pool,
+__global__ __launch_bounds__(NTHR, 2) void k_schur_gemm(double *__restrict__ pool,
                                                      const TileTask *__restrict__ tasks,
                                                      const TilePair *__restrict__ pairs,
                                                      int chunked) {
-  tile_gemm_task<double>(pool, tasks[task_index(chunked)], pairs, GEMM_NT, POST_NONE, 1.0, -1.0);
+  tile_gemm_task<double, true>(pool, tasks[task_index(chunked)], pairs, GEMM_NT, POST_NONE, 1.0, -1.0);
 }
 // the same update on FP32 tiles (FP32 interior factorization)
-__global__ __launch_bounds__(NTHR) void k_schur_gemm_f32(float *__restrict__ pool,
+__global__ __launch_bounds__(NTHR, 4) void k_schur_gemm_f32(float *__restrict__ pool,
                                                          const TileTask *__restrict__ tasks,
                                                          const TilePair *__restrict__ pairs,
                                                          int chunked) {
-  tile_gemm_task<float>(pool, tasks[task_index(chunked)], pairs, GEMM_NT, POST_NONE, 1.0, -1.0);
+  tile_gemm_task<float, true>(pool, tasks[task_index(chunked)], pairs, GEMM_NT, POST_NONE, 1.0, -1.0);
 }
 
 // acc += sum_{k < nk} A(r, k) B'(c, k) for one 16x16 block in the lane layout
@@ -412,7 +474,7 @@ __device__ __forceinline__ void inv16(const T *As, T *Bs, const T *dv, int c0) {
 // cores, then its panel Cholesky by one wave; then the four diagonal-block
 // inverses, one per wave, and the off-diagonal blocks of the inverse
 // (X_IJ = -inv(L_II) sum_{J<=K<I} L_IK X_KJ) on the matrix cores.
-template <typename T>
+template <typename T, bool SKIP>
 __device__ __forceinline__ void tile_potrf_task(T *__restrict__ pool, const TileTask t,
                                                 const TilePair *__restrict__ pairs,
                                                 int *__restrict__ err, T *As, T *Bs,
@@ -421,7 +483,7 @@ __device__ __forceinline__ void tile_potrf_task(T *__restrict__ pool, const Tile
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   v4 acc[2][2];
   zero_acc<T>(acc);
-  gemm_sum<T>(pool, pairs, t.p0, t.p1, t.base, GEMM_NT, As, Bs, acc);
+  gemm_sum<T, SKIP>(pool, pairs, t.p0, t.p1, t.base, GEMM_NT, As, Bs, acc);
   T *C = pool + (size_t)t.c * TILE_ELEMS;
   form_e<T>(C, t.fresh ? 0.0 : 1.0, -1.0, acc, As);  // ends with a barrier
   for (int e = tid; e < 64 * LDL; e += NTHR) Bs[e] = (T)0;
@@ -479,8 +541,8 @@ __device__ __forceinline__ void tile_potrf_task(T *__restrict__ pool, const Tile
   if (tid == 0 && bad) atomicOr(err, 1);
 }
 
-template <typename T>
-__global__ __launch_bounds__(NTHR) void k_tile_potrf(T *__restrict__ pool,
+template <typename T, bool SKIP>
+__global__ __launch_bounds__(NTHR, Mfma<T>::WPS) void k_tile_potrf(T *__restrict__ pool,
                                                      const TileTask *__restrict__ tasks,
                                                      const TilePair *__restrict__ pairs,
                                                      int *__restrict__ err, int chunked) {
@@ -489,14 +551,14 @@ __global__ __launch_bounds__(NTHR) void k_tile_potrf(T *__restrict__ pool,
   __shared__ T Ts[4][16 * 17];
   __shared__ T dv[64];
   __shared__ int bad;
-  tile_potrf_task<T>(pool, tasks[task_index(chunked)], pairs, err, As, Bs, Ts, dv, bad);
+  tile_potrf_task<T, SKIP>(pool, tasks[task_index(chunked)], pairs, err, As, Bs, Ts, dv, bad);
 }
 
 // A launch whose tasks are tile products with their own mode (task_mode) or
 // tile factorizations (mode kTaskPotrf): the trailing update of one column
 // of a right-looking Cholesky together with the factorization of the next
 // diagonal tile, whose update is among the tasks
-__global__ __launch_bounds__(NTHR) void k_tile_step(double *__restrict__ pool,
+__global__ __launch_bounds__(NTHR, 2) void k_tile_step(double *__restrict__ pool,
                                                     const TileTask *__restrict__ tasks,
                                                     const TilePair *__restrict__ pairs,
                                                     int *__restrict__ err, int chunked) {
@@ -507,9 +569,9 @@ __global__ __launch_bounds__(NTHR) void k_tile_step(double *__restrict__ pool,
   __shared__ int bad;
   const TileTask t = tasks[task_index(chunked)];
   if (t.mode == kTaskPotrf)
-    tile_potrf_task<double>(pool, t, pairs, err, As, Bs, Ts, dv, bad);
+    tile_potrf_task<double, false>(pool, t, pairs, err, As, Bs, Ts, dv, bad);
   else
-    tile_gemm_task_lds<double>(pool, t, pairs, t.mode & 3, (t.mode >> 2) & 3, 1.0,
+    tile_gemm_task_lds<double, false>(pool, t, pairs, t.mode & 3, (t.mode >> 2) & 3, 1.0,
                                (t.mode & 16) ? -1.0 : 0.0, As, Bs);
 }
 
@@ -603,15 +665,16 @@ void launch_zero_ranges(hipStream_t st, double *pool, const int2 *ranges, int nr
 
 template <typename T>
 void launch_tile_gemm(hipStream_t st, T *pool, const TileTask *tasks, const TilePair *pairs,
-                      int ntasks, int kind, int post, double alpha, double beta) {
+                      int ntasks, int kind, int post, double alpha, double beta, bool skip) {
   if (ntasks <= 0) return;
-  hipLaunchKernelGGL(k_tile_gemm<T>, dim3(ntasks), dim3(NTHR), 0, st, pool, tasks, pairs, kind,
-                     post, alpha, beta, g_task_order);
+  auto k = skip ? k_tile_gemm<T, true> : k_tile_gemm<T, false>;
+  hipLaunchKernelGGL(k, dim3(ntasks), dim3(NTHR), 0, st, pool, tasks, pairs, kind, post, alpha,
+                     beta, g_task_order);
 }
 template void launch_tile_gemm<double>(hipStream_t, double *, const TileTask *, const TilePair *,
-                                       int, int, int, double, double);
+                                       int, int, int, double, double, bool);
 template void launch_tile_gemm<float>(hipStream_t, float *, const TileTask *, const TilePair *, int,
-                                      int, int, double, double);
+                                      int, int, double, double, bool);
 void launch_schur_gemm(hipStream_t st, double *pool, const TileTask *tasks, const TilePair *pairs,
                        int ntasks) {
   if (ntasks <= 0) return;
@@ -626,15 +689,15 @@ void launch_schur_gemm(hipStream_t st, float *pool, const TileTask *tasks, const
 }
 template <typename T>
 void launch_tile_potrf(hipStream_t st, T *pool, const TileTask *tasks, const TilePair *pairs,
-                       int ntasks, int *err) {
+                       int ntasks, int *err, bool skip) {
   if (ntasks <= 0) return;
-  hipLaunchKernelGGL(k_tile_potrf<T>, dim3(ntasks), dim3(NTHR), 0, st, pool, tasks, pairs, err,
-                     g_task_order);
+  auto k = skip ? k_tile_potrf<T, true> : k_tile_potrf<T, false>;
+  hipLaunchKernelGGL(k, dim3(ntasks), dim3(NTHR), 0, st, pool, tasks, pairs, err, g_task_order);
 }
 template void launch_tile_potrf<double>(hipStream_t, double *, const TileTask *, const TilePair *,
-                                        int, int *);
+                                        int, int *, bool);
 template void launch_tile_potrf<float>(hipStream_t, float *, const TileTask *, const TilePair *, int,
-                                       int *);
+                                       int *, bool);
 void launch_tile_step(hipStream_t st, double *pool, const TileTask *tasks, const TilePair *pairs,
                       int ntasks, int *err) {
   if (ntasks <= 0) return;

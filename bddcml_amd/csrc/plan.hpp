@@ -142,6 +142,9 @@ constexpr int task_mode(int kind, int post, bool minus) { return kind | post << 
 constexpr int kTaskPotrf = 64;
 struct TilePair {
   int a, b;
+  // 16 x 16 blocks of the operands that may be nonzero, for products A B^T:
+  // bit 4 k + r of the low half: block (r, k) of A; of the high half: of B
+  uint32_t m = 0xFFFFFFFFu;
 };
 
 struct TaskList {

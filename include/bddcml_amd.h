@@ -55,7 +55,8 @@ int bddcml_amd_residual_history(double *out, int maxn);
  * and algorithmic bytes of one local preconditioner launch; seconds of the
  * next levels' setup; the GEMM launches of the interior factorization
  * (k_tile_gemm on FP64 tiles): summed event milliseconds, summed algorithmic
- * flops (2*64^3 per tile product, post multiplies included) and their number;
+ * flops (2*16^3 per product of two 16 x 16 blocks that is computed, post
+ * multiplies included) and their number;
  * with refinement: corrections solved, final relative interface residual,
  * wall seconds of the refinement, event milliseconds and algorithmic bytes of
  * one FP64 residual launch */
