@@ -307,6 +307,7 @@ struct Device {
   std::vector<SubTiles> sub;
   // setup phases
   std::vector<Phase> a_diag, a_off, p_diag, p_off, z_bwd, w_rows;
+  std::vector<Phase> a_upd, p_upd, z_upd, w_upd;  // behind a step (split_steps), most empty
   // explicit interior inverse (levels below the first): its formation steps,
   // the four GEMV lists of the interior solves, their work vectors
   bool xint = false;
@@ -949,6 +950,14 @@ static void check_tasks(const TaskList &l, int64_t ntiles, bool uses_x, const ch
     if (bad(p.a) || bad(p.b)) fatal("BDDCML_DEVICE_PLAN", std::string("invalid tile pair in ") + what);
 }
 
+// workgroups of a product launch that the chip holds at once (two of FP64,
+// four of FP32 per CU)
+constexpr int kResident64 = 512, kResident32 = 1024;
+template <typename T>
+static void launch_update(hipStream_t st, T *pool, const Phase &u, bool skip) {
+  launch_tile_gemm(st, pool, u.tasks.p, u.pairs.p, u.ntask, GEMM_NT, POST_NONE, 1.0, -1.0, skip);
+}
+
 static void upload_phases(std::vector<Phase> &dst, const std::vector<TaskList> &src, Arena &a) {
   dst.resize(src.size());
   for (size_t k = 0; k < src.size(); k++) dst[k].upload(src[k], a);
@@ -1022,6 +1031,101 @@ static std::vector<TaskList> merge_steps(const std::vector<Q> &sts, std::vector<
         [&](const Q &q) -> const TaskList * { return k < (q.*member).size() ? &(q.*member)[k] : nullptr; },
         cls, base_of);
   return out;
+}
+
+// ---- left-looking steps cut into chunks.  A task of a left-looking sequence
+// (tile Cholesky, sweeps, inverse by rows) sums its products one after the
+// other, and the later the step the longer its sums and the fewer its tasks.
+// Once a step no longer fills the chip, the sums are that step's time.  The
+// steps from there on are cut into chunks: behind the last step of a chunk one
+// launch adds its products to every tile that later steps write, all tiles
+// and subdomains at once, and a task keeps the products of its own chunk.
+//
+// A product takes a workgroup about 3.5 us (FP64, alone on a CU or one of two),
+// so a sum of 46 was 160 us with 5 to 70 workgroups running.  36 uneven boxes
+// (up to 49 tile rows): interface phase 22.3 -> 14.8 ms, interior GEMM launches
+// 5.6 -> 4.5; 64 subdomains of 16^3 (24 rows): 7.2 -> 5.8 and 3.1 -> 2.8; 27:
+// 5.2 -> 3.4 and 1.7 -> 1.3; 512, whose steps fill the chip, unchanged.
+// Chunks of 2 steps move more tiles per product (boxes 16.9 ms), of 8 leave
+// longer sums (15.2; 64 subdomains 6.0).  An interface step counts as too small
+// below one round of resident workgroups (four rounds: boxes 16.9 ms, its
+// updates cover all rows behind it), an interior one, with few columns
+// behind it, below four (one round: 5.1 and 3.1 ms).
+constexpr int kChunk = 4;
+template <class Q>
+static std::vector<int> step_chunks(const std::vector<Q> &sts, std::vector<TaskList> Q::*member,
+                                    const std::vector<int> &cls, size_t full) {
+  std::vector<size_t> count(sts.size(), 0);
+  for (int c : cls) count[c]++;
+  size_t nsteps = 0;
+  for (auto &q : sts) nsteps = std::max(nsteps, (q.*member).size());
+  std::vector<int> chunk(nsteps, 0);
+  int c = 0, first = 0;
+  for (size_t l = 0; l < nsteps; l++) {
+    size_t tasks = 0;
+    for (size_t k = 0; k < sts.size(); k++)
+      if (l < (sts[k].*member).size()) tasks += count[k] * (sts[k].*member)[l].tasks.size();
+    if ((int)l - first >= kChunk && tasks < full) c++, first = (int)l;
+    chunk[l] = c;
+  }
+  return chunk;
+}
+// moves the products of earlier chunks out of the tasks of `lists` (the lists
+// of a step run in this order) into upd[l], launched behind step l
+static void split_steps(const std::vector<std::vector<TaskList> *> &lists, int kind,
+                        const std::vector<int> &chunk, std::vector<TaskList> &upd) {
+  size_t nsteps = 0;
+  int ntile = 0;
+  for (auto *v : lists) {
+    nsteps = std::max(nsteps, v->size());
+    for (const TaskList &L : *v)
+      for (const TileTask &t : L.tasks) ntile = std::max(ntile, t.c + 1);
+  }
+  if (nsteps == 0 || chunk[nsteps - 1] == 0) return;
+  std::vector<int> step(ntile, -1), last(chunk.back() + 1, 0);
+  for (size_t l = 0; l < chunk.size(); l++) last[chunk[l]] = (int)l;
+  for (auto *v : lists)
+    for (size_t l = 0; l < v->size(); l++)
+      for (const TileTask &t : (*v)[l].tasks) step[t.c] = std::max(step[t.c], (int)l);
+  upd.resize(nsteps);
+  std::vector<std::vector<TilePair>> part(chunk.back() + 1);
+  for (size_t l = 0; l < nsteps; l++) {
+    const int own = chunk[l];
+    if (own == 0) continue;
+    for (auto *v : lists) {
+      if (l >= v->size()) continue;
+      TaskList out;
+      for (TileTask t : (*v)[l].tasks) {
+        const TaskList &L = (*v)[l];
+        for (int p = t.p0; p < t.p1; p++) {
+          const TilePair &q = L.pairs[p];
+          const int src = std::max(q.a < ntile ? step[q.a] : -1, q.b < ntile ? step[q.b] : -1);
+          part[src < 0 ? own : chunk[src]].push_back(q);
+        }
+        const bool plain = t.mode >= 0 && t.mode != kTaskPotrf && ((t.mode >> 2) & 3) == POST_NONE;
+        bool moved = false;
+        for (int c = 0; c < own; c++) {
+          if (part[c].empty()) continue;
+          TaskList &U = upd[last[c]];
+          TileTask u{t.c, -1, (int)U.pairs.size(), 0};
+          U.pairs.insert(U.pairs.end(), part[c].begin(), part[c].end());
+          u.p1 = (int)U.pairs.size();
+          u.fresh = std::exchange(t.fresh, 0);
+          u.mode = task_mode(t.mode >= 0 ? t.mode & 3 : kind, POST_NONE, true);
+          U.tasks.push_back(u);
+          part[c].clear();
+          moved = true;
+        }
+        t.p0 = (int)out.pairs.size();
+        out.pairs.insert(out.pairs.end(), part[own].begin(), part[own].end());
+        t.p1 = (int)out.pairs.size();
+        part[own].clear();
+        if (moved && plain && t.p0 == t.p1) continue;  // a partial sum, moved whole
+        out.tasks.push_back(t);
+      }
+      (*v)[l] = std::move(out);
+    }
+  }
 }
 
 // work done: 2*64^3 flops per tile product, 64^3/3 per tile Cholesky plus
@@ -1161,7 +1265,7 @@ void device_setup_begin(Solver &S) {
   const std::vector<int> &cls = S.ord_cls, &reps = S.ord_reps;
   const int ncls = (int)reps.size();
   struct SubTasks {
-    std::vector<TaskList> a_diag, a_off;
+    std::vector<TaskList> a_diag, a_off, a_upd;
     std::vector<TaskList> m_rows;  // explicit interior inverse, one step per tile row
     TaskList a_schur;
     std::vector<int> clear;  // pattern tiles (relative) that start as zeros
@@ -1491,8 +1595,15 @@ void device_setup_begin(Solver &S) {
   HIPCHECK(hipGetLastError());
   ph("scatter launched");
   auto base_of = [&](int is) { return D.sub[is].base; };
+  const std::vector<int> chunk =
+      step_chunks(sts, &SubTasks::a_off, cls, 4 * (D.f32i ? kResident32 : kResident64));
+#pragma omp parallel for schedule(dynamic)
+  for (int k = 0; k < ncls; k++)
+    split_steps({&sts[k].a_diag, &sts[k].a_off}, GEMM_NT, chunk, sts[k].a_upd);
   std::vector<TaskList> a_diag = merge_steps(sts, &SubTasks::a_diag, cls, base_of),
-                        a_off = merge_steps(sts, &SubTasks::a_off, cls, base_of);
+                        a_off = merge_steps(sts, &SubTasks::a_off, cls, base_of),
+                        a_upd = merge_steps(sts, &SubTasks::a_upd, cls, base_of);
+  a_upd.resize(a_off.size());
   TaskList a_schur = materialize(
       sts, [](const SubTasks &Q) -> const TaskList * { return &Q.a_schur; }, cls, base_of);
   std::vector<TaskList> m_rows;
@@ -1504,6 +1615,7 @@ void device_setup_begin(Solver &S) {
                 nsub, a_diag.size());
   upload_phases(D.a_diag, a_diag, D.plan);
   upload_phases(D.a_off, a_off, D.plan);
+  upload_phases(D.a_upd, a_upd, D.plan);
   D.a_schur.upload(a_schur, D.plan);
   if (D.xint) {
     upload_phases(D.m_rows, m_rows, D.plan);
@@ -1591,14 +1703,15 @@ void device_setup_begin(Solver &S) {
 
   S.t.schur_flops = kTileGemm * tile_products(a_schur);
   S.t.interior_flops = tile_work(a_diag, 2 * kTileChol) + tile_work(a_off, kTilePost) +
-                       tile_work(m_rows, kTileGemm) + S.t.schur_flops;
+                       tile_work(a_upd, 0.0) + tile_work(m_rows, kTileGemm) + S.t.schur_flops;
   // ---- numerics, first half: Dirichlet elimination into the tiles,
   // interior factorization, Schur complements
   D.ev_gemm.assign(2 * D.a_off.size(), nullptr);
   for (hipEvent_t &e : D.ev_gemm) HIPCHECK(hipEventCreate(&e));
   D.gemm_flops.clear();
-  for (const TaskList &l : a_off)
-    D.gemm_flops.push_back(kTileGemm * tile_products(l) + kTilePost * posted_tasks(l));
+  for (size_t l = 0; l < a_off.size(); l++)
+    D.gemm_flops.push_back(kTileGemm * (tile_products(a_off[l]) + tile_products(a_upd[l])) +
+                           kTilePost * posted_tasks(a_off[l]));
   HIPCHECK(hipEventCreateWithFlags(&D.ev_up, hipEventDisableTiming));
   HIPCHECK(hipEventCreateWithFlags(&D.ev_rhs, hipEventDisableTiming));
   // element type of the subdomain tiles: FP64, or FP32 with refinement
@@ -1609,6 +1722,7 @@ void device_setup_begin(Solver &S) {
       HIPCHECK(hipEventRecord(D.ev_gemm[2 * J], st));
       launch_tile_gemm(st, pool, D.a_off[J].tasks.p, D.a_off[J].pairs.p, D.a_off[J].ntask, GEMM_NT,
                        POST_RIGHT_XT, 1.0, -1.0, true);
+      launch_update(st, pool, D.a_upd[J], true);
       HIPCHECK(hipEventRecord(D.ev_gemm[2 * J + 1], st));
     }
     HIPCHECK(hipEventRecord(ev[1], st));
@@ -1644,9 +1758,11 @@ static void form_inverse(Solver &S) {
   hipStream_t st = D.st;
   auto run = [&](auto *fp) {
     constexpr bool skip = skip_interface<decltype(fp)>;
-    for (size_t i = 0; i < D.w_rows.size(); i++)
+    for (size_t i = 0; i < D.w_rows.size(); i++) {
       launch_tile_gemm(st, fp, D.w_rows[i].tasks.p, D.w_rows[i].pairs.p, D.w_rows[i].ntask, GEMM_NN,
                        POST_LEFT_X, 1.0, -1.0, skip);
+      launch_update(st, fp, D.w_upd[i], skip);
+    }
     launch_tile_gemm(st, fp, D.kinv.tasks.p, D.kinv.pairs.p, D.kinv.ntask, GEMM_TN, POST_NONE, 1.0,
                      1.0);
   };
@@ -1767,16 +1883,15 @@ static double interface_rho(const Sub &s) {
 // rows n of each subdomain's S', its factor's element size).  The constants
 // were fitted on one MI355X over Poisson, elasticity and uneven boxes, 8 to
 // 512 subdomains, n = 1 to 76:
-//  - forming: tile products at 50 / 95 TFLOP/s (FP64 / FP32) behind one
-//    launch per tile row (10 us) whose longest task is a chain of products
-//    (2.6 / 1.9 us each);
+//  - forming: tile products at 50 / 95 TFLOP/s (FP64 / FP32) and, per tile
+//    row, 40 us of launches with too few workgroups;
 //  - an apply by sweeps: the larger of the slowest workgroup (3.4 us per
 //    tile row and direction, 0.7 / 0.4 us per tile) and both reads of the
-//    factors at 5.5 TB/s; by the inverse: one read at 4.7 TB/s and 15 us.
-// FP64, ms formed / sweeps / inverse: 64 subdomains n = 25: 2.9 / 0.60 / 0.10
-// (pays after 6); 36 boxes n <= 49: 8.7 / 2.25 / 0.17 (4); 60 boxes n <= 76:
-// 35.6 / 5.1 / 0.50 (8); 216 subdomains n = 25: 9.5 / 0.76 / 0.36 (23); 512:
-// 24 / 1.57 / 0.92 (37).
+//    factors at 5.5 TB/s; by the inverse: one read at 5.9 TB/s and 15 us.
+// FP64, ms formed / sweeps / inverse: 64 subdomains n = 25: 2.8 / 0.57 / 0.08
+// (pays after 6); 36 boxes n <= 49: 7.6 / 2.19 / 0.12 (4); 60 boxes n <= 76:
+// 34.9 / 4.9 / 0.51 (8); 216 subdomains n = 25: 9.7 / 0.76 / 0.28 (20); 512:
+// 24.6 / 1.64 / 0.73 (27).
 static double inverse_pays_after(const std::vector<SubTiles> &sub, bool f32) {
   double prods = 0.0, tiles = 0.0;
   int nmax = 0;
@@ -1787,11 +1902,10 @@ static double inverse_pays_after(const std::vector<SubTiles> &sub, bool f32) {
     nmax = std::max(nmax, T.nti);
   }
   const double n = nmax, bytes = tiles * TILE_ELEMS * (f32 ? 4.0 : 8.0);
-  const double form = prods * kTileGemm / (f32 ? 95e12 : 50e12) + n * 10e-6 +
-                      0.5 * n * (n - 1.0) * (f32 ? 1.9e-6 : 2.6e-6);
+  const double form = prods * kTileGemm / (f32 ? 95e12 : 50e12) + n * 40e-6;
   const double sweeps = std::max(2.0 * n * 3.4e-6 + n * (n + 1.0) * (f32 ? 0.4e-6 : 0.7e-6),
                                  2.0 * bytes / 5.5e12);
-  const double saved = sweeps - (bytes / 4.7e12 + 15e-6);
+  const double saved = sweeps - (bytes / 5.9e12 + 15e-6);
   return saved > 0.0 ? form / saved : 1e30;
 }
 // a solve rarely takes fewer applies than this: an inverse that pays for
@@ -1871,7 +1985,7 @@ void device_setup_interface(Solver &S) {
       fcls[is] = it->second;
     }
     struct FactorTasks {
-      std::vector<TaskList> p_diag, p_off, z_bwd, w_rows;
+      std::vector<TaskList> p_diag, p_off, z_bwd, w_rows, p_upd, z_upd, w_upd;
       TaskList phi, kinv;
     };
     std::vector<FactorTasks> fts(fkeys.size());
@@ -1949,27 +2063,47 @@ void device_setup_interface(Solver &S) {
       if (D.sub[is].fbase < 0 || (int64_t)D.sub[is].fbase + D.sub[is].fspan > D.ntilesf)
         fatal("BDDCML_DEVICE_PLAN", "factor tile range");
     auto fbase_of = [&](int is) { return D.sub[is].fbase; };
+    const size_t resident = D.mixed ? kResident32 : kResident64;
+    const std::vector<int> pch = step_chunks(fts, &FactorTasks::p_off, fcls, resident),
+                           zch = step_chunks(fts, &FactorTasks::z_bwd, fcls, resident),
+                           wch = step_chunks(fts, &FactorTasks::w_rows, fcls, resident);
+#pragma omp parallel for schedule(dynamic)
+    for (int k = 0; k < (int)fts.size(); k++) {
+      FactorTasks &Q = fts[k];
+      split_steps({&Q.p_diag, &Q.p_off}, GEMM_NT, pch, Q.p_upd);
+      split_steps({&Q.z_bwd}, GEMM_TN, zch, Q.z_upd);
+      split_steps({&Q.w_rows}, GEMM_NN, wch, Q.w_upd);
+    }
     std::vector<TaskList> p_diag = merge_steps(fts, &FactorTasks::p_diag, fcls, fbase_of),
                           p_off = merge_steps(fts, &FactorTasks::p_off, fcls, fbase_of),
                           z_bwd = merge_steps(fts, &FactorTasks::z_bwd, fcls, fbase_of);
+    std::vector<TaskList> p_upd = merge_steps(fts, &FactorTasks::p_upd, fcls, fbase_of),
+                          z_upd = merge_steps(fts, &FactorTasks::z_upd, fcls, fbase_of);
+    p_upd.resize(p_off.size()), z_upd.resize(z_bwd.size());
     TaskList phi = materialize(
         fts, [](const FactorTasks &Q) -> const TaskList * { return &Q.phi; }, fcls, fbase_of);
-    std::vector<TaskList> w_rows = merge_steps(fts, &FactorTasks::w_rows, fcls, fbase_of);
+    std::vector<TaskList> w_rows = merge_steps(fts, &FactorTasks::w_rows, fcls, fbase_of),
+                          w_upd = merge_steps(fts, &FactorTasks::w_upd, fcls, fbase_of);
+    w_upd.resize(w_rows.size());
     TaskList kinv = materialize(
         fts, [](const FactorTasks &Q) -> const TaskList * { return &Q.kinv; }, fcls, fbase_of);
     // the explicit inverse's rows and product count only where the setup
     // forms it (option 1); the automatic mode forms it during a solve
     S.t.interface_flops = tile_work(p_diag, 2 * kTileChol) + tile_work(p_off, kTileGemm) +
-                          tile_work(z_bwd, kTileGemm) +
-                          kTileGemm * tile_products(phi);
+                          tile_work(z_bwd, kTileGemm) + tile_work(p_upd, 0.0) +
+                          tile_work(z_upd, 0.0) + kTileGemm * tile_products(phi);
     if (D.inv_planned && !D.inv_auto)
-      S.t.interface_flops += tile_work(w_rows, kTileGemm) + kTileGemm * tile_products(kinv);
+      S.t.interface_flops += tile_work(w_rows, kTileGemm) + tile_work(w_upd, 0.0) +
+                             kTileGemm * tile_products(kinv);
     D.plan2.verbose = S.verbose;
     upload_phases(D.p_diag, p_diag, D.plan2);
     upload_phases(D.p_off, p_off, D.plan2);
     upload_phases(D.z_bwd, z_bwd, D.plan2);
+    upload_phases(D.p_upd, p_upd, D.plan2);
+    upload_phases(D.z_upd, z_upd, D.plan2);
     D.phi.upload(phi, D.plan2);
     upload_phases(D.w_rows, w_rows, D.plan2);
+    upload_phases(D.w_upd, w_upd, D.plan2);
     D.kinv.upload(kinv, D.plan2);
   }
   {
@@ -2220,10 +2354,13 @@ void device_setup_interface(Solver &S) {
       launch_tile_potrf(st, fp, D.p_diag[J].tasks.p, D.p_diag[J].pairs.p, D.p_diag[J].ntask, D.err.p);
       launch_tile_gemm(st, fp, D.p_off[J].tasks.p, D.p_off[J].pairs.p, D.p_off[J].ntask, GEMM_NT,
                        POST_RIGHT_XT, 1.0, -1.0, skip_interface<decltype(fp)>);
+      launch_update(st, fp, D.p_upd[J], skip_interface<decltype(fp)>);
     }
-    for (size_t i = 0; i < D.z_bwd.size(); i++)
+    for (size_t i = 0; i < D.z_bwd.size(); i++) {
       launch_tile_gemm(st, fp, D.z_bwd[i].tasks.p, D.z_bwd[i].pairs.p, D.z_bwd[i].ntask, GEMM_TN,
                        POST_LEFT_XT, 1.0, -1.0, skip_interface<decltype(fp)>);
+      launch_update(st, fp, D.z_upd[i], skip_interface<decltype(fp)>);
+    }
     launch_y_to_z(st, fp, D.desc.p, nsub, D.Z.p, D.maxNI, 0);
   };
   // Phi = Z G^{-1} on the tile GEMM, in the factor space

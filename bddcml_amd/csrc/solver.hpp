@@ -69,7 +69,7 @@ struct Solver {
   // tile GEMV) instead of two sweeps over the factor of S': 0 never, 1 formed
   // at setup, 2 (the default) formed at setup where about eight applies pay
   // for it (few or large subdomains), else once as many applies as pay for it
-  // have run on the same setup (many equal subdomains: about 40)
+  // have run on the same setup (many equal subdomains: about 30)
   int explicit_inverse = 2;
   // levels below the first: interior solves of the level's apply through the
   // explicit inverse of the interior factor (tile GEMVs) instead of sweeps

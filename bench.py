@@ -230,7 +230,7 @@ def main():
     ap.add_argument("--nsub2", type=int, default=8, help="subdomains of the second level")
     ap.add_argument("--explicit-inverse", type=int, default=2, choices=(0, 1, 2),
                     help="explicit inverse of S' for the local preconditioner: 0 never, 1 at "
-                         "setup, 2 after 40 applies (the library's default)")
+                         "setup, 2 once applies have paid for it (the library's default)")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--set", action="append", default=[], metavar="KEY=VALUE",
                     help="further library option (bddcml_amd_set_option), repeatable")
