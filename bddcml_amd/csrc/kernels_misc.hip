@@ -511,7 +511,19 @@ __device__ __forceinline__ double row_reduce(double s, double *red) {
 // wave are published to the others with a workgroup fence before the barrier.
 // P: element type of the factor tiles (FP64, or FP32 with the FP32 interior
 // factorization); the vector and the sums stay FP64.
-template <typename P, int NW, bool GV>
+// Tile entries are read once per sweep; with more than one workgroup per CU
+// the sweeps are bound by HBM, where nontemporal loads reach 6.0 TB/s and
+// plain ones 5.5 (512 subdomains of 16^3, forward / backward sweep 2.39 /
+// 2.31 -> 2.06 / 2.08 ms).
+template <typename P> __device__ __forceinline__ double stream_load(const P *p) {
+  return (double)__builtin_nontemporal_load(p);
+}
+
+// DEEP (16 waves, one workgroup per CU): four tiles of a row in flight and the
+// inverse diagonal tile loaded ahead of the row sum; a sweep is then bound by
+// the largest subdomain's chain of rows (64 subdomains of 16^3: 0.73 / 0.89 ->
+// 0.70 / 0.82 ms; two tiles in flight 0.80 / 0.89).
+template <typename P, int NW, bool GV, bool DEEP>
 __global__ __launch_bounds__(64 * NW) void k_trsv_fwd(const P *__restrict__ pool,
                                                   const TrsvDesc *__restrict__ ds,
                                                   const int *__restrict__ rptr,
@@ -529,13 +541,21 @@ __global__ __launch_bounds__(64 * NW) void k_trsv_fwd(const P *__restrict__ pool
   if (!GV)
     for (int k = threadIdx.x; k < nt * 64; k += blockDim.x) v[k] = gv[k];
   __syncthreads();
+  constexpr int CW = 64 / NW;  // tile columns per wave
   for (int I = 0; I < nt; I++) {
+    double lv[CW];
+    if (DEEP && I < d.nto) {
+      const P *L = pool + (size_t)(d.linv + I) * TILE_ELEMS + r;
+#pragma unroll
+      for (int m = 0; m < CW; m++) lv[m] = stream_load(L + (g + NW * m) * 64);
+    }
     double s = 0.0;
+#pragma unroll(DEEP ? 4 : NW == 16 ? 2 : 1)
     for (int q = rptr[d.rptr_off + I]; q < rptr[d.rptr_off + I + 1]; q++) {
       const P *T = pool + (size_t)rt[q] * TILE_ELEMS + r;
       const double *x = v + rk[q] * 64;
 #pragma unroll 4
-      for (int c = g; c < 64; c += NW) s += T[c * 64] * x[c];
+      for (int m = 0; m < CW; m++) s += stream_load(T + (g + NW * m) * 64) * x[g + NW * m];
     }
     double tv = row_reduce<NW>(s, red);
     if (threadIdx.x < 64) t[r] = v[I * 64 + r] - tv;
@@ -544,7 +564,8 @@ __global__ __launch_bounds__(64 * NW) void k_trsv_fwd(const P *__restrict__ pool
       const P *L = pool + (size_t)(d.linv + I) * TILE_ELEMS + r;
       double u = 0.0;
 #pragma unroll 4
-      for (int c = g; c < 64; c += NW) u += L[c * 64] * t[c];
+      for (int m = 0; m < CW; m++)
+        u += (DEEP ? lv[m] : stream_load(L + (g + NW * m) * 64)) * t[g + NW * m];
       double w = row_reduce<NW>(u, red);
       if (threadIdx.x < 64) v[I * 64 + r] = w;
     } else if (threadIdx.x < 64) {
@@ -557,7 +578,7 @@ __global__ __launch_bounds__(64 * NW) void k_trsv_fwd(const P *__restrict__ pool
     for (int k = threadIdx.x; k < nt * 64; k += blockDim.x) gv[k] = v[k];
 }
 
-template <typename P, int NW, bool GV>
+template <typename P, int NW, bool GV, bool DEEP>
 __global__ __launch_bounds__(64 * NW) void k_trsv_bwd(const P *__restrict__ pool,
                                                   const TrsvDesc *__restrict__ ds,
                                                   const int *__restrict__ cptr,
@@ -581,12 +602,19 @@ __global__ __launch_bounds__(64 * NW) void k_trsv_bwd(const P *__restrict__ pool
     // g + 16 m (m < 4) by wave reductions, every load a 512-byte column
     const int l = r;
     for (int I = d.nto - 1; I >= 0; I--) {
+      const P *L = pool + (size_t)(d.linv + I) * TILE_ELEMS + l;
+      double lv[4];
+      if (DEEP) {
+#pragma unroll
+        for (int m = 0; m < 4; m++) lv[m] = stream_load(L + (g + 16 * m) * 64);
+      }
       double a[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll(DEEP ? 4 : 2)
       for (int q = cptr[d.cptr_off + I]; q < cptr[d.cptr_off + I + 1]; q++) {
         const P *T = pool + (size_t)ct[q] * TILE_ELEMS + l;
         const double xv = v[ck[q] * 64 + l];
 #pragma unroll
-        for (int m = 0; m < 4; m++) a[m] += T[(g + 16 * m) * 64] * xv;
+        for (int m = 0; m < 4; m++) a[m] += stream_load(T + (g + 16 * m) * 64) * xv;
       }
 #pragma unroll
       for (int m = 0; m < 4; m++) a[m] = wave_sum(a[m]);
@@ -595,10 +623,10 @@ __global__ __launch_bounds__(64 * NW) void k_trsv_bwd(const P *__restrict__ pool
         for (int m = 0; m < 4; m++) t[g + 16 * m] = v[I * 64 + g + 16 * m] - a[m];
       }
       __syncthreads();
-      const P *L = pool + (size_t)(d.linv + I) * TILE_ELEMS + l;
       const double tv = t[l];
 #pragma unroll
-      for (int m = 0; m < 4; m++) a[m] = wave_sum(L[(g + 16 * m) * 64] * tv);
+      for (int m = 0; m < 4; m++)
+        a[m] = wave_sum((DEEP ? lv[m] : stream_load(L + (g + 16 * m) * 64)) * tv);
       if (l == 0) {
 #pragma unroll
         for (int m = 0; m < 4; m++) v[I * 64 + g + 16 * m] = a[m];
@@ -687,27 +715,35 @@ static void trsv_launch(hipStream_t st, int nsub, int maxnt, K1 lds_kernel, K2 g
     hipLaunchKernelGGL(gv_kernel, dim3(nsub), dim3(64 * NW), sg, st, pool, d, p, k, t, v);
   }
 }
+// one workgroup per CU at most: more tiles in flight in each (DEEP)
+static constexpr int kTrsvDeepSubs = 256;
 template <typename P>
 void launch_trsv_fwd(hipStream_t st, const P *pool, const TrsvDesc *d, int nsub, const int *rptr,
                      const int *rk, const int *rt, double *v, int maxnt) {
   if (nsub <= 0) return;
-  if (few_subdomains(nsub))
-    trsv_launch<16>(st, nsub, maxnt, k_trsv_fwd<P, 16, false>, k_trsv_fwd<P, 16, true>, pool, d,
-                    rptr, rk, rt, v);
+  if (few_subdomains(nsub) && nsub <= kTrsvDeepSubs)
+    trsv_launch<16>(st, nsub, maxnt, k_trsv_fwd<P, 16, false, true>, k_trsv_fwd<P, 16, true, true>,
+                    pool, d, rptr, rk, rt, v);
+  else if (few_subdomains(nsub))
+    trsv_launch<16>(st, nsub, maxnt, k_trsv_fwd<P, 16, false, false>,
+                    k_trsv_fwd<P, 16, true, false>, pool, d, rptr, rk, rt, v);
   else
-    trsv_launch<4>(st, nsub, maxnt, k_trsv_fwd<P, 4, false>, k_trsv_fwd<P, 4, true>, pool, d, rptr,
-                   rk, rt, v);
+    trsv_launch<4>(st, nsub, maxnt, k_trsv_fwd<P, 4, false, false>, k_trsv_fwd<P, 4, true, false>,
+                   pool, d, rptr, rk, rt, v);
 }
 template <typename P>
 void launch_trsv_bwd(hipStream_t st, const P *pool, const TrsvDesc *d, int nsub, const int *cptr,
                      const int *ck, const int *ct, double *v, int maxnt) {
   if (nsub <= 0) return;
-  if (few_subdomains(nsub))
-    trsv_launch<16>(st, nsub, maxnt, k_trsv_bwd<P, 16, false>, k_trsv_bwd<P, 16, true>, pool, d,
-                    cptr, ck, ct, v);
+  if (few_subdomains(nsub) && nsub <= kTrsvDeepSubs)
+    trsv_launch<16>(st, nsub, maxnt, k_trsv_bwd<P, 16, false, true>, k_trsv_bwd<P, 16, true, true>,
+                    pool, d, cptr, ck, ct, v);
+  else if (few_subdomains(nsub))
+    trsv_launch<16>(st, nsub, maxnt, k_trsv_bwd<P, 16, false, false>,
+                    k_trsv_bwd<P, 16, true, false>, pool, d, cptr, ck, ct, v);
   else
-    trsv_launch<4>(st, nsub, maxnt, k_trsv_bwd<P, 4, false>, k_trsv_bwd<P, 4, true>, pool, d, cptr,
-                   ck, ct, v);
+    trsv_launch<4>(st, nsub, maxnt, k_trsv_bwd<P, 4, false, false>, k_trsv_bwd<P, 4, true, false>,
+                   pool, d, cptr, ck, ct, v);
 }
 template void launch_trsv_fwd<double>(hipStream_t, const double *, const TrsvDesc *, int,
                                       const int *, const int *, const int *, double *, int);
@@ -1179,7 +1215,9 @@ __global__ __launch_bounds__(256) void k_phit(const SubDesc *__restrict__ subs,
 // per CU) -- for few or uneven subdomains, where the largest subdomain's
 // sweep is the tail.  Otherwise two tiles in flight (56 VGPRs, two
 // workgroups per CU), for many subdomains of similar size, where the
-// launch is HBM-bound as a whole.
+// launch is HBM-bound as a whole: nontemporal loads (512 subdomains of 16^3
+// 1.58 -> 1.47 ms, 6.0 TB/s; FP32 0.84 -> 0.77).  The deep form keeps plain
+// loads (64 subdomains 0.574 ms, nontemporal 0.589).
 // barrier that also publishes global-memory writes to the other waves of
 // the workgroup when the working vector lives there
 template <bool GV>
@@ -1241,7 +1279,7 @@ __global__ __launch_bounds__(KA_THR) void k_kapply(
         const T *L = pool + (size_t)(d.pbase + packed_lower(n, I, k)) * TILE_ELEMS + l;
         const double *x = xs + k * 64;
 #pragma unroll
-        for (int m = 0; m < 4; m++) s += (double)L[(g + 16 * m) * 64] * x[g + 16 * m];
+        for (int m = 0; m < 4; m++) s += stream_load(L + (g + 16 * m) * 64) * x[g + 16 * m];
       }
     }
     red[g * 64 + l] = s;
@@ -1296,7 +1334,7 @@ __global__ __launch_bounds__(KA_THR) void k_kapply(
         const T *L = pool + (size_t)(d.pbase + packed_lower(n, k, I)) * TILE_ELEMS + g * 64 + l;
         const double xv = xs[k * 64 + l];
 #pragma unroll
-        for (int m = 0; m < 4; m++) a[m] += (double)L[m * 16 * 64] * xv;
+        for (int m = 0; m < 4; m++) a[m] += stream_load(L + m * 16 * 64) * xv;
       }
     }
 #pragma unroll
