@@ -3424,9 +3424,12 @@ static void count_pc_applies(Solver &S, int add) {
     if (L->dev->inv_auto && !L->dev->explicit_inv) L->dev->pc_count += add;
 }
 
-// what a captured iteration depends on beyond the solver's fixed buffers
-static std::vector<const void *> pcg_graph_key(Solver &S, const double *rz) {
-  std::vector<const void *> key{rz, S.dev->hrr_dev};
+// what a captured iteration depends on beyond the solver's fixed buffers: all
+// three scalar arrays (kept memory may put a larger array, with other offsets
+// of pap and rr, where the smaller one was) and the preconditioner's form
+static std::vector<const void *> pcg_graph_key(Solver &S, const double *rz, const double *pap,
+                                               const double *rr) {
+  std::vector<const void *> key{rz, pap, rr, S.dev->hrr_dev};
   for (Solver *L = &S; L && L->dev; L = L->lev2.get()) {
     const Device &E = *L->dev;
     // the factor pool of the level's precision once it holds S'^{-1}
@@ -3470,7 +3473,7 @@ static void pcg_graph_capture(Solver &S, double *rz, double *pap, double *rr) {
   HIPCHECK(hipGraphInstantiate(&D.pcg_exec, D.pcg_graph, nullptr, nullptr, 0));
   int q = 0;
   for (Solver *L = &S; L && L->dev; L = L->lev2.get()) L->dev->pc_count = counts[q++];
-  D.pcg_key = pcg_graph_key(S, rz);
+  D.pcg_key = pcg_graph_key(S, rz, pap, rr);
 }
 
 // iteration k by the graph; returns once r.r of iteration k is in hrr[k]
@@ -3478,7 +3481,7 @@ static void pcg_graph_capture(Solver &S, double *rz, double *pap, double *rr) {
 static void pcg_graph_replay(Solver &S, int k, double *rz, double *pap, double *rr) {
   Device &D = *S.dev;
   hipStream_t st = D.st;
-  if (!D.pcg_exec || D.pcg_key != pcg_graph_key(S, rz)) pcg_graph_capture(S, rz, pap, rr);
+  if (!D.pcg_exec || D.pcg_key != pcg_graph_key(S, rz, pap, rr)) pcg_graph_capture(S, rz, pap, rr);
   if (k == 3) launch_count_set(st, D.kcount.p, k);  // later replays step it themselves
   volatile double *h = D.hrr + k;
   *h = -1.0;  // r.r >= 0 replaces it

@@ -72,3 +72,28 @@ def test_graph_kept_across_solves(oracle_lib):
             o2.close()
     finally:
         b.finalize()
+
+
+@pytest.mark.parametrize("steps", [(200, 300), (300, 200), (60, 120, 250, 600)])
+def test_graph_follows_a_larger_maxit(steps):
+    """Solves with another maxit on one setup: the scalars of the iterations
+    are laid out by the largest maxit so far, also where the larger array
+    comes to lie at the address of the smaller one, and the condition number
+    is formed from them.  As on a setup that sees that maxit first."""
+    _say(f"case pcg graph maxit {steps}")
+    p = CubeProblem(4, 3, rhs="random", seed=3)
+    subs = list(p.subdomains())
+    ref, (it_ref, r_ref, c_ref) = bddcml_amd.solve_cube(p, tol=1e-11, maxit=max(steps))
+    u_ref = ref.interface_solution()
+    ref.finalize()
+    assert r_ref == 0 and it_ref >= 5
+    b, (it, r, c) = bddcml_amd.solve_cube(p, tol=1e-11, maxit=steps[0])
+    for k, m in enumerate(steps):
+        if k > 0:
+            for d in subs:
+                b.change_subdomain_data(d)
+            b.setup_new_data()
+            it, r, c = b.solve(0, 1e-11, m, 50)
+        assert (it, r, c) == (it_ref, 0, c_ref), (m, it, r, c, it_ref, c_ref)
+        assert np.array_equal(b.interface_solution(), u_ref)
+    b.finalize()
