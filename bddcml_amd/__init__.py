@@ -38,7 +38,7 @@ EXTRA_SYMBOLS = [
     "bddcml_amd_selftest_ginv", "bddcml_amd_selftest_symeig",
     "bddcml_amd_selftest_copy", "bddcml_amd_element_gradient", "bddcml_amd_recycling_basis",
     "bddcml_amd_level2_counts", "bddcml_amd_level_counts", "bddcml_amd_element_gradient_noalloc",
-    "bddcml_amd_adaptive_pairs",
+    "bddcml_amd_adaptive_pairs", "bddcml_amd_inverse_state",
 ]
 
 
@@ -398,6 +398,14 @@ class Bddcml:
         n, orth = C.c_int(), C.c_double()
         self.L.bddcml_amd_recycling_basis(C.byref(n), C.byref(orth))
         return n.value, orth.value
+
+    def inverse_state(self, level=1):
+        """Explicit inverse of a level: (formed, applies counted by the
+        automatic mode, applies after which it is estimated to pay)."""
+        out = np.zeros(3)
+        if self.L.bddcml_amd_inverse_state(int(level), out.ctypes.data_as(C.POINTER(C.c_double))):
+            raise RuntimeError("no such level")
+        return bool(out[0]), int(out[1]), float(out[2])
 
     def residual_history(self):
         n = self.L.bddcml_amd_residual_history(None, 0)

@@ -787,6 +787,17 @@ int bddcml_amd_reduced_rhs(double *g) try {
 catch (const Error &e) {
   record_error(e); return -100;
 }
+int bddcml_amd_inverse_state(int ilevel, double *out) try {
+  Solver *L = &solver();
+  if (!L->is_setup || L->plan_only) return -1;
+  for (int l = 1; l < ilevel && L; l++) L = L->lev2.get();
+  if (ilevel < 1 || !L || !L->dev) return -1;
+  device_inverse_state(*L, out);
+  return 0;
+}
+catch (const Error &e) {
+  record_error(e); return -100;
+}
 int bddcml_amd_recycling_basis(int *nvec, double *orth) try {
   Solver &S = solver();
   if (!S.is_setup || S.plan_only || !S.dev) return -1;

@@ -3271,6 +3271,13 @@ static void dots(Solver &S, std::initializer_list<std::pair<const double *, cons
   HIPCHECK(hipStreamSynchronize(D.st));
 }
 
+void device_inverse_state(const Solver &S, double *out) {
+  const Device &D = *S.dev;
+  out[0] = D.explicit_inv;
+  out[1] = D.pc_count;
+  out[2] = D.inv_after;
+}
+
 void device_recycling_check(Solver &S, int *nvec, double *orth) {
   *nvec = S.rec_n;
   *orth = 0.0;

@@ -268,6 +268,8 @@ void device_solve(Solver &S, int method, double tol, int maxit, int ndecrmax, bo
                   int maxvec, int *num_iter, int *reason, double *cond);
 // stored recycling directions and ||V^T W - I||_F of the basis
 void device_recycling_check(Solver &S, int *n, double *orth);
+// explicit inverse: formed, applies counted, applies after which it pays
+void device_inverse_state(const Solver &S, double *out);
 void device_apply_schur(Solver &S, const double *x, double *y);
 void device_apply_pc(Solver &S, const double *r, double *z);
 void device_reduced_rhs_download(Solver &S, double *g);

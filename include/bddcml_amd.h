@@ -126,6 +126,11 @@ int bddcml_amd_timings(double *out, int n);
  *     the first solve after as many applies as pay for it have run on the
  *     same setup; a solve never changes its preconditioner while it runs) */
 int bddcml_amd_set_option(const char *key, double value);
+/* explicit inverse of level ilevel (1: the first): out[0] = 1 once it is
+ * formed, out[1] = preconditioner applies that the automatic mode has counted
+ * on this setup, out[2] = applies after which it is estimated to pay; returns
+ * -1 if that level has no device setup */
+int bddcml_amd_inverse_state(int ilevel, double *out);
 /* per subdomain (isub in numbase): out[0]=ndofi out[1]=nconstr out[2]=ndofo */
 int bddcml_amd_sub_info(int isub, int *out);
 /* global dof of each local interface dof (reference interface order) and

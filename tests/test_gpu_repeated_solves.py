@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 import bddcml_amd
-from bddcml_amd.cube import CubeProblem
+from bddcml_amd.cube import BoxProblem, CubeProblem
 
 pytestmark = pytest.mark.gpu
 
@@ -16,19 +16,34 @@ def test_iterations_do_not_change_over_many_solves(form, kind):
     print("case repeated solves", form, kind, flush=True)
     p = CubeProblem(4, 3, kind=kind, rhs="random", seed=3)
     subs = list(p.subdomains())
-    # the automatic mode against the inverse formed at setup (1) and never (0)
+    # the automatic mode against the inverse formed at setup (1) and never (0).
+    # Poisson: estimated to pay after 33 (FP64) and 98 (FP32) applies, so the
+    # automatic mode starts with the sweeps; elasticity: after 6, so the inverse
+    # would be formed at setup, unless the form of the sweeps is asked for
+    pc_form = 1 if kind == "elasticity" else 0
     runs = {}
     for mode in (0, 1, 2):
-        b, (it, reason, _) = bddcml_amd.solve_cube(p, tol=1e-9, maxit=300,
-                                                   options=dict(form, explicit_inverse=mode))
+        b, (it, reason, _) = bddcml_amd.solve_cube(
+            p, tol=1e-9, maxit=300, options=dict(form, explicit_inverse=mode, pc_form=pc_form))
         out = [(it, reason, b.interface_solution())]
-        for _ in range(9):
+        formed, applies, after = b.inverse_state()
+        assert formed == (mode == 1)
+        swept = 1  # solves by the sweeps
+        while len(out) < 10 or (mode == 2 and len(out) < swept + 3):
+            assert len(out) < 60
             for d in subs:
                 b.change_subdomain_data(d)
             b.setup_new_data()
+            before = b.inverse_state()
             it, reason, _ = b.solve(0, 1e-9, 300, 50)
             out.append((it, reason, b.interface_solution()))
+            assert it >= 4  # the captured iteration is replayed
+            formed, applies, _ = b.inverse_state()
+            swept += not formed
+            if mode == 2:  # formed at the start of a solve, once that many applies have run
+                assert formed == (before[0] or before[1] >= after)
         b.finalize()
+        assert formed == (mode > 0) and (mode < 2 or swept >= 2 or after < 8)
         runs[mode] = out
     ref = runs[0][0]
     scale = np.abs(ref[2]).max()
@@ -37,3 +52,27 @@ def test_iterations_do_not_change_over_many_solves(form, kind):
             assert reason == 0 and abs(it - ref[0]) <= 1, (mode, k, it, reason)
             # two solutions of the same stopping test (1e-9, condition below 10)
             assert np.abs(u - ref[2]).max() < 1e-7 * scale
+
+
+@pytest.mark.parametrize("form", [{}, {"precision": 32}, {"refinement": 1}])
+@pytest.mark.parametrize("jump", [1e3, 1e6])
+def test_inverse_at_setup_on_stiff_layers(form, jump):
+    """Few uneven boxes with stiff layers: by default the inverse is formed
+    before the first apply, in FP32 too.  Iterations as by the sweeps: at jumps
+    of 1e6, where FP32 factors themselves cost iterations, the two counts
+    differed by one in 293."""
+    print("case stiff inverse", form, jump, flush=True)
+    p = BoxProblem(16, 8, seed=3, layers=5, jump=jump, rhs="random")
+    out = []
+    for mode in (0, 2):
+        b, (it, reason, _) = bddcml_amd.solve_cube(p, tol=1e-8, maxit=2000, ndecrmax=200,
+                                                   weights_type=1,
+                                                   options=dict(form, explicit_inverse=mode))
+        assert b.inverse_state()[0] == (mode == 2)
+        out.append((it, reason, b.interface_solution()))
+        b.finalize()
+    (it0, r0, u0), (it2, r2, u2) = out
+    assert r0 == 0 and r2 == 0
+    assert abs(it2 - it0) <= 1 + it0 // 100, (it0, it2)
+    # both stop at 1e-8 of the residual; condition number below 100 here
+    assert np.abs(u2 - u0).max() < 2e-6 * np.abs(u0).max()
