@@ -2,6 +2,8 @@
 subdomains, full storage) and on the device (from 16,384 triplets): any input
 order gives the same matrix, and a bad entry is refused with its message
 wherever it stands."""
+import time
+
 import numpy as np
 import pytest
 
@@ -58,8 +60,8 @@ def _matrices(p, change, matrixtype=1):
 
 @pytest.mark.gpu
 def test_long_rows_on_the_device():
-    """Every triplet in 20 parts: rows of up to 1,280 entries, beyond what the
-    device sort stages in LDS (512)."""
+    """Every triplet in 20 parts: rows of up to 1,280 entries, beyond what a
+    wave of the device sort holds in LDS (512)."""
     print("case long rows", flush=True)
     p = CubeProblem(4, 2, rhs="random", seed=3)  # 46,080 triplets
 
@@ -74,6 +76,80 @@ def test_long_rows_on_the_device():
         # sums of 160 terms in another order: 160 eps of the entries' sum of moduli
         assert np.abs(a - b).max() <= 1e-12 * np.abs(a).max()
     assert np.abs(u - v).max() <= 1e-9 * np.abs(u).max()
+
+
+def _with_long_row(p, d, length, columns):
+    """d with `length` more entries in one row, over `columns` columns in
+    random order, and the diagonal that keeps the matrix positive definite."""
+    rng = np.random.RandomState(length)
+    n = d["ndofs"]
+    r = n - 1 - columns
+    v = rng.rand(length) - 0.5
+    j = rng.permutation(np.arange(length) % columns) + r + 1
+    add = np.bincount(j, np.abs(v), minlength=n)
+    add[r] += np.abs(v).sum()
+    k = np.nonzero(add)[0]
+    cat = lambda x, *y: np.concatenate((x,) + y).astype(x.dtype)
+    return dict(d, i_sparse=cat(d["i_sparse"], np.full(length, r) + p.numbase, k + p.numbase),
+                j_sparse=cat(d["j_sparse"], j + p.numbase, k + p.numbase),
+                a_sparse=cat(d["a_sparse"], v, add[k]))
+
+
+# rows about the ends of what a wave (512) and a run (1,024) hold, of an even
+# and an odd number of merges; one column (all duplicates) to 700
+@pytest.mark.gpu
+@pytest.mark.parametrize("length,columns", [(480, 400), (512, 512), (513, 512), (1024, 700), (1025, 1),
+                                            (2048, 700), (2049, 700), (4097, 37), (20000, 700),
+                                            (20000, 1), (70000, 2)])
+def test_one_long_row(length, columns):
+    """One row of many entries, of many duplicates: the device assembly
+    against the host's of the same matrix in full storage."""
+    print("case one long row", length, columns, flush=True)
+    p = CubeProblem(8, 2, rhs="random", seed=3)
+    out = []
+    for full in (False, True):
+        def change(d, k):
+            d = _with_long_row(p, d, length, columns) if k == 0 else d
+            return _shuffled(d, k, True) if full else d
+        out.append(_matrices(p, change, 0 if full else 1))
+    (x, u), (y, v) = out
+    for a, b in zip(x, y):
+        # sums of up to 70,000 terms in another order: 70,000 eps of the sum of
+        # moduli, which the diagonals hold
+        assert np.abs(a - b).max() <= 2e-11 * np.abs(a).max()
+    assert np.abs(u - v).max() <= 1e-8 * np.abs(u).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("columns", [1, 364])
+def test_a_long_row_costs_no_more_than_its_entries(columns):
+    """20,000 more entries in one row: as the same number spread over all rows,
+    and 50 ms (ranks over the whole row took 590 ms)."""
+    print("case cost of a long row", columns, flush=True)
+    p = CubeProblem(8, 2, rhs="random", seed=3)
+    subs = list(p.subdomains())
+    d0 = subs[0]
+    n = d0["ndofs"]
+    zeros = np.zeros(20000)
+    lo = np.random.RandomState(1).randint(0, n, (2, 20000))
+    best = []
+    for i, j in ((lo.min(0), lo.max(0)),
+                 (np.full(20000, n - 1 - columns), n - columns + np.arange(20000) % columns)):
+        d = dict(d0, i_sparse=np.concatenate([d0["i_sparse"], i + p.numbase]).astype(np.int32),
+                 j_sparse=np.concatenate([d0["j_sparse"], j + p.numbase]).astype(np.int32),
+                 a_sparse=np.concatenate([d0["a_sparse"], zeros]))
+        t = []
+        for _ in range(3):
+            b = bddcml_amd.Bddcml()
+            b.init(2, [p.nsub, 1], numbase=p.numbase)
+            t0 = time.perf_counter()
+            for s in [d] + subs[1:]:
+                b.upload_subdomain_data(s)
+            b.setup_preconditioner()
+            t.append(time.perf_counter() - t0)
+            b.finalize()
+        best.append(min(t))
+    assert best[1] < best[0] + 0.05, best
 
 
 @pytest.mark.gpu
