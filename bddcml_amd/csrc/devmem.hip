@@ -17,7 +17,7 @@ namespace {
 struct Block {
   void *p;
   size_t bytes;
-  int dev;
+  int dev;   // device it lies on; of pinned memory: current when handed out
   int used;  // problem that used it last
 };
 
@@ -40,21 +40,34 @@ int current_device() {
   return d;
 }
 
-// the smallest kept block that fits without wasting more than a quarter
+// a device current for a scope
+struct OnDevice {
+  int before = -1;
+  explicit OnDevice(int dev) {
+    if (hipGetDevice(&before) != hipSuccess || before == dev || hipSetDevice(dev) != hipSuccess) before = -1;
+  }
+  ~OnDevice() {
+    if (before >= 0) (void)hipSetDevice(before);
+  }
+};
+
+// the smallest kept block (of one device, or -1) that fits without wasting
+// more than a quarter
 int best_fit(const std::vector<Block> &v, size_t bytes, int dev) {
   int best = -1;
   for (int k = 0; k < (int)v.size(); k++)
-    if (v[k].dev == dev && v[k].bytes >= bytes && v[k].bytes <= bytes + bytes / 4 + 4096 &&
+    if ((dev < 0 || v[k].dev == dev) && v[k].bytes >= bytes && v[k].bytes <= bytes + bytes / 4 + 4096 &&
         (best < 0 || v[k].bytes < v[best].bytes))
       best = k;
   return best;
 }
 
-void *take(Keep &K, std::vector<Block> &v, int k) {
+void *take(Keep &K, std::vector<Block> &v, int k, int dev) {
   Block b = v[k];
   v[k] = v.back();
   v.pop_back();
   b.used = K.problem;
+  b.dev = dev;
   K.out[b.p] = b;
   return b.p;
 }
@@ -84,7 +97,7 @@ void *dev_alloc(size_t bytes) {
   const int k = best_fit(K.idle, bytes, dev);
   if (k >= 0) {
     K.idle_bytes[dev] -= K.idle[k].bytes;
-    return take(K, K.idle, k);
+    return take(K, K.idle, k, dev);
   }
   void *p = nullptr;
   hipError_t e = hipMalloc(&p, bytes);
@@ -101,18 +114,28 @@ void *dev_alloc(size_t bytes) {
   return p;
 }
 
-void dev_free(void *p) {
-  if (!p) return;
-  (void)hipDeviceSynchronize();
-  Keep &K = keep();
+// the block handed out at p, no longer held by its user; false: none
+static bool withdraw(Keep &K, void *p, Block &b) {
   std::lock_guard<std::mutex> lock(K.m);
   const auto it = K.out.find(p);
-  if (it == K.out.end()) {
+  if (it == K.out.end()) return false;
+  b = it->second;
+  K.out.erase(it);
+  return true;
+}
+
+void dev_free(void *p) {
+  if (!p) return;
+  Keep &K = keep();
+  Block b{};
+  if (!withdraw(K, p, b)) {
     (void)hipFree(p);
     return;
   }
-  const Block b = it->second;
-  K.out.erase(it);
+  // work that uses it runs on the block's device, whichever is current now
+  OnDevice on(b.dev);
+  (void)hipDeviceSynchronize();
+  std::lock_guard<std::mutex> lock(K.m);
   size_t &bound = K.bound[b.dev];
   if (bound == 0) {
     size_t avail = 0, total = 0;
@@ -128,27 +151,27 @@ void dev_free(void *p) {
 }
 
 void *pinned_alloc(size_t bytes) {
+  const int dev = current_device();
   bytes = (std::max<size_t>(bytes, 1) + 4095) / 4096 * 4096;
   Keep &K = keep();
   std::lock_guard<std::mutex> lock(K.m);
-  const int k = best_fit(K.idle_pinned, bytes, 0);
-  if (k >= 0) return take(K, K.idle_pinned, k);
+  const int k = best_fit(K.idle_pinned, bytes, -1);
+  if (k >= 0) return take(K, K.idle_pinned, k, dev);
   void *p = nullptr;
   const hipError_t e = hipHostMalloc(&p, bytes, hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable);
   if (e != hipSuccess) fatal("BDDCML_DEVICE", std::string("hipHostMalloc failed: ") + hipGetErrorString(e));
-  K.out[p] = Block{p, bytes, 0, K.problem};
+  K.out[p] = Block{p, bytes, dev, K.problem};
   return p;
 }
 
 void pinned_free(void *p) {
-  if (!p) return;
-  (void)hipDeviceSynchronize();
   Keep &K = keep();
+  Block b{};
+  if (!p || !withdraw(K, p, b)) return;
+  OnDevice on(b.dev);
+  (void)hipDeviceSynchronize();
   std::lock_guard<std::mutex> lock(K.m);
-  const auto it = K.out.find(p);
-  if (it == K.out.end()) return;
-  K.idle_pinned.push_back(it->second);
-  K.out.erase(it);
+  K.idle_pinned.push_back(b);
 }
 
 hipStream_t stream_get() {

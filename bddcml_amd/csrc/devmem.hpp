@@ -20,7 +20,8 @@ namespace bddc {
 // device block of at least `bytes` on the current device, contents undefined
 void *dev_alloc(size_t bytes);
 // back to the kept blocks, or to the driver beyond their bound.  Waits for
-// the device first, as hipFree does: work on any stream may still use it.
+// the block's device first, as hipFree does: work on any stream may still use
+// it.
 void dev_free(void *p);
 // mapped coherent pinned host memory (for values a kernel writes and the
 // host polls)

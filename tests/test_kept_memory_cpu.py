@@ -1,0 +1,62 @@
+"""Device memory kept between problems, against a stand-in of the HIP runtime
+(tests/drivers/fake_hip.c): which device a returned block waits for.  No GPU is
+needed."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    cc = shutil.which("gcc") or shutil.which("cc")
+    if not cc:
+        pytest.skip("no C compiler")
+    out = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.check_call([cc, "-shared", "-fPIC", "-O1", "-w", "-o", out,
+                           os.path.join(ROOT, "tests", "drivers", "fake_hip.c")])
+    return out
+
+
+def _run(fake, body):
+    # its own process: the stand-in comes before the HIP runtime in the search
+    code = f"""
+import ctypes, sys
+sys.path.insert(0, {ROOT!r})
+fake = ctypes.CDLL({fake!r}, mode=ctypes.RTLD_GLOBAL)
+import bddcml_amd
+from bddcml_amd.cube import CubeProblem
+p = CubeProblem(8, 2)  # 18,432 triplets a subdomain: assembled on the device
+subs = list(p.subdomains())
+def start():
+    b = bddcml_amd.Bddcml()
+    b.init(2, [p.nsub, 1], numbase=p.numbase)
+    return b
+""" + body
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_blocks_wait_for_their_own_device(fake):
+    """The caller has gone on to another device when the problem ends."""
+    _run(fake, """
+fake.fake_device(1)
+b = start()
+for d in subs[:3]:
+    b.upload_subdomain_data(d)
+assert fake.fake_busy(1) == 1
+fake.fake_device(0)
+b.finalize()
+assert fake.fake_busy(1) == 0, "blocks taken back while their device works"
+assert fake.fake_current() == 0
+# the blocks serve device 1 again, not device 0
+before = fake.fake_copies()
+b = start()
+b.upload_subdomain_data(subs[0])
+assert fake.fake_copies() > before and fake.fake_bad_copies() == 0
+b.finalize()
+""")
