@@ -52,6 +52,7 @@
 #include <cstdio>
 #include <map>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "devmem.hpp"
@@ -614,9 +615,10 @@ template <class T> struct ABuf {
     dev_free(p);
   }
   void alloc(size_t cnt) {
-    dev_free(p);
-    n = cnt;
+    dev_free(std::exchange(p, nullptr));
+    n = 0;
     p = static_cast<T *>(dev_alloc(std::max<size_t>(cnt, 1) * sizeof(T)));
+    n = cnt;
   }
   void swap(ABuf &o) {
     std::swap(p, o.p);

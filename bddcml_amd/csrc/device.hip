@@ -108,8 +108,8 @@ struct DBuf {
   void alloc(size_t cnt) {
     const double t = wall_time();
     release();
-    n = cnt;
     p = static_cast<T *>(dev_alloc(std::max<size_t>(cnt, 1) * sizeof(T)));
+    n = cnt;  // (after the allocation, which may throw)
     g_alloc_s += wall_time() - t;
   }
   void upload(const std::vector<T> &v, hipStream_t st) {

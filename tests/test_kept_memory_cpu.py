@@ -1,6 +1,6 @@
 """Device memory kept between problems, against a stand-in of the HIP runtime
-(tests/drivers/fake_hip.c): which device a returned block waits for.  No GPU is
-needed."""
+(tests/drivers/fake_hip.c): which device a returned block waits for, and what
+an upload does after one that ran out of memory.  No GPU is needed."""
 import os
 import shutil
 import subprocess
@@ -58,5 +58,28 @@ before = fake.fake_copies()
 b = start()
 b.upload_subdomain_data(subs[0])
 assert fake.fake_copies() > before and fake.fake_bad_copies() == 0
+b.finalize()
+""")
+
+
+@pytest.mark.parametrize("nth", range(8))
+def test_upload_after_out_of_memory(fake, nth):
+    """The nth device allocation fails: that upload reports it, and the next
+    ones copy into memory that is there."""
+    _run(fake, f"""
+b = start()
+fake.fake_fail_at({nth})
+failed = 0
+for d in subs:
+    for again in range(2):
+        try:
+            b.upload_subdomain_data(d)
+            break
+        except RuntimeError as e:
+            assert "hipMalloc" in str(e), e
+            failed += 1
+assert fake.fake_bad_copies() == 0, fake.fake_bad_copies()
+assert failed <= 1
+assert failed == 1 or {nth} > 3
 b.finalize()
 """)
