@@ -429,10 +429,8 @@ void bddcml_setup_preconditioner_c(int *matrixtype, int *use_defaults_int,
   };
   // what the interior factorization needs: the interior / interface split
   // and the orderings; globs and constraints follow while the device factors
-  if (!S.plan_only) {
-    device_finish_uploads(S);
-    phase("uploads finished");
-  }
+  device_finish_uploads(S);  // (also of uploads before the option plan_only was set)
+  phase("uploads finished");
   build_topology(S);
   phase("topology");
   build_orderings(S);

@@ -464,9 +464,9 @@ struct DeviceInput {
 // that of its candidate cand[i] where the uploaded copies are (HBM), instead
 // of reading both patterns on the host.  eq[i] = 1 when equal.  False (eq
 // untouched) when the host arrays are not the uploaded ones (a Dirichlet
-// elimination added diagonal entries) or in the plan-only mode.
+// elimination added diagonal entries) or nothing was uploaded (plan-only mode).
 bool device_same_patterns(Solver &S, const std::vector<int> &cand, std::vector<char> &eq) {
-  if (S.plan_only || !S.din) return false;
+  if (!S.din) return false;
   DeviceInput &I = *S.din;
   const int n = S.nsub;
   if ((int)I.ai.size() != n || (int)I.aj.size() != n || (int)cand.size() != n) return false;

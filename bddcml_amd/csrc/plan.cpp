@@ -1218,7 +1218,7 @@ void build_orderings(Solver &S) {
         if (!device_same_patterns(S, cand, pat_eq)) pat_eq.clear();
       });
   phase("classes");
-  if (!S.plan_only) device_fetch_patterns(S, S.ord_reps);
+  device_fetch_patterns(S, S.ord_reps);
 #pragma omp parallel for schedule(dynamic)
   for (int k = 0; k < (int)S.ord_reps.size(); k++)
     order_subdomain(S.subs[S.ord_reps[k]], S.ordering, S.nd_leaf, S.ndim);

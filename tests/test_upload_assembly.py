@@ -248,6 +248,31 @@ def test_bad_entries_are_refused_before_the_device(place):
     b.finalize()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("nel", [4, 8])
+def test_plan_only_after_the_uploads(nel):
+    """plan_only set between the uploads and the setup: the plan has the
+    diagonals (stiffness weights) and patterns that were assembled on the
+    device, as a plan from host assemblies and a whole setup have."""
+    print("case plan after uploads", nel, flush=True)
+    p = CubeProblem(nel, 2, rhs="random", seed=3, dirichlet="random")
+    out = []
+    for before, after in ((0, 1), (1, 1), (0, 0)):
+        b = bddcml_amd.Bddcml()
+        b.init(2, [p.nsub, 1], numbase=p.numbase)
+        b.set_option("plan_only", before)
+        for d in p.subdomains():
+            b.upload_subdomain_data(d)
+        b.set_option("plan_only", after)
+        b.setup_preconditioner(1, weights_type=1)
+        maps = [b.sub_maps(s + p.numbase) for s in range(p.nsub)]
+        out.append((b.counts(), [x for m in maps for x in m], b.interface_dofs()))
+        b.finalize()
+    for c, maps, dofs in out[1:]:
+        assert c == out[0][0] and np.array_equal(dofs, out[0][2])
+        assert all(np.array_equal(x, y) for x, y in zip(maps, out[0][1]))
+
+
 def test_first_bad_entry_names_the_error():
     """Two bad entries in different threads' shares: the first one counts."""
     p = CubeProblem(12, 2)
