@@ -39,6 +39,7 @@ EXTRA_SYMBOLS = [
     "bddcml_amd_selftest_copy", "bddcml_amd_element_gradient", "bddcml_amd_recycling_basis",
     "bddcml_amd_level2_counts", "bddcml_amd_level_counts", "bddcml_amd_element_gradient_noalloc",
     "bddcml_amd_adaptive_pairs", "bddcml_amd_inverse_state",
+    "bddcml_amd_device_memory",
 ]
 
 
@@ -398,6 +399,12 @@ class Bddcml:
         n, orth = C.c_int(), C.c_double()
         self.L.bddcml_amd_recycling_basis(C.byref(n), C.byref(orth))
         return n.value, orth.value
+
+    def device_memory(self):
+        """Device bytes (held by the problem, kept for the next one)."""
+        out = np.zeros(2)
+        self.L.bddcml_amd_device_memory(out.ctypes.data_as(C.POINTER(C.c_double)))
+        return float(out[0]), float(out[1])
 
     def inverse_state(self, level=1):
         """Explicit inverse of a level: (formed, applies counted by the

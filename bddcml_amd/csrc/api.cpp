@@ -785,6 +785,13 @@ int bddcml_amd_reduced_rhs(double *g) try {
 catch (const Error &e) {
   record_error(e); return -100;
 }
+int bddcml_amd_device_memory(double *out) try {
+  device_memory(out);
+  return 0;
+}
+catch (const Error &e) {
+  record_error(e); return -100;
+}
 int bddcml_amd_inverse_state(int ilevel, double *out) try {
   Solver *L = &solver();
   if (!L->is_setup || L->plan_only) return -1;

@@ -198,14 +198,18 @@ __device__ __forceinline__ uint64_t mix64(uint64_t z) {
 
 // the assembled entries: one wave per row, the first lane of each column
 // sums its duplicates in input order; info->hash = sum of a hash of every
-// (row, column), whatever the order of the rows
+// (row, column), whatever the order of the rows.  Also diag (0 where a row has
+// no diagonal entry: it leads its row in the upper triangle) and, where the
+// subdomain has fixed dofs (bptr), the row's entries that touch one: cur
 __global__ __launch_bounds__(ASM_THR) void k_asm_sum(const AsmSub *__restrict__ subs) {
   const AsmSub d = subs[blockIdx.y];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   uint64_t h = 0;
   for (int r = blockIdx.x * (ASM_THR / 64) + w; r < d.nd; r += gridDim.x * (ASM_THR / 64)) {
     const int p0 = d.rowp[r], p1 = d.rowp[r + 1];
-    int o = d.uptr[r];
+    int o = d.uptr[r], nbc = 0;
+    const bool fr = d.bptr && d.fix[r] != 0;
+    if (p0 == p1 && lane == 0) d.diag[r] = 0.0;
     for (int q0 = p0; q0 < p1; q0 += 64) {
       const int q = q0 + lane;
       const bool live = q < p1;
@@ -249,41 +253,27 @@ __global__ __launch_bounds__(ASM_THR) void k_asm_sum(const AsmSub *__restrict__ 
         d.aj[e] = (int)j;
         d.av[e] = s;
         h += mix64((uint64_t)(uint32_t)r << 32 | j);
+        if (q == p0) d.diag[r] = (int)j == r ? s : 0.0;
       }
       o += __popcll(m);
+      if (d.bptr) nbc += __popcll(__ballot(head && (fr || d.fix[j] != 0)));
     }
+    if (d.bptr && lane == 0) d.cur[r] = nbc;
   }
 #pragma unroll
   for (int s = 32; s > 0; s >>= 1) h += __shfl_xor((unsigned long long)h, s);
   if (lane == 0 && h) atomicAdd((unsigned long long *)&d.info->hash, (unsigned long long)h);
 }
 
-// what the host keeps of the assembled matrix: the diagonal (diag, 0 where a
-// row has none: it leads its row in the upper triangle) and, where the
-// subdomain has fixed dofs, the entries that touch one, in order
-__global__ __launch_bounds__(ASM_THR) void k_asm_diag(const AsmSub *__restrict__ subs) {
-  const AsmSub d = subs[blockIdx.y];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  for (int r = blockIdx.x * (ASM_THR / 64) + w; r < d.nd; r += gridDim.x * (ASM_THR / 64)) {
-    const int p0 = d.uptr[r], p1 = d.uptr[r + 1];
-    if (lane == 0) d.diag[r] = p0 < p1 && d.aj[p0] == r ? d.av[p0] : 0.0;
-    if (!d.bptr) continue;
-    const bool fr = d.fix[r] != 0;
-    int n = 0;
-    for (int q = p0 + lane; q < p1; q += 64) n += fr || d.fix[d.aj[q]] != 0;
-#pragma unroll
-    for (int s = 32; s > 0; s >>= 1) n += __shfl_xor(n, s);
-    if (lane == 0) d.cur[r] = n;
-  }
-}
+// the entries that touch a fixed dof, in order
 __global__ __launch_bounds__(ASM_THR) void k_asm_fixed(const AsmSub *__restrict__ subs) {
   const AsmSub d = subs[blockIdx.y];
-  if (!d.bptr) return;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   for (int r = blockIdx.x * (ASM_THR / 64) + w; r < d.nd; r += gridDim.x * (ASM_THR / 64)) {
+    int o = d.bptr[r];
+    if (o == d.bptr[r + 1]) continue;
     const int p0 = d.uptr[r], p1 = d.uptr[r + 1];
     const bool fr = d.fix[r] != 0;
-    int o = d.bptr[r];
     for (int q0 = p0; q0 < p1; q0 += 64) {
       const int q = q0 + lane;
       const bool in = q < p1 && (fr || d.fix[d.aj[q]] != 0);
@@ -299,30 +289,29 @@ __global__ __launch_bounds__(ASM_THR) void k_asm_fixed(const AsmSub *__restrict_
   }
 }
 
-void launch_assemble_triplets(hipStream_t st, const AsmSub *subs, int nsub, int maxn, int maxnd) {
+static unsigned row_grid(int maxnd) {
+  return (unsigned)std::min((maxnd + 15) / 16, 1024);  // 4 rows a wave or more
+}
+void launch_sort_triplets(hipStream_t st, const AsmSub *subs, int nsub, int maxn, int maxnd) {
   if (nsub <= 0) return;
   const unsigned gn = (unsigned)std::min((maxn + 1023) / 1024, 256);
-  const unsigned gr = (unsigned)std::min((maxnd + 15) / 16, 1024);  // 4 rows a wave or more
   hipLaunchKernelGGL(k_asm_zero, dim3((maxnd + 255) / 256, nsub), dim3(256), 0, st, subs);
   hipLaunchKernelGGL(k_asm_count, dim3(gn, nsub), dim3(256), 0, st, subs);
   hipLaunchKernelGGL(k_asm_scan, dim3(nsub), dim3(1024), 0, st, subs, 0);
   hipLaunchKernelGGL(k_asm_place, dim3(gn, nsub), dim3(256), 0, st, subs);
-  hipLaunchKernelGGL(k_asm_sort, dim3(gr, nsub), dim3(ASM_THR), 0, st, subs);
+  hipLaunchKernelGGL(k_asm_sort, dim3(row_grid(maxnd), nsub), dim3(ASM_THR), 0, st, subs);
   hipLaunchKernelGGL(k_asm_sort_long, dim3(std::min((maxnd + ASM_SCAN - 1) / ASM_SCAN, 256), nsub),
                      dim3(ASM_RUN), 0, st, subs);
   hipLaunchKernelGGL(k_asm_scan, dim3(nsub), dim3(1024), 0, st, subs, 1);
-  hipLaunchKernelGGL(k_asm_sum, dim3(gr, nsub), dim3(ASM_THR), 0, st, subs);
 }
-void launch_assembled_diag(hipStream_t st, const AsmSub *subs, int nsub, int maxnd) {
+void launch_sum_triplets(hipStream_t st, const AsmSub *subs, int nsub, int maxnd) {
   if (nsub <= 0) return;
-  const unsigned gr = (unsigned)std::min((maxnd + 15) / 16, 1024);
-  hipLaunchKernelGGL(k_asm_diag, dim3(gr, nsub), dim3(ASM_THR), 0, st, subs);
+  hipLaunchKernelGGL(k_asm_sum, dim3(row_grid(maxnd), nsub), dim3(ASM_THR), 0, st, subs);
   hipLaunchKernelGGL(k_asm_scan, dim3(nsub), dim3(1024), 0, st, subs, 2);
 }
 void launch_assembled_fixed(hipStream_t st, const AsmSub *subs, int nsub, int maxnd) {
   if (nsub <= 0) return;
-  const unsigned gr = (unsigned)std::min((maxnd + 15) / 16, 1024);
-  hipLaunchKernelGGL(k_asm_fixed, dim3(gr, nsub), dim3(ASM_THR), 0, st, subs);
+  hipLaunchKernelGGL(k_asm_fixed, dim3(row_grid(maxnd), nsub), dim3(ASM_THR), 0, st, subs);
 }
 
 }  // namespace bddc

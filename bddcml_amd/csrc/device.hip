@@ -435,22 +435,48 @@ struct DeviceInput {
   std::vector<View<double>> av;
   std::vector<DBuf<char>> chunks;
   size_t used = 0;  // bytes taken of the last chunk
-  // assemblies on the device: queued ones, their work space, row starts and
-  // Dirichlet flags of the assembled matrices
-  std::vector<AsmSub> pending;
-  DBuf<char> work;
-  size_t work_used = 0;
+  // Assemblies on the device, in batches of as many subdomains as fit the work
+  // space, two batches in turn: once a batch is full its entries are sorted and
+  // counted in the background, and when the next one is full the counts are
+  // there, room for exactly the assembled entries is taken and they are summed.
+  struct Batch {
+    std::vector<AsmSub> subs;
+    std::vector<int> is;
+    DBuf<char> work;
+    size_t used = 0;
+    size_t rows = 0;
+    View<double> diag;  // of all its subdomains, one after the other
+    bool sorted = false;
+    hipEvent_t counted = nullptr;
+    AsmInfo *info = nullptr;  // pinned: every subdomain's counts, by then
+  };
+  Batch batch[2];
+  int cur = 0;
   DBuf<AsmInfo> info;
-  std::vector<View<int>> uptr;
-  std::vector<View<char>> fix;
+  struct Assembled {  // what the device keeps beside the entries
+    int *uptr, *bptr;
+    const char *fix;
+  };
+  std::vector<Assembled> done;
+  struct DiagRange {  // diagonals of a batch, in the order of its subdomains
+    View<double> v;
+    std::vector<int> is;
+  };
+  std::vector<DiagRange> diags;
   bool fetched = true;
   DBuf<char> cmp;   // pointer tables and flags of the pattern comparison
+  ~DeviceInput() {
+    for (Batch &B : batch) {
+      if (B.counted) (void)hipEventDestroy(B.counted);
+      pinned_free(B.info);
+    }
+  }
   template <class T> void carve(View<T> &v, size_t n) {
     const size_t bytes = (std::max<size_t>(n, 1) * sizeof(T) + 255) / 256 * 256;
     if (chunks.empty() || used + bytes > chunks.back().n) {
       const size_t last = chunks.empty() ? (size_t)1 << 20 : chunks.back().n;
       DBuf<char> c;
-      c.alloc(std::max(bytes, std::min<size_t>(2 * last, (size_t)256 << 20)));
+      c.alloc(std::max(bytes, std::min<size_t>(2 * last, (size_t)32 << 20)));
       chunks.push_back(std::move(c));
       used = 0;
     }
@@ -554,27 +580,76 @@ void device_upload_entries(Solver &S, int is) {
   HIPCHECK(hipMemcpyAsync(I.aj[is].p, h + 12 * n, bi, hipMemcpyHostToDevice, nullptr));
 }
 
-// launches the assemblies queued so far
-static void flush_assemblies(DeviceInput &I) {
-  if (I.pending.empty()) return;
-  int maxn = 0, maxnd = 0;
-  for (const AsmSub &a : I.pending) maxn = std::max(maxn, a.n), maxnd = std::max(maxnd, a.nd);
-  const size_t bytes = I.pending.size() * sizeof(AsmSub);
-  char *h = upload_room(bytes);
-  std::memcpy(h, I.pending.data(), bytes);
+// a batch's descriptors on the device
+static const AsmSub *send_batch(DeviceInput &I, const std::vector<AsmSub> &subs) {
+  const size_t bytes = subs.size() * sizeof(AsmSub);
   View<char> v;
   I.carve(v, bytes);
+  char *h = upload_room(bytes);
+  std::memcpy(h, subs.data(), bytes);
   HIPCHECK(hipMemcpyAsync(v.p, h, bytes, hipMemcpyHostToDevice, nullptr));
-  launch_assemble_triplets(nullptr, reinterpret_cast<const AsmSub *>(v.p), (int)I.pending.size(), maxn,
-                           maxnd);
+  return reinterpret_cast<const AsmSub *>(v.p);
+}
+
+static void batch_sizes(const DeviceInput::Batch &B, int &maxn, int &maxnd) {
+  maxn = maxnd = 0;
+  for (const AsmSub &a : B.subs) maxn = std::max(maxn, a.n), maxnd = std::max(maxnd, a.nd);
+}
+
+// a full batch: its entries sorted and counted in the background
+static void sort_batch(Solver &S, DeviceInput &I, DeviceInput::Batch &B) {
+  int maxn, maxnd;
+  batch_sizes(B, maxn, maxnd);
+  if (!B.info) B.info = static_cast<AsmInfo *>(pinned_alloc(S.nsub * sizeof(AsmInfo)));
+  if (!B.counted) HIPCHECK(hipEventCreateWithFlags(&B.counted, hipEventDisableTiming));
+  launch_sort_triplets(nullptr, send_batch(I, B.subs), (int)B.subs.size(), maxn, maxnd);
   HIPCHECK(hipGetLastError());
-  I.pending.clear();
-  I.work_used = 0;  // reused in stream order
+  HIPCHECK(hipMemcpyAsync(B.info, I.info.p, S.nsub * sizeof(AsmInfo), hipMemcpyDeviceToHost, nullptr));
+  HIPCHECK(hipEventRecord(B.counted, nullptr));
+  B.sorted = true;
+}
+
+// a sorted batch: room for its assembled entries, their sums, diagonals and
+// couplings with fixed dofs; its work space is free (in stream order)
+static void sum_batch(DeviceInput &I, DeviceInput::Batch &B) {
+  if (!B.sorted) return;
+  HIPCHECK(hipEventSynchronize(B.counted));
+  View<double> diag;
+  I.carve(diag, B.rows);
+  size_t row = 0;
+  for (size_t k = 0; k < B.subs.size(); k++) {
+    AsmSub &t = B.subs[k];
+    const int is = B.is[k], n = B.info[is].nnz;
+    if (n < 0 || n > t.n) fatal("BDDCML_DEVICE", "invalid triplet assembly");
+    I.carve(I.ai[is], n);
+    I.carve(I.aj[is], n);
+    I.carve(I.av[is], n);
+    t.ai = I.ai[is].p, t.aj = I.aj[is].p, t.av = I.av[is].p;
+    t.diag = diag.p + row;
+    row += t.nd;
+  }
+  int maxn, maxnd;
+  batch_sizes(B, maxn, maxnd);
+  launch_sum_triplets(nullptr, send_batch(I, B.subs), (int)B.subs.size(), maxnd);
+  HIPCHECK(hipGetLastError());
+  I.diags.push_back({diag, std::move(B.is)});
+  B.subs.clear();
+  B.is.clear();
+  B.used = B.rows = 0;
+  B.sorted = false;
+}
+
+// ends the current batch (none: nothing to do); the other one becomes current
+static void end_batch(Solver &S, DeviceInput &I) {
+  DeviceInput::Batch &B = I.batch[I.cur], &other = I.batch[1 - I.cur];
+  if (B.subs.empty()) return;
+  sum_batch(I, other);
+  sort_batch(S, I, B);
+  I.cur = 1 - I.cur;
 }
 
 // Unassembled triplets into pinned memory (by all threads, which check them
-// on the way), to the device and into the queue of assemblies; a flush takes
-// as many subdomains as fit the work space.
+// on the way), to the device and into the current batch of assemblies.
 int device_assemble_entries(Solver &S, int is, int la, const int *ii, const int *jj, const double *aa,
                             int b) {
   DeviceInput &I = device_input(S);
@@ -584,13 +659,15 @@ int device_assemble_entries(Solver &S, int is, int la, const int *ii, const int 
   const size_t cap = (size_t)la + (s.has_fix ? nd : 0);
   const size_t oi = 8 * cap, oj = oi + 4 * cap, ofx = oj + 4 * cap, raw = (ofx + nd + 255) / 256 * 256;
   // work space: the input and the keys and counts of its assembly (before the
-  // staging area is taken: a flush stages its descriptors there)
+  // staging area is taken: the end of a batch stages its descriptors there)
   const size_t keys = (cap * 8 + 255) / 256 * 256, rows = ((size_t)(nd + 1) * 4 + 255) / 256 * 256;
   const size_t need = raw + 2 * keys + 2 * rows;
-  if (I.work_used + need > I.work.n) {
-    flush_assemblies(I);
-    if (need > I.work.n) I.work.alloc(std::min(std::max<size_t>(need, (size_t)96 << 20), 8 * need));
+  if (I.batch[I.cur].used + need > I.batch[I.cur].work.n) {
+    end_batch(S, I);
+    DBuf<char> &work = I.batch[I.cur].work;
+    if (need > work.n) work.alloc(std::min(std::max<size_t>(need, (size_t)96 << 20), 8 * need));
   }
+  DeviceInput::Batch &B = I.batch[I.cur];
   char *h = upload_room(raw);
   double *ha = reinterpret_cast<double *>(h);
   int *hi = reinterpret_cast<int *>(h + oi), *hj = reinterpret_cast<int *>(h + oj);
@@ -626,17 +703,16 @@ int device_assemble_entries(Solver &S, int is, int la, const int *ii, const int 
     hf[d] = s.ifix[d] != 0;
     if (dg && hf[d] && !dg[d]) hi[n] = hj[n] = d + b, ha[n] = 0.0, n++;
   }
-  char *w = I.work.p + I.work_used;
-  I.work_used += need;
-  HIPCHECK(hipMemcpyAsync(w, h, raw, hipMemcpyHostToDevice, nullptr));
   if (I.info.n < (size_t)S.nsub) I.info.alloc(S.nsub);
-  if (I.uptr.empty()) I.uptr.resize(S.nsub), I.fix.resize(S.nsub);
-  I.carve(I.ai[is], n);
-  I.carve(I.aj[is], n);
-  I.carve(I.av[is], n);
-  I.carve(I.uptr[is], nd + 1);
-  I.carve(I.fix[is], nd);
-  HIPCHECK(hipMemcpyAsync(I.fix[is].p, h + ofx, nd, hipMemcpyHostToDevice, nullptr));
+  I.done.resize(S.nsub);
+  View<int> uptr, bptr;
+  View<char> fix;
+  I.carve(uptr, nd + 1);
+  if (s.has_fix) I.carve(bptr, nd + 1);
+  I.carve(fix, nd);
+  char *w = B.work.p + B.used;
+  HIPCHECK(hipMemcpyAsync(w, h, raw, hipMemcpyHostToDevice, nullptr));
+  HIPCHECK(hipMemcpyAsync(fix.p, h + ofx, nd, hipMemcpyHostToDevice, nullptr));
   AsmSub t{};
   t.a = reinterpret_cast<const double *>(w);
   t.i = reinterpret_cast<const int *>(w + oi);
@@ -646,9 +722,13 @@ int device_assemble_entries(Solver &S, int is, int la, const int *ii, const int 
   t.key2 = reinterpret_cast<uint64_t *>(w + raw + keys);
   t.rowp = reinterpret_cast<int *>(w + raw + 2 * keys);
   t.cur = reinterpret_cast<int *>(w + raw + 2 * keys + rows);
-  t.uptr = I.uptr[is].p, t.ai = I.ai[is].p, t.aj = I.aj[is].p, t.av = I.av[is].p;
+  t.uptr = uptr.p, t.bptr = bptr.p, t.fix = fix.p;
   t.info = I.info.p + is;
-  I.pending.push_back(t);
+  I.done[is] = {uptr.p, bptr.p, fix.p};
+  B.used += need;
+  B.rows += nd;
+  B.subs.push_back(t);
+  B.is.push_back(is);
   I.fetched = false;
   return la;
 }
@@ -656,73 +736,62 @@ int device_assemble_entries(Solver &S, int is, int la, const int *ii, const int 
 void device_finish_uploads(Solver &S) {
   if (!S.din || S.din->fetched) return;
   DeviceInput &I = *S.din;
-  flush_assemblies(I);
+  end_batch(S, I);
+  sum_batch(I, I.batch[1 - I.cur]);
+  HIPCHECK(hipMemcpyAsync(I.batch[1 - I.cur].info, I.info.p, S.nsub * sizeof(AsmInfo),
+                          hipMemcpyDeviceToHost, nullptr));
+  HIPCHECK(hipStreamSynchronize(nullptr));
+  const AsmInfo *info = I.batch[1 - I.cur].info;
+  // the couplings of each subdomain with fixed dofs, counted by now, to one
+  // buffer
   std::vector<int> subs;
-  int maxnd = 0;
+  std::vector<size_t> ro, bo(1, 0);  // first diagonal, first coupling
+  std::vector<AsmSub> t;
   size_t rows = 0;
-  for (int is = 0; is < S.nsub; is++)
-    if (!S.subs[is].on_host) {
+  int maxnd = 0;
+  for (const DeviceInput::DiagRange &r : I.diags)
+    for (int is : r.is) {
+      Sub &s = S.subs[is];
+      const AsmInfo &f = info[is];
+      if (f.nnz < 0 || (size_t)f.nnz != I.ai[is].n || (s.has_fix && (f.nbc < 0 || f.nbc > f.nnz)))
+        fatal("BDDCML_DEVICE", "invalid triplet assembly");
+      s.nnz = f.nnz;
+      s.pat_hash = f.hash;
       subs.push_back(is);
-      maxnd = std::max(maxnd, S.subs[is].ndofs);
-      rows += S.subs[is].ndofs;
+      ro.push_back(rows);
+      rows += s.ndofs;
+      bo.push_back(bo.back() + (s.has_fix ? f.nbc : 0));
+      if (!s.has_fix || !f.nbc) continue;
+      AsmSub a{};
+      a.nd = s.ndofs;
+      a.uptr = I.done[is].uptr, a.bptr = I.done[is].bptr, a.fix = I.done[is].fix;
+      a.ai = I.ai[is].p, a.aj = I.aj[is].p, a.av = I.av[is].p;
+      t.push_back(a);
+      maxnd = std::max(maxnd, s.ndofs);
     }
   const int n = (int)subs.size();
-  // diagonals, and the couplings of each subdomain with fixed dofs: counted,
-  // then written to one buffer
-  DBuf<double> diag;
-  DBuf<int> cnt, bptr;
-  diag.alloc(rows);
-  cnt.alloc(rows);
-  bptr.alloc(rows + n);
-  std::vector<AsmSub> t(n);
-  std::vector<size_t> ro(n + 1, 0);
-  for (int k = 0; k < n; k++) {
-    const int is = subs[k];
-    const Sub &s = S.subs[is];
-    ro[k + 1] = ro[k] + s.ndofs;
-    AsmSub &a = t[k];
-    a = AsmSub{};
-    a.nd = s.ndofs;
-    a.cur = cnt.p + ro[k];
-    a.uptr = I.uptr[is].p, a.ai = I.ai[is].p, a.aj = I.aj[is].p, a.av = I.av[is].p;
-    a.info = I.info.p + is;
-    a.fix = I.fix[is].p;
-    a.diag = diag.p + ro[k];
-    a.bptr = s.has_fix ? bptr.p + ro[k] + k : nullptr;
-  }
-  DBuf<AsmSub> dt;
-  dt.upload(t, nullptr);
-  launch_assembled_diag(nullptr, dt.p, n, maxnd);
-  HIPCHECK(hipGetLastError());
-  std::vector<AsmInfo> info(S.nsub);
-  HIPCHECK(hipMemcpy(info.data(), I.info.p, S.nsub * sizeof(AsmInfo), hipMemcpyDeviceToHost));
-  std::vector<size_t> bo(n + 1, 0);
-  for (int k = 0; k < n; k++) {
-    Sub &s = S.subs[subs[k]];
-    const AsmInfo &f = info[subs[k]];
-    if (f.nnz < 0 || (size_t)f.nnz > I.ai[subs[k]].n || (s.has_fix && (f.nbc < 0 || f.nbc > f.nnz)))
-      fatal("BDDCML_DEVICE", "invalid triplet assembly");
-    s.nnz = f.nnz;
-    s.pat_hash = f.hash;
-    I.ai[subs[k]].n = I.aj[subs[k]].n = I.av[subs[k]].n = f.nnz;
-    bo[k + 1] = bo[k] + (s.has_fix ? f.nbc : 0);
-  }
-  // one read-back: diagonals, coupling values, rows, columns
-  DBuf<char> bc;
   const size_t nb = bo[n];
-  bc.alloc(16 * nb);
-  for (int k = 0; k < n; k++) {
-    t[k].ba = reinterpret_cast<double *>(bc.p) + bo[k];
-    t[k].bi = reinterpret_cast<int *>(bc.p + 8 * nb) + bo[k];
-    t[k].bj = reinterpret_cast<int *>(bc.p + 12 * nb) + bo[k];
+  DBuf<char> bc;  // values, rows, columns
+  if (nb) {
+    bc.alloc(16 * nb);
+    for (size_t k = 0, q = 0; k < (size_t)n; k++) {
+      if (bo[k + 1] == bo[k]) continue;
+      AsmSub &a = t[q++];
+      a.ba = reinterpret_cast<double *>(bc.p) + bo[k];
+      a.bi = reinterpret_cast<int *>(bc.p + 8 * nb) + bo[k];
+      a.bj = reinterpret_cast<int *>(bc.p + 12 * nb) + bo[k];
+    }
+    launch_assembled_fixed(nullptr, send_batch(I, t), (int)t.size(), maxnd);
+    HIPCHECK(hipGetLastError());
   }
-  HIPCHECK(hipMemcpyAsync(dt.p, t.data(), n * sizeof(AsmSub), hipMemcpyHostToDevice, nullptr));
-  launch_assembled_fixed(nullptr, dt.p, n, maxnd);
-  HIPCHECK(hipGetLastError());
   Staging &h = staging();
   h.used = 0;
   h.grow(8 * rows + 16 * nb);
-  HIPCHECK(hipMemcpyAsync(h.p, diag.p, 8 * rows, hipMemcpyDeviceToHost, nullptr));
+  size_t o = 0;
+  for (const DeviceInput::DiagRange &r : I.diags) {
+    HIPCHECK(hipMemcpyAsync(h.p + o, r.v.p, 8 * r.v.n, hipMemcpyDeviceToHost, nullptr));
+    o += 8 * r.v.n;
+  }
   if (nb) HIPCHECK(hipMemcpyAsync(h.p + 8 * rows, bc.p, 16 * nb, hipMemcpyDeviceToHost, nullptr));
   HIPCHECK(hipStreamSynchronize(nullptr));
   const double *hd = reinterpret_cast<const double *>(h.p), *hb = hd + rows;
@@ -730,13 +799,12 @@ void device_finish_uploads(Solver &S) {
 #pragma omp parallel for schedule(dynamic, 4)
   for (int k = 0; k < n; k++) {
     Sub &s = S.subs[subs[k]];
-    s.diag.assign(hd + ro[k], hd + ro[k + 1]);
+    s.diag.assign(hd + ro[k], hd + ro[k] + s.ndofs);
     s.bc_a.assign(hb + bo[k], hb + bo[k + 1]);
     s.bc_i.assign(hi + bo[k], hi + bo[k + 1]);
     s.bc_j.assign(hj + bo[k], hj + bo[k + 1]);
   }
-  I.work.release();
-  I.work_used = 0;
+  for (DeviceInput::Batch &B : I.batch) B.work.release();
   I.fetched = true;
 }
 
@@ -774,6 +842,8 @@ void device_fetch_patterns(Solver &S, const std::vector<int> &subs) {
 void device_release_input(Solver &S) { S.din.reset(); }
 
 void device_end_of_problem(bool nothing_held) { devmem_end_of_problem(nothing_held); }
+
+void device_memory(double *out) { devmem_bytes(out[0], out[1]); }
 
 void device_release(Solver &S) {
   if (S.lev2) {  // borrows this level's stream: released first

@@ -19,6 +19,7 @@ struct Block {
   size_t bytes;
   int dev;   // device it lies on; of pinned memory: current when handed out
   int used;  // problem that used it last
+  bool pinned;
 };
 
 struct Keep {
@@ -110,7 +111,7 @@ void *dev_alloc(size_t bytes) {
     (void)hipGetLastError();
     fatal("BDDCML_DEVICE", "hipMalloc of " + std::to_string(bytes) + " bytes failed: " + hipGetErrorString(e));
   }
-  K.out[p] = Block{p, bytes, dev, K.problem};
+  K.out[p] = Block{p, bytes, dev, K.problem, false};
   return p;
 }
 
@@ -160,7 +161,7 @@ void *pinned_alloc(size_t bytes) {
   void *p = nullptr;
   const hipError_t e = hipHostMalloc(&p, bytes, hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable);
   if (e != hipSuccess) fatal("BDDCML_DEVICE", std::string("hipHostMalloc failed: ") + hipGetErrorString(e));
-  K.out[p] = Block{p, bytes, dev, K.problem};
+  K.out[p] = Block{p, bytes, dev, K.problem, true};
   return p;
 }
 
@@ -203,6 +204,14 @@ void stream_put(hipStream_t st) {
   std::lock_guard<std::mutex> lock(K.m);
   if (K.streams.size() >= 16) (void)hipStreamDestroy(st);
   else K.streams.push_back({(int)dev, st});
+}
+
+void devmem_bytes(double &held, double &kept) {
+  Keep &K = keep();
+  std::lock_guard<std::mutex> lock(K.m);
+  held = kept = 0.0;
+  for (const auto &o : K.out) held += o.second.pinned ? 0.0 : (double)o.second.bytes;
+  for (const Block &b : K.idle) kept += (double)b.bytes;
 }
 
 void devmem_end_of_problem(bool nothing_held) {

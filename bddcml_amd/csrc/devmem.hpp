@@ -33,5 +33,7 @@ void stream_put(hipStream_t st);
 // end of one problem: gives back what it did not use; with nothing_held,
 // everything that is kept
 void devmem_end_of_problem(bool nothing_held);
+// bytes of device blocks handed out and kept
+void devmem_bytes(double &held, double &kept);
 
 }  // namespace bddc

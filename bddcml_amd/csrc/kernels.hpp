@@ -82,8 +82,8 @@ void launch_scatter_ones(hipStream_t st, double *pool, const int64_t *idx, int64
 
 // One subdomain of a batched triplet assembly (assemble.hip).  Input: n
 // triplets (i, j, a; indices from b) and nd rows; work: row counts and places
-// (rowp nd + 1, cur nd), keys (n each); result: the assembled entries (room
-// for n) with their row starts uptr (nd + 1) and info.
+// (rowp nd + 1, cur nd), keys (n each); result: row starts uptr (nd + 1) and
+// info, then the assembled entries (room for info->nnz).
 struct AsmInfo {
   int nnz, nbc;  // assembled entries; those touching a fixed dof
   uint64_t hash;  // of the assembled pattern
@@ -97,17 +97,19 @@ struct AsmSub {
   int *uptr, *ai, *aj;
   double *av;
   AsmInfo *info;
-  // diagonal and Dirichlet couplings (launch_assembled_diag / _fixed):
-  // Dirichlet flags, row starts of the couplings (null: none wanted), lists
+  // Dirichlet flags, diagonal, and couplings with fixed dofs: row starts (null:
+  // none wanted), lists
   const char *fix;
   double *diag;
   int *bptr, *bi, *bj;
   double *ba;
 };
-void launch_assemble_triplets(hipStream_t st, const AsmSub *subs, int nsub, int maxn, int maxnd);
-// diag, and with bptr the number of couplings per row and info->nbc
-void launch_assembled_diag(hipStream_t st, const AsmSub *subs, int nsub, int maxnd);
-// the couplings (bi, bj, ba), sorted by row and column
+// sorted keys, row starts uptr and info->nnz
+void launch_sort_triplets(hipStream_t st, const AsmSub *subs, int nsub, int maxn, int maxnd);
+// then the entries (ai, aj, av), diag, info->hash, and with bptr the row
+// starts of the couplings and info->nbc
+void launch_sum_triplets(hipStream_t st, const AsmSub *subs, int nsub, int maxnd);
+// then the couplings (bi, bj, ba), sorted by row and column
 void launch_assembled_fixed(hipStream_t st, const AsmSub *subs, int nsub, int maxnd);
 
 // diff[i] = 1 where the triplet pattern (ai, aj: device pointers) of

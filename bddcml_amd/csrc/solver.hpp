@@ -289,6 +289,8 @@ void device_release(Solver &S);
 // device memory kept for the next problem (devmem.hpp): what the problem
 // that ends did not use goes back, with nothing_held all of it
 void device_end_of_problem(bool nothing_held);
+// bytes handed out and kept
+void device_memory(double *out);
 
 double wall_time();
 // ask the runtime to spin (not sleep) in host waits on the device; called

@@ -126,6 +126,10 @@ int bddcml_amd_timings(double *out, int n);
  *     the first solve after as many applies as pay for it have run on the
  *     same setup; a solve never changes its preconditioner while it runs) */
 int bddcml_amd_set_option(const char *key, double value);
+/* device memory in bytes, on all devices of the process: out[0] held by the
+ * problem, out[1] kept for the next one (given back when an allocation would
+ * fail, and by a bddcml_finalize_c without a problem) */
+int bddcml_amd_device_memory(double *out);
 /* explicit inverse of level ilevel (1: the first): out[0] = 1 once it is
  * formed, out[1] = preconditioner applies that the automatic mode has counted
  * on this setup, out[2] = applies after which it is estimated to pay; returns

@@ -80,6 +80,6 @@ for d in subs:
             failed += 1
 assert fake.fake_bad_copies() == 0, fake.fake_bad_copies()
 assert failed <= 1
-assert failed == 1 or {nth} > 3
+assert failed == 1 or {nth} > 2
 b.finalize()
 """)

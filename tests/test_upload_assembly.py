@@ -153,6 +153,30 @@ def test_a_long_row_costs_no_more_than_its_entries(columns):
 
 
 @pytest.mark.gpu
+def test_room_for_the_assembled_entries_only():
+    """9.4 M triplets of 151 MB, 4.3 M assembled entries of 69 MB: the device
+    assembly, in several batches, holds no more than the assembled entries,
+    which are all that the host assembly (full storage) sends, row starts and
+    flags."""
+    print("case room for entries", flush=True)
+    p = CubeProblem(16, 4, rhs="random", seed=3)
+    held = []
+    for full in (True, False):
+        b = bddcml_amd.Bddcml()
+        b.init(2, [p.nsub, 1], numbase=p.numbase)
+        for k, d in enumerate(p.subdomains()):
+            b.upload_subdomain_data(_shuffled(d, k, True) if full else d)
+        b.setup_preconditioner(0 if full else 1)
+        held.append(b.device_memory()[0])
+        assert b.solve(0, 1e-8, 100, 50)[1] == 0
+        b.finalize()
+    assert b.device_memory()[0] == 0.0
+    # 13 to 25 bytes a dof beside the entries, blocks of up to 32 MiB (with room
+    # for all triplets 192 MB more)
+    assert held[1] <= held[0] + 42e6, held
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("nel", [4, 8, 9])
 def test_fixed_dofs_without_diagonal(nel):
     """Missing diagonals of fixed dofs become 1, nonzero fixed values move to
