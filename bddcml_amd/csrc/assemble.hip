@@ -289,6 +289,18 @@ __global__ __launch_bounds__(ASM_THR) void k_asm_fixed(const AsmSub *__restrict_
   }
 }
 
+__global__ __launch_bounds__(256) void k_gather_ranges(const GatherRange *__restrict__ g,
+                                                       char *__restrict__ dst) {
+  const GatherRange r = g[blockIdx.y];
+  const int *s = static_cast<const int *>(r.src);
+  int *d = reinterpret_cast<int *>(dst + r.off);
+  for (int64_t k = blockIdx.x * 256 + threadIdx.x; k < r.bytes / 4; k += gridDim.x * 256) d[k] = s[k];
+}
+void launch_gather_ranges(hipStream_t st, const GatherRange *g, int n, char *dst) {
+  for (int k = 0; k < n; k += 65535)
+    hipLaunchKernelGGL(k_gather_ranges, dim3(32, std::min(n - k, 65535)), dim3(256), 0, st, g + k, dst);
+}
+
 static unsigned row_grid(int maxnd) {
   return (unsigned)std::min((maxnd + 15) / 16, 1024);  // 4 rows a wave or more
 }

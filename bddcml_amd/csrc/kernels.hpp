@@ -112,6 +112,13 @@ void launch_sum_triplets(hipStream_t st, const AsmSub *subs, int nsub, int maxnd
 // then the couplings (bi, bj, ba), sorted by row and column
 void launch_assembled_fixed(hipStream_t st, const AsmSub *subs, int nsub, int maxnd);
 
+// ranges (bytes: whole words) copied to dst + off
+struct GatherRange {
+  const void *src;
+  int64_t off, bytes;
+};
+void launch_gather_ranges(hipStream_t st, const GatherRange *g, int n, char *dst);
+
 // diff[i] = 1 where the triplet pattern (ai, aj: device pointers) of
 // subdomain i differs from that of cand[i] (equal lengths cnt)
 void launch_same_pattern(hipStream_t st, const uint64_t *pai, const uint64_t *paj, const int *cand,

@@ -1219,6 +1219,7 @@ void build_orderings(Solver &S) {
       });
   phase("classes");
   device_fetch_patterns(S, S.ord_reps);
+  phase("patterns fetched");
 #pragma omp parallel for schedule(dynamic)
   for (int k = 0; k < (int)S.ord_reps.size(); k++)
     order_subdomain(S.subs[S.ord_reps[k]], S.ordering, S.nd_leaf, S.ndim);
