@@ -39,7 +39,7 @@ EXTRA_SYMBOLS = [
     "bddcml_amd_selftest_copy", "bddcml_amd_element_gradient", "bddcml_amd_recycling_basis",
     "bddcml_amd_level2_counts", "bddcml_amd_level_counts", "bddcml_amd_element_gradient_noalloc",
     "bddcml_amd_adaptive_pairs", "bddcml_amd_inverse_state",
-    "bddcml_amd_device_memory",
+    "bddcml_amd_device_memory", "bddcml_amd_selftest_inverse",
 ]
 
 
@@ -97,6 +97,23 @@ def selftest_tile(op, A, B, C_, X=None, alpha=1.0, beta=1.0):
                                Cm.ctypes.data_as(dp), Xm.ctypes.data_as(dp), alpha, beta,
                                out.ctypes.data_as(dp))
     return out[:4096].reshape(64, 64).T.copy(), out[4096:].reshape(64, 64).T.copy()
+
+
+def selftest_inverse(mats):
+    """Inverses of symmetric positive definite matrices in one device launch
+    (see include/bddcml_amd.h): (list of inverses, error flag)."""
+    L = _Checked(lib())
+    L.bddcml_amd_set_option(b"throw_on_error", 1.0)
+    mats = [np.ascontiguousarray(m, dtype=np.float64) for m in mats]
+    n = np.array([m.shape[0] for m in mats], dtype=np.int32)
+    a = np.concatenate([m.ravel() for m in mats] + [np.zeros(1)])
+    out = np.zeros_like(a)
+    err = C.c_int(0)
+    dp = C.POINTER(C.c_double)
+    L.bddcml_amd_selftest_inverse(len(mats), n.ctypes.data_as(C.POINTER(C.c_int)),
+                                  a.ctypes.data_as(dp), out.ctypes.data_as(dp), C.byref(err))
+    cut = np.concatenate([[0], np.cumsum(n.astype(np.int64) ** 2)])
+    return [out[cut[k]:cut[k + 1]].reshape(n[k], n[k]) for k in range(len(mats))], err.value
 
 
 def selftest_symeig(a):

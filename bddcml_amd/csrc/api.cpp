@@ -1026,6 +1026,19 @@ catch (const Error &e) {
   return -100;
 }
 
+int bddcml_amd_selftest_inverse(int nmat, const int *n, const double *a, double *out, int *err) try {
+  device_prefer_spin_wait();
+  for (int k = 0; k < nmat; k++)
+    if (n[k] < 0 || n[k] > 1024) fatal("BDDCML_SELFTEST", "order out of range");
+  *err = 0;
+  if (nmat > 0) device_selftest_inverse(nmat, n, a, out, err);
+  return 0;
+}
+catch (const Error &e) {
+  record_error(e);
+  return -100;
+}
+
 int bddcml_amd_selftest_symeig(int n, const double *a, double *w, double *v) try {
   if (n < 0) fatal("BDDCML_AMD_SELFTEST_SYMEIG", "negative order");
   std::vector<double> A(a, a + (size_t)n * n), W, V;

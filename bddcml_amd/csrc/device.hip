@@ -2945,6 +2945,31 @@ void device_reduced_rhs_download(Solver &S, double *g) {
 }
 
 // ------------------------------------------------------------- debug probes
+void device_selftest_inverse(int nmat, const int *n, const double *a, double *out, int *err) {
+  std::vector<SubDesc> d(nmat);
+  int64_t total = 0;
+  int maxn = 0;
+  for (int k = 0; k < nmat; k++) {
+    d[k] = SubDesc{};
+    d[k].nc = n[k];
+    d[k].goff = total;
+    total += (int64_t)n[k] * n[k];
+    maxn = std::max(maxn, n[k]);
+  }
+  DBuf<SubDesc> dd;
+  DBuf<double> G;
+  DBuf<int> e;
+  dd.upload(d, nullptr);
+  G.alloc(total);
+  e.alloc(1);
+  e.zero(nullptr);
+  if (total) HIPCHECK(hipMemcpy(G.p, a, total * sizeof(double), hipMemcpyHostToDevice));
+  launch_ginv(nullptr, dd.p, nmat, G.p, e.p, maxn);
+  HIPCHECK(hipGetLastError());
+  if (total) HIPCHECK(hipMemcpy(out, G.p, total * sizeof(double), hipMemcpyDeviceToHost));
+  HIPCHECK(hipMemcpy(err, e.p, sizeof(int), hipMemcpyDeviceToHost));
+}
+
 void device_selftest_tile(int op, int npairs, const double *A, const double *B, const double *C,
                           const double *X, double alpha, double beta, double *out) {
   if (npairs < 0 || npairs > 16) fatal("BDDCML_SELFTEST", "npairs out of range");

@@ -285,6 +285,7 @@ void device_element_gradient_noalloc(Solver &S, const double *ae, int nke, bool 
                                      const double *u, const double *lam, double *grad);
 void device_selftest_tile(int op, int npairs, const double *A, const double *B, const double *C,
                           const double *X, double alpha, double beta, double *out);
+void device_selftest_inverse(int nmat, const int *n, const double *a, double *out, int *err);
 void device_release(Solver &S);
 // device memory kept for the next problem (devmem.hpp): what the problem
 // that ends did not use goes back, with nothing_held all of it

@@ -155,6 +155,11 @@ int bddcml_amd_last_error(char *buf, int len);
  * op 3 the inverse in out[4096..8191] */
 int bddcml_amd_selftest_tile(int op, int npairs, const double *A, const double *B, const double *C,
                              const double *X, double alpha, double beta, double *out);
+/* inverses of nmat symmetric positive definite matrices in one launch, as the
+ * setup forms G^{-1} of every subdomain: matrix k has n[k] rows (0 to 1,024),
+ * stored one after the other; out as a, and *err is not 0 if a pivot was not
+ * positive */
+int bddcml_amd_selftest_inverse(int nmat, const int *n, const double *a, double *out, int *err);
 /* host symmetric eigendecomposition used for the Rayleigh-Ritz steps of the
  * adaptive constraints' LOBPCG (Householder tridiagonalization + implicit
  * QR): a (n x n, row major) in, eigenvalues w (unordered) and eigenvectors
