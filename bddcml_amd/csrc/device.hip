@@ -1130,15 +1130,21 @@ static std::vector<TaskList> merge_steps(const std::vector<Q> &sts, std::vector<
 // and subdomains at once, and a task keeps the products of its own chunk.
 //
 // A product takes a workgroup about 3.5 us (FP64, alone on a CU or one of two),
-// so a sum of 46 was 160 us with 5 to 70 workgroups running.  36 uneven boxes
-// (up to 49 tile rows): interface phase 22.3 -> 14.8 ms, interior GEMM launches
-// 5.6 -> 4.5; 64 subdomains of 16^3 (24 rows): 7.2 -> 5.8 and 3.1 -> 2.8; 27:
-// 5.2 -> 3.4 and 1.7 -> 1.3; 512, whose steps fill the chip, unchanged.
-// Chunks of 2 steps move more tiles per product (boxes 16.9 ms), of 8 leave
-// longer sums (15.2; 64 subdomains 6.0).  An interface step counts as too small
-// below one round of resident workgroups (four rounds: boxes 16.9 ms, its
-// updates cover all rows behind it), an interior one, with few columns
-// behind it, below four (one round: 5.1 and 3.1 ms).
+// so a sum of 46 was 160 us with 5 to 70 workgroups running.  Without chunks /
+// chunks of 2, 4, 8 steps, ms, measured in turn:
+// - interface phase with the inverse: 36 uneven boxes (up to 49 tile rows) 22.0
+//   / 16.1, 15.2, 15.8; 64 subdomains of 16^3 (25 rows) 7.2 / 5.9, 5.9, 6.0; 27:
+//   4.9 / 3.7, 3.6, 3.8; without it: boxes 13.3 / 7.9, 7.9, 8.2; 216: 9.7 / 9.3,
+//   9.2, 9.2; 512: 21.9 / 21.7, 21.7, 21.6;
+// - interior GEMM launches: boxes 5.6 / 4.6, 4.5, 4.5; 64: 3.05 / 2.86, 2.84,
+//   2.84; 27: 1.69 / 1.33, 1.30, 1.35; 512 (most steps fill the chip; the last
+//   one becomes a chunk of its own, whose extra launch of 80 us its shorter
+//   sums repay): 20.4 / 20.4, 20.4, 20.4.
+// Fewer steps a chunk move more tiles per product, more leave longer sums.  An
+// interface step counts as too small below one round of resident workgroups
+// (four rounds: boxes 16.9 ms, its updates cover all rows behind it), an
+// interior one, with few columns behind it, below four (one round: 5.1 and 3.1
+// ms for boxes and 64 subdomains).
 constexpr int kChunk = 4;
 template <class Q>
 static std::vector<int> step_chunks(const std::vector<Q> &sts, std::vector<TaskList> Q::*member,
@@ -1975,11 +1981,15 @@ static double interface_rho(const Sub &s) {
 //    row, 40 us of launches with too few workgroups;
 //  - an apply by sweeps: the larger of the slowest workgroup (3.4 us per
 //    tile row and direction, 0.7 / 0.4 us per tile) and both reads of the
-//    factors at 5.5 TB/s; by the inverse: one read at 5.9 TB/s and 15 us.
-// FP64, ms formed / sweeps / inverse: 64 subdomains n = 25: 2.8 / 0.57 / 0.08
-// (pays after 6); 36 boxes n <= 49: 7.6 / 2.19 / 0.12 (4); 60 boxes n <= 76:
-// 34.9 / 4.9 / 0.51 (8); 216 subdomains n = 25: 9.7 / 0.76 / 0.28 (20); 512:
-// 24.6 / 1.64 / 0.73 (27).
+//    factors at 5.7 / 5.5 TB/s; by the inverse: one read at 5.9 TB/s and 15 us.
+// Measured, ms formed / sweeps / inverse (pays after; estimated):
+// - FP64: 64 subdomains n = 25: 2.6 / 0.58 / 0.08 (5; 5); 36 boxes n <= 49:
+//   7.2 / 2.18 / 0.13 (3.5; 3.6); 60 boxes n <= 76: 33.6 / 4.91 / 0.50 (7.6; 6.9);
+//   216 subdomains n = 25: 9.7 / 0.74 / 0.29 (21; 29); 512: 24.2 / 1.52 / 0.73
+//   (31; 31).
+// - FP32: 64 subdomains 1.5 / 0.30 / 0.05 (6; 5); 60 boxes 23.3 / 2.74 / 0.47
+//   (10; 6: k_symv gathers inputs of more than 72 tile rows tile by tile,
+//   at 2.5 TB/s); 512: 12.0 / 0.82 / 0.40 (29; 32).
 static double inverse_pays_after(const std::vector<SubTiles> &sub, bool f32) {
   double prods = 0.0, tiles = 0.0;
   int nmax = 0;
@@ -1992,7 +2002,7 @@ static double inverse_pays_after(const std::vector<SubTiles> &sub, bool f32) {
   const double n = nmax, bytes = tiles * TILE_ELEMS * (f32 ? 4.0 : 8.0);
   const double form = prods * kTileGemm / (f32 ? 95e12 : 50e12) + n * 40e-6;
   const double sweeps = std::max(2.0 * n * 3.4e-6 + n * (n + 1.0) * (f32 ? 0.4e-6 : 0.7e-6),
-                                 2.0 * bytes / 5.5e12);
+                                 2.0 * bytes / (f32 ? 5.5e12 : 5.7e12));
   const double saved = sweeps - (bytes / 5.9e12 + 15e-6);
   return saved > 0.0 ? form / saved : 1e30;
 }
