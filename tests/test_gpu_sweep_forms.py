@@ -1,7 +1,8 @@
 """The sweeps over interior and interface factors in the forms that the number
-of subdomains selects (up to 256, up to 1023 and more): the reduced right-hand
-side and the solution against dense elimination of each subdomain's interior,
-FP64 and FP32 factors."""
+of subdomains selects (up to 256, up to 1023 and more), FP64 and FP32 factors:
+the residual of the assembled matrix at the solution, which the sweeps of the
+reduced right-hand side and of the interiors leave at the tolerance of the
+interface problem."""
 import numpy as np
 import pytest
 
@@ -17,7 +18,7 @@ def test_sweeps_solve_the_interiors(nel, ns, refined):
     print("case sweep forms", nel, ns, refined, flush=True)
     p = CubeProblem(nel, ns, rhs="random", seed=8)
     b, (it, reason, _) = bddcml_amd.solve_cube(p, tol=1e-12, options={"refinement": refined})
-    assert reason >= 0
+    assert reason == 0
     u = b.download_global_solution(p.ndof)
     b.finalize()
     # the residual of the assembled matrix on the free dofs: backward stable

@@ -17,8 +17,6 @@ pytestmark = pytest.mark.gpu
                                          (5, 5, "elasticity"), (16, 3, "elasticity")])
 def test_schur_apply_equals_dense_products(nel, ns, kind, refined):
     print("case symmetric GEMV", nel, ns, kind, refined, flush=True)
-    if nel == 16 and refined:
-        pytest.skip("the FP64 case covers the form; FP32 differs in the loads only")
     p = CubeProblem(nel, ns, kind=kind, rhs="random", seed=3)
     b = bddcml_amd.Bddcml()
     b.init(2, [p.nsub, 1], numbase=p.numbase)
