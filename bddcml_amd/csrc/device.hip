@@ -1071,6 +1071,29 @@ static bool relative_ids(TaskList &L, int b0, int nb) {
   return ok;
 }
 
+// tile products of a list's tasks, each by its share of 16 x 16 blocks that its
+// mask leaves, and the tasks that end with a post multiply or a factorization
+// (a task of its own mode may have neither).  One thread took 120 ms, of a
+// setup of 510, over the 10 M products of 400 uneven boxes of up to 12,600
+// dofs before the factorization could start; per class, by all threads, 5 ms.
+static void count_work(const TaskList &l, double &products, double &posted) {
+  int64_t blocks = 0, post = 0;
+  for (const TileTask &t : l.tasks) {
+    post += t.mode < 0 || t.mode == kTaskPotrf || ((t.mode >> 2) & 3) != 0;
+    for (int p = t.p0; p < t.p1; p++) {
+      const uint32_t m = l.pairs[p].m;
+      if (m == 0xFFFFFFFFu) {
+        blocks += 64;
+        continue;
+      }
+      for (int k = 0; k < 16; k += 4)
+        blocks += __builtin_popcount(m >> k & 15) * __builtin_popcount(m >> (16 + k) & 15);
+    }
+  }
+  products = blocks / 64.0;
+  posted = (double)post;
+}
+
 // One launch over every subdomain from the class lists (tile ids relative
 // to the subdomain's base): the pairs once per class, the tasks per
 // subdomain with its base added, subdomain-major.
@@ -1090,18 +1113,26 @@ static TaskList materialize(const std::vector<Q> &sts, Get get, const std::vecto
   }
   out.pairs.resize(poff[ncls]);
   out.tasks.resize(toff[nsub]);
-  for (int ic = 0; ic < ncls; ic++)
-    if (const TaskList *L = get(sts[ic]))
-      std::copy(L->pairs.begin(), L->pairs.end(), out.pairs.begin() + poff[ic]);
-#pragma omp parallel for schedule(static)
-  for (int is = 0; is < nsub; is++) {
-    const TaskList *L = get(sts[cls[is]]);
-    if (!L) continue;
-    const int b = base_of(is), po = (int)poff[cls[is]];
-    TileTask *o = out.tasks.data() + toff[is];
-    for (const TileTask &t : L->tasks)
-      *o++ = TileTask{t.c + b, t.x >= 0 ? t.x + b : -1, t.p0 + po, t.p1 + po, b, t.fresh, t.mode};
+  std::vector<double> products(ncls, 0.0), posted(ncls, 0.0);
+#pragma omp parallel
+  {
+#pragma omp for schedule(dynamic) nowait
+    for (int ic = 0; ic < ncls; ic++)
+      if (const TaskList *L = get(sts[ic])) {
+        std::copy(L->pairs.begin(), L->pairs.end(), out.pairs.begin() + poff[ic]);
+        count_work(*L, products[ic], posted[ic]);
+      }
+#pragma omp for schedule(static)
+    for (int is = 0; is < nsub; is++) {
+      const TaskList *L = get(sts[cls[is]]);
+      if (!L) continue;
+      const int b = base_of(is), po = (int)poff[cls[is]];
+      TileTask *o = out.tasks.data() + toff[is];
+      for (const TileTask &t : L->tasks)
+        *o++ = TileTask{t.c + b, t.x >= 0 ? t.x + b : -1, t.p0 + po, t.p1 + po, b, t.fresh, t.mode};
+    }
   }
+  for (int c : cls) out.products += products[c], out.posted += posted[c];
   return out;
 }
 
@@ -1225,33 +1256,12 @@ static void split_steps(const std::vector<std::vector<TaskList> *> &lists, int k
 // work done: 2*64^3 flops per tile product, 64^3/3 per tile Cholesky plus
 // 64^3/3 for its inverse, 2*64^3 per post multiply; of products with masks
 // and of post multiplies by triangular tiles (kTilePost) the 16 x 16 blocks
-// that are computed.  Pair lists are shared between subdomains, so the pairs
-// of each task are counted.
+// that are computed (counted per class by materialize)
 static const double kTileGemm = 2.0 * 64 * 64 * 64, kTileChol = 64.0 * 64 * 64 / 3.0;
 static const double kTilePost = kTileGemm * 10 / 16;
-static double tile_products(const TaskList &l) {
-  std::vector<double> upto(l.pairs.size() + 1, 0.0);
-  for (size_t p = 0; p < l.pairs.size(); p++) {
-    int blocks = 0;
-    for (int k = 0; k < 16; k += 4)
-      blocks += __builtin_popcount(l.pairs[p].m >> k & 15) *
-                __builtin_popcount(l.pairs[p].m >> (16 + k) & 15);
-    upto[p + 1] = upto[p] + blocks / 64.0;
-  }
-  double n = 0;
-  for (const TileTask &t : l.tasks) n += upto[t.p1] - upto[t.p0];
-  return n;
-}
-// tasks that end with a post multiply or a factorization (a task of its own
-// mode may have neither)
-static double posted_tasks(const TaskList &l) {
-  double n = 0;
-  for (const TileTask &t : l.tasks) n += t.mode < 0 || t.mode == kTaskPotrf || ((t.mode >> 2) & 3) != 0;
-  return n;
-}
 static double tile_work(const std::vector<TaskList> &v, double per_task) {
   double f = 0;
-  for (auto &l : v) f += kTileGemm * tile_products(l) + per_task * posted_tasks(l);
+  for (auto &l : v) f += kTileGemm * l.products + per_task * l.posted;
   return f;
 }
 
@@ -1795,7 +1805,7 @@ void device_setup_begin(Solver &S) {
                 (long long)D.ntiles, D.ntiles * (D.f32i ? 16384.0 : 32768.0) / 1e9,
                 (size_t)D.sc_pads.n);
 
-  S.t.schur_flops = kTileGemm * tile_products(a_schur);
+  S.t.schur_flops = kTileGemm * a_schur.products;
   S.t.interior_flops = tile_work(a_diag, 2 * kTileChol) + tile_work(a_off, kTilePost) +
                        tile_work(a_upd, 0.0) + tile_work(m_rows, kTileGemm) + S.t.schur_flops;
   // ---- numerics, first half: Dirichlet elimination into the tiles,
@@ -1804,8 +1814,8 @@ void device_setup_begin(Solver &S) {
   for (hipEvent_t &e : D.ev_gemm) HIPCHECK(hipEventCreate(&e));
   D.gemm_flops.clear();
   for (size_t l = 0; l < a_off.size(); l++)
-    D.gemm_flops.push_back(kTileGemm * (tile_products(a_off[l]) + tile_products(a_upd[l])) +
-                           kTilePost * posted_tasks(a_off[l]));
+    D.gemm_flops.push_back(kTileGemm * (a_off[l].products + a_upd[l].products) +
+                           kTilePost * a_off[l].posted);
   HIPCHECK(hipEventCreateWithFlags(&D.ev_up, hipEventDisableTiming));
   HIPCHECK(hipEventCreateWithFlags(&D.ev_rhs, hipEventDisableTiming));
   // element type of the subdomain tiles: FP64, or FP32 with refinement
@@ -2189,10 +2199,10 @@ void device_setup_interface(Solver &S) {
     // forms it (option 1); the automatic mode forms it during a solve
     S.t.interface_flops = tile_work(p_diag, 2 * kTileChol) + tile_work(p_off, kTileGemm) +
                           tile_work(z_bwd, kTileGemm) + tile_work(p_upd, 0.0) +
-                          tile_work(z_upd, 0.0) + kTileGemm * tile_products(phi);
+                          tile_work(z_upd, 0.0) + kTileGemm * phi.products;
     if (D.inv_planned && !D.inv_auto)
       S.t.interface_flops += tile_work(w_rows, kTileGemm) + tile_work(w_upd, 0.0) +
-                             kTileGemm * tile_products(kinv);
+                             kTileGemm * kinv.products;
     D.plan2.verbose = S.verbose;
     upload_phases(D.p_diag, p_diag, D.plan2);
     upload_phases(D.p_off, p_off, D.plan2);

@@ -150,6 +150,9 @@ struct TilePair {
 struct TaskList {
   std::vector<TileTask> tasks;
   std::vector<TilePair> pairs;
+  // of the merged lists: products (by the blocks computed) and tasks with a
+  // post multiply or a factorization
+  double products = 0.0, posted = 0.0;
   void clear() {
     tasks.clear();
     pairs.clear();
