@@ -1998,8 +1998,8 @@ static double interface_rho(const Sub &s) {
 //   216 subdomains n = 25: 9.7 / 0.74 / 0.29 (21; 29); 512: 24.2 / 1.52 / 0.73
 //   (31; 31).
 // - FP32: 64 subdomains 1.5 / 0.30 / 0.05 (6; 5); 60 boxes 23.3 / 2.74 / 0.47
-//   (10; 6: k_symv gathers inputs of more than 72 tile rows tile by tile,
-//   at 2.5 TB/s); 512: 12.0 / 0.82 / 0.40 (29; 32).
+//   (10; 6: interfaces of more than 72 tile rows, whose input k_symv gathers,
+//   0.41 since); 512: 12.0 / 0.82 / 0.40 (29; 32).
 static double inverse_pays_after(const std::vector<SubTiles> &sub, bool f32) {
   double prods = 0.0, tiles = 0.0;
   int nmax = 0;

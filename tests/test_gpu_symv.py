@@ -37,3 +37,28 @@ def test_schur_apply_equals_dense_products(nel, ns, kind, refined):
     b.finalize()
     # the same products summed in another order: n eps of the row sums of moduli
     assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+def test_inverse_apply_of_gathered_inputs(precision):
+    """The local preconditioner through the explicit inverse, whose weighted
+    input is gathered tile by tile (interfaces of up to 73 tiles), against the
+    sweeps over the factor."""
+    print("case gathered inverse", precision, flush=True)
+    p = CubeProblem(16, 3, kind="elasticity", rhs="random", seed=3)
+    subs = list(p.subdomains())
+    out = []
+    for inverse in (0, 1):
+        b = bddcml_amd.Bddcml()
+        b.init(2, [p.nsub, 1], numbase=p.numbase)
+        b.set_option("precision", precision)
+        b.set_option("explicit_inverse", inverse)
+        for d in subs:
+            b.upload_subdomain_data(d)
+        b.setup_preconditioner()
+        x = np.random.RandomState(6).uniform(-1, 1, len(b.interface_dofs()))
+        out.append(b.apply_pc(x))
+        b.finalize()
+    # two backward stable applies of one matrix of condition <= 1e4
+    eps = 2.0 ** (-53 if precision == 64 else -24)
+    assert np.abs(out[0] - out[1]).max() <= 1e4 * eps * np.abs(out[0]).max()
