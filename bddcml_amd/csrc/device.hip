@@ -2396,6 +2396,13 @@ void device_setup_interface(Solver &S) {
       for (int g = 0; g < P; g++) sg.push_back({T.slow, n, is, g, P, po + (int64_t)g * n * 64});
       po += (int64_t)P * n * 64;
     }
+    // the largest first: there are more groups than the chip holds at once when
+    // many subdomains are too small to be shared, and the last ones then decide
+    // (400 uneven boxes of 10 to 97 tile rows: FP64 2.58 -> 2.21 ms, FP32 1.61
+    // -> 1.21; 512 subdomains of 16^3 0.71 -> 0.67, 0.370 -> 0.347)
+    auto tiles = [](const SymvGroup &g) { return (int64_t)g.n * (g.n + 1) / g.P; };
+    std::stable_sort(sg.begin(), sg.end(),
+                     [&](const SymvGroup &a, const SymvGroup &b) { return tiles(a) > tiles(b); });
     if (D.inv_planned) {
       std::vector<SymvGroup> pg(sg);
       for (SymvGroup &g : pg) {
