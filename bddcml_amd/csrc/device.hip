@@ -2398,7 +2398,7 @@ void device_setup_interface(Solver &S) {
     }
     // the largest first: there are more groups than the chip holds at once when
     // many subdomains are too small to be shared, and the last ones then decide
-    // (400 uneven boxes of 10 to 97 tile rows: FP64 2.58 -> 2.21 ms, FP32 1.61
+    // (400 uneven boxes of 21 to 68 tile rows: FP64 2.58 -> 2.21 ms, FP32 1.61
     // -> 1.21; 512 subdomains of 16^3 0.71 -> 0.67, 0.370 -> 0.347)
     auto tiles = [](const SymvGroup &g) { return (int64_t)g.n * (g.n + 1) / g.P; };
     std::stable_sort(sg.begin(), sg.end(),
