@@ -41,8 +41,10 @@ namespace bddc {
 #define HIPCHECK(x)                                                                       \
   do {                                                                                    \
     hipError_t e_ = (x);                                                                  \
-    if (e_ != hipSuccess)                                                                 \
+    if (e_ != hipSuccess) {                                                               \
+      (void)hipGetLastError(); /* reported here, not by the next problem's checks */      \
       fatal("BDDCML_DEVICE", std::string(#x) + " failed: " + hipGetErrorString(e_));      \
+    }                                                                                     \
   } while (0)
 
 // Host waits on the device spin instead of sleeping: a sleeping wait woke

@@ -160,7 +160,10 @@ void *pinned_alloc(size_t bytes) {
   if (k >= 0) return take(K, K.idle_pinned, k, dev);
   void *p = nullptr;
   const hipError_t e = hipHostMalloc(&p, bytes, hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable);
-  if (e != hipSuccess) fatal("BDDCML_DEVICE", std::string("hipHostMalloc failed: ") + hipGetErrorString(e));
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    fatal("BDDCML_DEVICE", std::string("hipHostMalloc failed: ") + hipGetErrorString(e));
+  }
   K.out[p] = Block{p, bytes, dev, K.problem, true};
   return p;
 }

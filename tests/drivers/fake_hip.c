@@ -7,19 +7,24 @@
 
 enum { MAXB = 4096, NDEV = 2 };
 static struct { char *p; size_t n; } blocks[MAXB];
-static int nblocks, current, busy[NDEV], fail_at = -1, bad_copies, copies;
+static int nblocks, current, busy[NDEV], fail_at = -1, fail_host_at = -1, bad_copies, copies, last;
 
 void fake_device(int d) { current = d; }
 int fake_current(void) { return current; }
 int fake_busy(int d) { return busy[d]; }
 void fake_fail_at(int n) { fail_at = n; } /* the n-th hipMalloc from now fails (0: the next) */
+void fake_fail_host_at(int n) { fail_host_at = n; } /* the same for hipHostMalloc */
 int fake_bad_copies(void) { return bad_copies; }
 int fake_copies(void) { return copies; }
 
 int hipGetDevice(int *d) { *d = current; return 0; }
 int hipSetDevice(int d) { current = d; return 0; }
 int hipSetDeviceFlags(unsigned f) { (void)f; return 0; }
-int hipGetLastError(void) { return 0; }
+int hipGetLastError(void) {
+  const int e = last;
+  last = 0;
+  return e;
+}
 const char *hipGetErrorString(int e) { return e ? "fake error" : "no error"; }
 int hipDeviceSynchronize(void) { busy[current] = 0; return 0; }
 int hipStreamSynchronize(void *st) { (void)st; busy[current] = 0; return 0; }
@@ -43,11 +48,16 @@ static int drop(void *p) {
 }
 int hipMalloc(void **p, size_t n) {
   *p = 0;
-  if (fail_at >= 0 && fail_at-- == 0) return 2;
+  if (fail_at >= 0 && fail_at-- == 0) return last = 2;
   return put(p, n);
 }
 int hipFree(void *p) { return drop(p); }
-int hipHostMalloc(void **p, size_t n, unsigned f) { (void)f; return put(p, n); }
+int hipHostMalloc(void **p, size_t n, unsigned f) {
+  (void)f;
+  *p = 0;
+  if (fail_host_at >= 0 && fail_host_at-- == 0) return last = 2;
+  return put(p, n);
+}
 int hipHostFree(void *p) { return drop(p); }
 static int inside(const char *p, size_t n) {
   for (int k = 0; k < nblocks; k++)

@@ -1,6 +1,7 @@
 """Device memory kept between problems, against a stand-in of the HIP runtime
 (tests/drivers/fake_hip.c): which device a returned block waits for, and what
-an upload does after one that ran out of memory.  No GPU is needed."""
+an upload and the next problem do after one that ran out of memory.  No GPU is
+needed."""
 import os
 import shutil
 import subprocess
@@ -81,5 +82,27 @@ for d in subs:
 assert fake.fake_bad_copies() == 0, fake.fake_bad_copies()
 assert failed <= 1
 assert failed == 1 or {nth} > 2
+b.finalize()
+""")
+
+
+@pytest.mark.parametrize("what", ["fake_fail_at", "fake_fail_host_at"])
+def test_next_problem_after_out_of_memory(fake, what):
+    """An allocation that failed and was reported is not reported again by the
+    error checks of the next problem."""
+    _run(fake, f"""
+p = CubeProblem(8, 3)  # 27 subdomains: several batches
+subs = list(p.subdomains())
+b = start()
+fake.{what}(0)
+try:
+    b.upload_subdomain_data(subs[0])
+    assert False, "taken without memory"
+except RuntimeError as e:
+    assert "Malloc" in str(e), e
+b.finalize()
+b = start()
+for d in subs:
+    b.upload_subdomain_data(d)
 b.finalize()
 """)
