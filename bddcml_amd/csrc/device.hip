@@ -1116,7 +1116,8 @@ static TaskList materialize(const std::vector<Q> &sts, Get get, const std::vecto
   out.pairs.resize(poff[ncls]);
   out.tasks.resize(toff[nsub]);
   std::vector<double> products(ncls, 0.0), posted(ncls, 0.0);
-#pragma omp parallel
+  // (a few thousand entries take one thread less time than waking the others)
+#pragma omp parallel if (out.pairs.size() + out.tasks.size() > 4096)
   {
 #pragma omp for schedule(dynamic) nowait
     for (int ic = 0; ic < ncls; ic++)
